@@ -44,9 +44,9 @@ struct AmgParams {
   int post_smooth = 2;
   double omega = 0.8;
   double equil_threshold = 1e-6;  // equilibrate when median |a_ii| is below this
-  int dense_max = 500;            // largest coarsest level solved densely (<= 4096; above 160 rows
-                                  // the inverse is formed on the matrix cores when the level is
-                                  // SPD, else by pivoted Gauss-Jordan up to 512 rows)
+  int dense_max = 500;            // largest coarsest level solved densely (<= 4096): the
+                                  // inverse is formed on the matrix cores when the level is SPD,
+                                  // else by pivoted Gauss-Jordan up to 512 rows
   int coarse_sweeps = 50;         // Jacobi sweeps on a coarsest level above dense_max
   int anchor = -1;                // forced C point on every level (reference anchor_idx), -1 = none
   // Additions that change the preconditioner (not the converged answer).
@@ -108,11 +108,9 @@ struct Level {
   // work vectors (x: solution, b: right-hand side, r: residual, t: Jacobi ping-pong)
   DevBuf<double> x64, b64, r64, t64;
   DevBuf<float> x32, b32, r32, t32;
-  // coarsest level: [A_pinned^-1] stored in the right half of an n x 2n matrix
-  DevBuf<double> aug;
-  // coarsest level above 160 rows: A_pinned^-1 padded to dense_pad(n) (matrix cores)
-  bool mfma = false;
-  DevBuf<double> inv, gj_w, gj_p;
+  // dense coarsest level: A_pinned^-1 padded to dense_pad(n), the work of its
+  // elimination and its failure flag; [A | I] of the pivoted form (n <= 512)
+  DevBuf<double> inv, gj_w, gj_p, aug;
   DevBuf<int> gj_bad;
 };
 
@@ -213,7 +211,7 @@ class Hierarchy {
   void build_levels(hipStream_t s);
   void finish_level_values(int l, hipStream_t s);
   void build_coarsest(int l, hipStream_t s);
-  void dense_inverse(Level& L, hipStream_t s);  // coarsest inverse on the matrix cores
+  void dense_inverse(Level& L, hipStream_t s);  // coarsest pin and inverse
   void refresh_f32(hipStream_t s);
   void build_pad4(Level& L, hipStream_t s);
   void build_pad4_transfer(int rows, int nnz, const int* rp, const int* ci, const double* v, Pad4& T, hipStream_t s);

@@ -245,9 +245,6 @@ struct Sel<double> {
   static void dense_mv(int n, const int* pin, const double* M, const double* b, double* x, hipStream_t s) {
     launch_dense_mv_f64(n, pin, M, b, x, s);
   }
-  static void dense(int n, const int* pin, const double* aug, const double* b, double* x, hipStream_t s) {
-    launch_dense_solve_f64(n, pin, aug, b, x, s);
-  }
 };
 template <>
 struct Sel<float> {
@@ -315,9 +312,6 @@ struct Sel<float> {
   }
   static void dense_mv(int n, const int* pin, const double* M, const float* b, float* x, hipStream_t s) {
     launch_dense_mv_f32(n, pin, M, b, x, s);
-  }
-  static void dense(int n, const int* pin, const double* aug, const float* b, float* x, hipStream_t s) {
-    launch_dense_solve_f32(n, pin, aug, b, x, s);
   }
 };
 
@@ -674,37 +668,28 @@ void Hierarchy::build_coarsest(int l, hipStream_t s) {
   L.dense = L.n <= prm_.dense_max;
   // a single-level hierarchy is solved without the pin: alone it would freeze DOF 0
   L.pin_mode = levels_.size() > 1 ? prm_.coarse_pin : kPinNever;
-  L.pin.alloc(2);  // [0] pin flag, [1] inverse produced by the SPD sweep
-  launch_pin_decide(L.n, L.rp.p, L.ci.p, L.v.p, L.pin_mode, L.pin.p, s);
-  if (!L.dense) return;
-  // above 160 rows the blocked matrix-core inverse is faster than the one-workgroup
-  // sweep (a 508-row coarsest level: 0.3 ms per refresh against 85 ms)
-  L.mfma = L.n > kDenseSweepMax;
-  if (L.mfma) {
-    const long long np = dense_pad(L.n);
-    L.inv.alloc(np * np);
-    L.gj_w.alloc(np * np);
-    L.gj_p.alloc(2 * 64 * 64);
-    L.gj_bad.alloc(1);
-    dense_inverse(L, s);
-    if (read_scalar(L.gj_bad.p, s) == 0) return;
-    // a non-positive pivot: not SPD; up to 512 rows the pivoted elimination below
-    IMPES_REQUIRE(L.n <= 512, "amg setup: coarsest operator above 512 rows is not symmetric positive definite "
-                              "(lower dense_max)");
-    L.mfma = false;
-    L.inv.release();
-    L.gj_w.release();
-    L.gj_p.release();
-    L.gj_bad.release();
+  L.pin.alloc(1);
+  L.gj_bad.alloc(1);
+  if (!L.dense) {
+    launch_pin_decide(L.n, L.rp.p, L.ci.p, L.v.p, L.pin_mode, L.pin.p, L.gj_bad.p, s);
+    return;
   }
-  L.aug.alloc(2LL * L.n * L.n);
-  launch_csr_to_dense(L.n, L.rp.p, L.ci.p, L.v.p, L.pin.p, L.aug.p, s);
-  launch_gauss_jordan_inverse(L.n, L.aug.p, L.pin.p + 1, s);
+  const long long np = dense_pad(L.n);
+  L.inv.alloc(np * np);
+  L.gj_w.alloc(np * np);
+  L.gj_p.alloc(kDenseWorkP);
+  if (L.n <= kDensePivotMax) L.aug.alloc(2LL * L.n * L.n);
+  dense_inverse(L, s);
+  if (L.n > kDensePivotMax)
+    IMPES_REQUIRE(read_scalar(L.gj_bad.p, s) == 0, "amg setup: coarsest operator above 512 rows is not symmetric "
+                                                   "positive definite (lower dense_max)");
 }
 
 void Hierarchy::dense_inverse(Level& L, hipStream_t s) {
-  launch_fill_i32(L.gj_bad.p, 0, 1, s);
+  launch_pin_decide(L.n, L.rp.p, L.ci.p, L.v.p, L.pin_mode, L.pin.p, L.gj_bad.p, s);
   launch_dense_inverse_mfma(L.n, L.rp.p, L.ci.p, L.v.p, L.pin.p, L.inv.p, L.gj_w.p, L.gj_p.p, L.gj_bad.p, s);
+  if (L.n <= kDensePivotMax)
+    launch_gauss_jordan_inverse(L.n, L.rp.p, L.ci.p, L.v.p, L.pin.p, L.gj_bad.p, L.aug.p, L.inv.p, s);
 }
 
 void Hierarchy::build_pad4(Level& L, hipStream_t s) {
@@ -846,13 +831,8 @@ void Hierarchy::update_levels(bool fine_done, hipStream_t s) {
       }
     }
     if (L.coarsest) {
-      launch_pin_decide(L.n, L.rp.p, L.ci.p, L.v.p, L.pin_mode, L.pin.p, s);
-      if (L.dense && L.mfma) {
-        dense_inverse(L, s);
-      } else if (L.dense) {
-        launch_csr_to_dense(L.n, L.rp.p, L.ci.p, L.v.p, L.pin.p, L.aug.p, s);
-        launch_gauss_jordan_inverse(L.n, L.aug.p, L.pin.p + 1, s);
-      }
+      if (L.dense) dense_inverse(L, s);
+      else launch_pin_decide(L.n, L.rp.p, L.ci.p, L.v.p, L.pin_mode, L.pin.p, L.gj_bad.p, s);
     }
   }
   if (stencil_ && !fine_done) refresh_stencil(s);
@@ -933,12 +913,8 @@ void Hierarchy::smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& z
 template <class T>
 void Hierarchy::coarse_solve(int l, const T* b, T* x, hipStream_t s) {
   Level& L = levels_[l];
-  if (L.dense && L.mfma) {
-    Sel<T>::dense_mv(L.n, L.pin.p, L.inv.p, b, x, s);
-    return;
-  }
   if (L.dense) {
-    Sel<T>::dense(L.n, L.pin.p, L.aug.p, b, x, s);
+    Sel<T>::dense_mv(L.n, L.pin.p, L.inv.p, b, x, s);
     return;
   }
   // reference: 50 L1-Jacobi sweeps from zero on the unpinned matrix with b_0 = 0

@@ -92,27 +92,27 @@ void launch_spgemm_numeric(int nnz_c, const long long* seg, const int* pe, const
 // coarsest level (coarse.hip). pin is a device flag written by launch_pin_decide and
 // read by the kernels below, so the decision never leaves the device.
 // pin = (mode == reference) || (mode == auto && every row has |row sum| <= 1e-8 |a_ii|)
-void launch_pin_decide(int n, const int* rp, const int* ci, const double* v, int mode, int* pin, hipStream_t s);
-// dense inverse of the (optionally DOF-0-pinned) matrix
-void launch_csr_to_dense(int n, const int* rp, const int* ci, const double* v, const int* pin, double* dense,
-                         hipStream_t s);
-// aug is n x 2n row-major [A | I], inverse into the right half: the LDS sweep for symmetric
-// positive definite A (n <= 199), else pivoted Gauss-Jordan; done: device int scratch
-void launch_gauss_jordan_inverse(int n, double* aug, int* done, hipStream_t s);
-// x = Ainv * b (with pin: b[0] treated as 0); FP64 and FP32 vector variants
-// Coarsest levels of more than kDenseSweepMax rows (up to kDenseMfmaMax): the inverse by
-// blocked Gauss-Jordan on the matrix cores (dense_mfma.hip) into M (dense_pad(n)^2
-// doubles), with W (dense_pad(n)^2) and P (2 x 64 x 64) as work; *bad is set when a
-// pivot is not positive (the operator is not SPD). Applied by launch_dense_mv_*.
+// *bad (the failure flag of the inverse) is cleared
+void launch_pin_decide(int n, const int* rp, const int* ci, const double* v, int mode, int* pin, int* bad,
+                       hipStream_t s);
+// Inverse of the (optionally DOF-0-pinned) level matrix in M (dense_pad(n)^2 doubles,
+// n <= kDenseMfmaMax): blocked Gauss-Jordan without pivoting on the matrix cores
+// (dense_mfma.hip), with W (dense_pad(n)^2) and P (kDenseWorkP) as work; sets *bad
+// when the operator is not SPD: a pivot that is not positive, and up to
+// kDenseStrictMax rows also an asymmetry or a pivot of rounding size. Then
+// launch_gauss_jordan_inverse with partial pivoting (n <= kDensePivotMax, aug n x 2n)
+// replaces M when *bad. Applied by launch_dense_mv_* (with pin: b[0] treated as 0).
 constexpr int kDenseMfmaMax = 4096;
-constexpr int kDenseSweepMax = 160;  // coarsest levels up to this size: the register sweep
+constexpr int kDenseStrictMax = 160;
+constexpr int kDensePivotMax = 512;
+constexpr int kDenseWorkP = 2 * 64 * 64 + 192;  // two pivot inverses, the diagonal (strict sizes)
 int dense_pad(int n);
 void launch_dense_inverse_mfma(int n, const int* rp, const int* ci, const double* v, const int* pin, double* M,
                                double* W, double* P, int* bad, hipStream_t s);
 void launch_dense_mv_f64(int n, const int* pin, const double* M, const double* b, double* x, hipStream_t s);
 void launch_dense_mv_f32(int n, const int* pin, const double* M, const float* b, float* x, hipStream_t s);
-void launch_dense_solve_f64(int n, const int* pin, const double* aug, const double* b, double* x, hipStream_t s);
-void launch_dense_solve_f32(int n, const int* pin, const double* aug, const float* b, float* x, hipStream_t s);
+void launch_gauss_jordan_inverse(int n, const int* rp, const int* ci, const double* v, const int* pin, const int* bad,
+                                 double* aug, double* M, hipStream_t s);
 // b[0] = 0 when *pin (Jacobi coarsest path)
 void launch_pin_rhs_f64(const int* pin, double* b, hipStream_t s);
 void launch_pin_rhs_f32(const int* pin, float* b, hipStream_t s);
