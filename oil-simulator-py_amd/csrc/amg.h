@@ -108,7 +108,7 @@ struct Level {
   // work vectors (x: solution, b: right-hand side, r: residual, t: Jacobi ping-pong)
   DevBuf<double> x64, b64, r64, t64;
   DevBuf<float> x32, b32, r32, t32;
-  // dense coarsest level: A_pinned^-1 padded to dense_pad(n), the work of its
+  // dense coarsest level: A_pinned^-1 padded to dense_pad(n) and its transpose, the work of its
   // elimination and its failure flag; [A | I] of the pivoted form (n <= 512)
   DevBuf<double> inv, gj_w, gj_p, aug;
   DevBuf<int> gj_bad;
@@ -218,8 +218,12 @@ class Hierarchy {
   void refresh_stencil(hipStream_t s);
   void alloc_vectors();
   // first_sweep_done: x already holds the first pre-smoothing sweep from zero
+  // tail: levels from tail_ down as one matrix (ensure_tail has run)
   template <class T>
-  void vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done = false);
+  void vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done = false,
+                    bool tail = false);
+  void choose_tail(hipStream_t s);
+  void ensure_tail(int precision, hipStream_t s);
   template <class T>
   void smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& zero, hipStream_t s);
   template <class T>
@@ -244,6 +248,19 @@ class Hierarchy {
   bool graphs_ = true;
   bool transposed_ = false;  // eager cycles of vcycle64/32 with nu1 and nu2 swapped
   hipGraphExec_t vexec_[2] = {nullptr, nullptr};  // [0] FP32, [1] FP64 V-cycle
+
+  // The preconditioner's cycle from level tail_ down as one matrix (tail.hip; -1:
+  // none), per precision ([0] FP32, [1] FP64): formed at the first cycle after a
+  // setup or update, which clear tail_ready_.
+  int tail_ = -1;
+  bool tail_ready_[2] = {false, false};
+  int tail_ld_ = 0;
+  std::vector<long long> tail_at_;   // per level from tail_: first slice offset in tail_so_
+  std::vector<long long> tail_line_; // per level from tail_: first line in tail_ell_ (last: the total)
+  DevBuf<int> tail_so_;
+  DevBuf<unsigned char> tail_ell_[2];
+  DevBuf<float> tail_b32_;
+  DevBuf<double> tail_b64_;
 
   AmgParams prm_;
   // device memory of builds: slab-carved small blocks, releases deferred to the

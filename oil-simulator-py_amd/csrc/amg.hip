@@ -378,8 +378,8 @@ void Hierarchy::capture_vcycle(int precision) {
   hipGraph_t g = nullptr;
   IMPES_HIP_CHECK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
   try {
-    if (precision == 32) vcycle_level<float>(0, L0.b32.p, L0.x32.p, true, cs);
-    else vcycle_level<double>(0, L0.b64.p, L0.x64.p, true, cs);
+    if (precision == 32) vcycle_level<float>(0, L0.b32.p, L0.x32.p, true, cs, false, true);
+    else vcycle_level<double>(0, L0.b64.p, L0.x64.p, true, cs, false, true);
   } catch (...) {
     (void)hipStreamEndCapture(cs, &g);
     if (g) (void)hipGraphDestroy(g);
@@ -419,6 +419,7 @@ void Hierarchy::setup_impl(int n, int nnz, const int* rp, const int* ci, const d
   refresh_f32(s);
   if (stencil_) refresh_stencil(s);
   alloc_vectors();
+  choose_tail(s);
   IMPES_HIP_CHECK(hipStreamSynchronize(s));
   }
   last_setup_seconds = wall() - t0;
@@ -675,7 +676,7 @@ void Hierarchy::build_coarsest(int l, hipStream_t s) {
     return;
   }
   const long long np = dense_pad(L.n);
-  L.inv.alloc(np * np);
+  L.inv.alloc(2 * np * np);
   L.gj_w.alloc(np * np);
   L.gj_p.alloc(kDenseWorkP);
   if (L.n <= kDensePivotMax) L.aug.alloc(2LL * L.n * L.n);
@@ -809,6 +810,7 @@ void Hierarchy::update_csr_values(const double* v, hipStream_t s) {
 }
 
 void Hierarchy::update_levels(bool fine_done, hipStream_t s) {
+  tail_ready_[0] = tail_ready_[1] = false;
   for (int l = 0; l + 1 < (int)levels_.size(); ++l) {
     Level& A = levels_[l];
     if (A.coarsest) break;
@@ -868,6 +870,104 @@ bool Hierarchy::coarse_pinned(hipStream_t s) const {
 LevelInfo Hierarchy::info(int l) const {
   const Level& L = levels_.at(l);
   return LevelInfo{L.n, L.nnz, L.coarsest ? 0 : L.pnnz, L.coarsest ? 1 : 0, L.dense ? 1 : 0};
+}
+
+// ---------------------------------------------------------------- coarse tail
+// The tail starts at the finest level that tail.hip's limits admit (both precisions),
+// down to a dense coarsest level. The limits: each cycle saves about 17 us per level
+// (six launches of ~3.2 us against one product of 4-6 us) and runs ten times and more
+// per update; forming costs 45-50 us at 1,200 rows and 8,600 entries below them, 107
+// us in FP64 at 1,343 rows and 16,700 entries (two rounds of workgroups), but 168 us
+// at 2,046 rows and 91,000 entries and 360 us above a 518-row coarsest level.
+void Hierarchy::choose_tail(hipStream_t s) {
+  tail_ = -1;
+  tail_ready_[0] = tail_ready_[1] = false;
+  tail_at_.clear();
+  tail_line_.clear();
+  const int last = (int)levels_.size() - 1;
+  if (!levels_[last].dense) return;
+  if (levels_[last].n > kTailCoarsest) return;
+  for (int l = std::max(0, last + 1 - kTailLevels); l < last; ++l) {
+    const int n = levels_[l].n;
+    if (n > kTailMax || levels_[l].nnz > kTailNnz) continue;
+    TailArgs A;
+    A.levels = last - l;
+    for (int q = l; q <= last; ++q) A.lv[q - l].n = levels_[q].n;
+    if (tail_lds_layout(A, 32) > kTailLds || tail_lds_layout(A, 64) > kTailLds) continue;
+    tail_ = l;
+    break;
+  }
+  if (tail_ < 0) return;
+  tail_ld_ = (levels_[tail_].n + 7) / 8 * 8;
+  // slice offsets of every level but the coarsest, from the longest row of each slice
+  std::vector<int> at;
+  int slices = 0;
+  for (int q = tail_; q < last; ++q) {
+    at.push_back(slices);
+    slices += tail_slices(levels_[q].n);
+  }
+  DevBuf<int> width;
+  width.alloc(slices);
+  for (int q = tail_; q < last; ++q) launch_tail_widths(levels_[q].n, levels_[q].rp.p, width.p + at[q - tail_], s);
+  std::vector<int> w(slices), so;
+  IMPES_HIP_CHECK(hipMemcpyAsync(w.data(), width.p, sizeof(int) * slices, hipMemcpyDeviceToHost, s));
+  IMPES_HIP_CHECK(hipStreamSynchronize(s));
+  long long lines = 0;
+  for (int q = tail_; q < last; ++q) {
+    tail_at_.push_back((long long)so.size());
+    tail_line_.push_back(lines);
+    const int ns = tail_slices(levels_[q].n);
+    int sum = 0;
+    for (int t = 0; t < ns; ++t) {
+      so.push_back(sum);
+      sum += w[at[q - tail_] + t];
+    }
+    so.push_back(sum);
+    lines += sum;
+  }
+  tail_line_.push_back(lines);
+  tail_so_.alloc(so.size());
+  IMPES_HIP_CHECK(hipMemcpyAsync(tail_so_.p, so.data(), sizeof(int) * so.size(), hipMemcpyHostToDevice, s));
+  IMPES_HIP_CHECK(hipStreamSynchronize(s));
+}
+
+void Hierarchy::ensure_tail(int precision, hipStream_t s) {
+  const int gi = precision == 32 ? 0 : 1;
+  if (tail_ < 0 || tail_ready_[gi]) return;
+  const int last = (int)levels_.size() - 1;
+  const size_t line = tail_ell_bytes(1, precision);
+  tail_ell_[gi].alloc(line * tail_line_.back());
+  const size_t nb = (size_t)levels_[tail_].n * tail_ld_;
+  if (precision == 32) tail_b32_.alloc(nb);
+  else tail_b64_.alloc(nb);
+  TailArgs A;
+  A.levels = last - tail_;
+  for (int q = tail_; q <= last; ++q) {
+    const Level& L = levels_[q];
+    TailLevel& t = A.lv[q - tail_];
+    t.n = L.n;
+    if (q == last) break;
+    t.so = (int)tail_at_[q - tail_];
+    unsigned char* ell = tail_ell_[gi].p + line * tail_line_[q - tail_];
+    launch_tail_pack(precision, L.n, L.rp.p, L.ci.p, L.v.p, tail_so_.p + t.so, ell, s);
+    t.ell = ell;
+    t.ir = L.ir64.p;
+    t.prp = L.prp.p; t.pci = L.pci.p; t.pv = L.pv.p;
+    t.rrp = L.rrp.p; t.rci = L.rci.p; t.rv = L.rv.p;
+  }
+  A.so = tail_so_.p;
+  A.so_len = (int)tail_so_.n;
+  const Level& C = levels_[last];
+  A.inv_ld = dense_pad(C.n);
+  A.inv_t = C.inv.p + (size_t)A.inv_ld * A.inv_ld;
+  A.pin = C.pin.p;
+  A.pre = prm_.pre_smooth;
+  A.post = prm_.post_smooth;
+  A.omega = prm_.omega;
+  A.ld = tail_ld_;
+  A.B = precision == 32 ? (void*)tail_b32_.p : (void*)tail_b64_.p;
+  launch_tail_form(precision, A, s);
+  tail_ready_[gi] = true;
 }
 
 // ---------------------------------------------------------------- V-cycle
@@ -1027,8 +1127,13 @@ void Hierarchy::level_times(int precision, int cycles, double* ms, double* cycle
 }
 
 template <class T>
-void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done) {
+void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done, bool tail) {
   Level& L = levels_[l];
+  if (tail && l == tail_) {
+    if constexpr (sizeof(T) == 8) launch_tail_mv_f64(L.n, tail_ld_, tail_b64_.p, b, x, s);
+    else launch_tail_mv_f32(L.n, tail_ld_, tail_b32_.p, b, x, s);
+    return;
+  }
   const int m0 = mark(s);
   if (L.coarsest) {
     coarse_solve<T>(l, b, x, s);
@@ -1054,7 +1159,7 @@ void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s
     Sel<T>::resL(L, cur, b, r, s);
   }
   Level& C = levels_[l + 1];
-  const bool fused = !C.coarsest && prm_.pre_smooth > 0;
+  const bool fused = !C.coarsest && prm_.pre_smooth > 0 && !(tail && l + 1 == tail_);
   if (fused) {
     // restriction fused with the coarse level's first sweep from zero
     Sel<T>::restrict_j0(L, r, Sel<T>::ir(C), prm_.omega, Sel<T>::b(C), Sel<T>::x(C), s);
@@ -1062,7 +1167,7 @@ void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s
     Sel<T>::restrict_to(L, r, Sel<T>::b(C), s);
   }
   segment(l, m0, mark(s));
-  vcycle_level<T>(l + 1, Sel<T>::b(C), Sel<T>::x(C), true, s, fused);
+  vcycle_level<T>(l + 1, Sel<T>::b(C), Sel<T>::x(C), true, s, fused, tail);
   const int m1 = mark(s);
   // Post-smoothing alternates between x and t: prolongate into the buffer from
   // which post_smooth sweeps end in x, so the cycle needs no final copy.
@@ -1184,10 +1289,11 @@ void Hierarchy::vcycle_only(int precision, hipStream_t s) {
   Level& L0 = levels_[0];
   const bool replay = graphs_ && !ktimer_enabled();
   const int gi = precision == 32 ? 0 : 1;
+  ensure_tail(precision, s);
   if (replay && !vexec_[gi]) capture_vcycle(precision);
   if (replay) IMPES_HIP_CHECK(hipGraphLaunch(vexec_[gi], s));
-  else if (precision == 32) vcycle_level<float>(0, L0.b32.p, L0.x32.p, true, s);
-  else vcycle_level<double>(0, L0.b64.p, L0.x64.p, true, s);
+  else if (precision == 32) vcycle_level<float>(0, L0.b32.p, L0.x32.p, true, s, false, true);
+  else vcycle_level<double>(0, L0.b64.p, L0.x64.p, true, s, false, true);
 }
 
 void Hierarchy::precondition(int precision, const double* v, double* z, hipStream_t s) {

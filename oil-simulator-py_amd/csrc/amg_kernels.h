@@ -96,7 +96,7 @@ void launch_spgemm_numeric(int nnz_c, const long long* seg, const int* pe, const
 void launch_pin_decide(int n, const int* rp, const int* ci, const double* v, int mode, int* pin, int* bad,
                        hipStream_t s);
 // Inverse of the (optionally DOF-0-pinned) level matrix in M (dense_pad(n)^2 doubles,
-// n <= kDenseMfmaMax): blocked Gauss-Jordan without pivoting on the matrix cores
+// and its transpose behind it, n <= kDenseMfmaMax): blocked Gauss-Jordan without pivoting on the matrix cores
 // (dense_mfma.hip), with W (dense_pad(n)^2) and P (kDenseWorkP) as work; sets *bad
 // when the operator is not SPD: a pivot that is not positive, and up to
 // kDenseStrictMax rows also an asymmetry or a pivot of rounding size. Then
@@ -116,5 +116,48 @@ void launch_gauss_jordan_inverse(int n, const int* rp, const int* ci, const doub
 // b[0] = 0 when *pin (Jacobi coarsest path)
 void launch_pin_rhs_f64(const int* pin, double* b, hipStream_t s);
 void launch_pin_rhs_f32(const int* pin, float* b, hipStream_t s);
+
+
+// The coarse end of the cycle as one matrix (tail.hip): levels of at most kTailMax
+// rows and kTailNnz entries above a coarsest level of at most kTailCoarsest rows,
+// whose vectors fit kTailLds bytes of LDS for one workgroup's columns.
+constexpr int kTailMax = 2048;
+constexpr int kTailNnz = 40000;
+constexpr int kTailCoarsest = 400;
+constexpr int kTailLevels = 8;  // the coarsest one included
+constexpr size_t kTailLds = 157 * 1024;
+struct TailLevel {
+  int n = 0;
+  int so = 0;                // first of its slice offsets (in 64-entry lines) in TailArgs::so
+  const void* ell = nullptr; // sliced operator
+  const double* ir = nullptr;
+  const int *prp = nullptr, *pci = nullptr, *rrp = nullptr, *rci = nullptr;
+  const double *pv = nullptr, *rv = nullptr;
+  int x = 0, y = 0, b = 0;   // LDS offsets of its vectors
+};
+struct TailArgs {
+  int levels = 0;  // non-coarsest levels; lv[levels] is the coarsest
+  TailLevel lv[kTailLevels];
+  const int* so = nullptr;        // slice offsets of all levels
+  int so_len = 0;
+  const double* inv_t = nullptr;  // transposed inverse of the coarsest operator
+  int inv_ld = 0;
+  const int* pin = nullptr;
+  int pre = 0, post = 0;
+  double omega = 0.0;
+  int part = 0, splits = 0;  // LDS offset and count of the coarsest solve's partial sums
+  int ld = 0;         // row stride of B, a multiple of 8
+  void* B = nullptr;  // float (precision 32) or double
+};
+int tail_slices(int n);
+void launch_tail_widths(int n, const int* rp, int* width, hipStream_t s);
+size_t tail_ell_bytes(long long lines, int precision);
+void launch_tail_pack(int precision, int n, const int* rp, const int* ci, const double* v, const int* so, void* ell,
+                      hipStream_t s);
+// assigns the LDS offsets; bytes of LDS (above kTailLds: does not fit)
+size_t tail_lds_layout(TailArgs& A, int precision);
+void launch_tail_form(int precision, TailArgs A, hipStream_t s);
+void launch_tail_mv_f32(int n, int ld, const float* B, const float* b, float* x, hipStream_t s);
+void launch_tail_mv_f64(int n, int ld, const double* B, const double* b, double* x, hipStream_t s);
 
 }  // namespace impes

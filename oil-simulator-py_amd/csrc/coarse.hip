@@ -51,7 +51,7 @@ __global__ void k_pin_rhs32(const int* __restrict__ pin, float* __restrict__ b) 
 
 // Single workgroup Gauss-Jordan with partial pivoting on the n x 2n matrix
 // [A_pinned | I] (n <= 512), formed in `aug`; the inverse goes to M (row stride
-// n_pad). Runs only when the unpivoted elimination on the matrix cores met an
+// n_pad), its transpose behind it. Runs only when the unpivoted elimination on the matrix cores met an
 // operator that is not SPD (*bad); else one load and out.
 __global__ __launch_bounds__(1024) void k_gauss_jordan(int n, int n_pad, const int* __restrict__ rp,
                                                        const int* __restrict__ ci, const double* __restrict__ v,
@@ -125,8 +125,12 @@ __global__ __launch_bounds__(1024) void k_gauss_jordan(int n, int n_pad, const i
     }
     __syncthreads();
   }
-  for (long long t = threadIdx.x; t < (long long)n * n; t += blockDim.x)
-    M[(t / n) * n_pad + t % n] = aug[(t / n) * w + n + t % n];
+  double* MT = M + (long long)n_pad * n_pad;
+  for (long long t = threadIdx.x; t < (long long)n * n; t += blockDim.x) {
+    const double a = aug[(t / n) * w + n + t % n];
+    M[(t / n) * n_pad + t % n] = a;
+    MT[(t % n) * n_pad + t / n] = a;
+  }
 }
 
 }  // namespace

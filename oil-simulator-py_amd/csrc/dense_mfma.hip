@@ -231,13 +231,15 @@ __device__ __forceinline__ bool invert_block(v4d (&acc)[4], double* __restrict__
 }
 
 // Block 0: the inverse of the first 64 x 64 pivot block, into P (leading dimension
-// 64; straight into the result when the matrix has no other block). Blocks 1..: with
+// 64; straight into the result, with its transpose PT, when the matrix has no other
+// block). Blocks 1..: with
 // sym_rows > 0, block b checks row b - 1 for symmetry, |a_ij - a_ji| <= 1e-10
 // sqrt(a_ii a_jj) (the rounding asymmetry of a Galerkin product passes, a
 // non-symmetric operator does not; well rows can exceed interior rows by 15 orders,
 // so the scale is per entry), and for a positive diagonal, and keeps the diagonal.
 __global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n_pad, int sym_rows, const double* __restrict__ M,
-                                                          double* __restrict__ P, double* __restrict__ dg, double tol,
+                                                          double* __restrict__ P, double* __restrict__ PT,
+                                                          double* __restrict__ dg, double tol,
                                                           int* __restrict__ bad) {
   if (blockIdx.x > 0) {
     const int r = blockIdx.x - 1;
@@ -277,6 +279,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n_pad, int sym_row
       int r, c;
       tile_pos(t, e, r, c);
       P[r * kB + c] = acc[t][e];
+      if (PT) PT[c * kB + r] = acc[t][e];
     }
 }
 
@@ -285,19 +288,25 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n_pad, int sym_row
 // itself with the same MFMA sequence, so the row panel it subtracts equals the one
 // its own row-k block stores. The longest path of a launch is the workgroup that
 // also inverts the next pivot block (fetches, two products of 1.7 us, the inverse);
-// every tile it needs is fetched before the first product. One launch per block
+// every tile it needs is fetched before the first product. The last block column
+// also writes the transposed inverse (AnT). One launch per block
 // column: 47-49 -> 18-25 us at 128-576 rows.
 __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, const double* __restrict__ A,
                                                           double* __restrict__ An, const double* __restrict__ P,
-                                                          double* __restrict__ Pn, const double* __restrict__ dg,
-                                                          double tol, int* __restrict__ bad) {
+                                                          double* __restrict__ Pn, double* __restrict__ AnT,
+                                                          const double* __restrict__ dg, double tol,
+                                                          int* __restrict__ bad) {
   __shared__ double As[kB * kLdA], Bs[kB * kLdB], Cs[kB * kLdA];
   __shared__ double d0[kB];  // the next pivot block's entries of dg
   const int j = blockIdx.x, i = blockIdx.y;
   const double* blk = A + (long long)i * kB * n_pad + (long long)j * kB;
   double* out = An + (long long)i * kB * n_pad + (long long)j * kB;
+  double* outT = AnT ? AnT + (long long)j * kB * n_pad + (long long)i * kB : nullptr;
   if (i == k && j == k) {
-    for (int q = threadIdx.x; q < kB * kB; q += blockDim.x) out[(long long)(q / kB) * n_pad + q % kB] = P[q];
+    for (int q = threadIdx.x; q < kB * kB; q += blockDim.x) {
+      out[(long long)(q / kB) * n_pad + q % kB] = P[q];
+      if (outT) outT[(long long)(q % kB) * n_pad + q / kB] = P[q];
+    }
     return;
   }
   v4d acc[4];
@@ -316,6 +325,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, cons
         int r, c;
         tile_pos(t, e, r, c);
         out[(long long)r * n_pad + c] = -acc[t][e];
+        if (outT) outT[(long long)c * n_pad + r] = -acc[t][e];
       }
     return;
   }
@@ -333,6 +343,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, cons
         int r, c;
         tile_pos(t, e, r, c);
         out[(long long)r * n_pad + c] = acc[t][e];
+        if (outT) outT[(long long)c * n_pad + r] = acc[t][e];
       }
     return;
   }
@@ -372,6 +383,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, cons
       tile_pos(t, e, r, c);
       own[t][e] -= acc[t][e];
       out[(long long)r * n_pad + c] = own[t][e];
+      if (outT) outT[(long long)c * n_pad + r] = own[t][e];
     }
   if (i != k + 1 || j != k + 1 || Pn == nullptr) return;
   // this block is the next step's pivot block: its inverse goes to step k + 1 in Pn
@@ -421,6 +433,7 @@ void launch_dense_inverse_mfma(int n, const int* rp, const int* ci, const double
                                double* W, double* P, int* bad, hipStream_t s) {
   IMPES_REQUIRE(n >= 1 && n <= kDenseMfmaMax, "MFMA dense inverse supports 1 <= n <= 4096");
   const int n_pad = dense_pad(n), nb = n_pad / kB;
+  double* MT = M + (long long)n_pad * n_pad;
   // small operators are checked for symmetry and their pivots against the diagonal
   // (a pivot of rounding size: not numerically SPD), so that a failed check reaches
   // the pivoted elimination; larger ones for positive pivots only
@@ -435,13 +448,14 @@ void launch_dense_inverse_mfma(int n, const int* rp, const int* ci, const double
   // P holds two 64 x 64 pivot inverses: step k reads P_k and its block (k+1, k+1)
   // workgroup writes P_{k+1} into the other half. With one block its inverse is the
   // result (n_pad = 64 = the leading dimension of P).
-  k_gj_diag<<<1 + (strict ? n : 0), kGemmThreads, 0, s>>>(n_pad, strict ? n : 0, cur, nb == 1 ? M : P, dg, tol, bad);
+  k_gj_diag<<<1 + (strict ? n : 0), kGemmThreads, 0, s>>>(n_pad, strict ? n : 0, cur, nb == 1 ? M : P,
+                                                              nb == 1 ? MT : nullptr, dg, tol, bad);
   IMPES_LAUNCH_CHECK();
   if (nb == 1) return;
   for (int k = 0; k < nb; ++k) {
     double* Pk = P + (k & 1) * kB * kB;
     double* Pn = (k + 1 < nb) ? P + ((k + 1) & 1) * kB * kB : nullptr;
-    k_gj_step<<<dim3(nb, nb), kGemmThreads, 0, s>>>(k, n_pad, cur, nxt, Pk, Pn, dg, tol, bad);
+    k_gj_step<<<dim3(nb, nb), kGemmThreads, 0, s>>>(k, n_pad, cur, nxt, Pk, Pn, k + 1 == nb ? MT : nullptr, dg, tol, bad);
     IMPES_LAUNCH_CHECK();
     std::swap(cur, nxt);
   }
