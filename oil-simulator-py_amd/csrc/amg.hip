@@ -1287,7 +1287,8 @@ const void* Hierarchy::vcycle_out(int precision) const {
 void Hierarchy::vcycle_only(int precision, hipStream_t s) {
   IMPES_REQUIRE(!levels_.empty(), "preconditioner before setup");
   Level& L0 = levels_[0];
-  const bool replay = graphs_ && !ktimer_enabled();
+  // a cycle that is one product needs no graph (its launch costs the host more)
+  const bool replay = graphs_ && !ktimer_enabled() && tail_ != 0;
   const int gi = precision == 32 ? 0 : 1;
   ensure_tail(precision, s);
   if (replay && !vexec_[gi]) capture_vcycle(precision);

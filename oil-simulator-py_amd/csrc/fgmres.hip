@@ -11,6 +11,7 @@
 #include <cstdint>
 
 #include "fgmres.h"
+#include "fgmres_small.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -22,24 +23,7 @@ namespace impes {
 namespace {
 
 constexpr int kGsThreads = 256;
-constexpr int kMaxFusedGs = 32;  // largest k of the register-resident Gram-Schmidt passes
-
-struct Layout {
-  int m;
-  __host__ __device__ int H(int i, int j) const { return i + j * (m + 1); }
-  __host__ __device__ int g() const { return (m + 1) * m; }
-  __host__ __device__ int cs() const { return g() + m + 1; }
-  __host__ __device__ int sn() const { return cs() + m; }
-  __host__ __device__ int h() const { return sn() + m; }
-  __host__ __device__ int h2() const { return h() + m + 1; }
-  __host__ __device__ int y() const { return h2() + m + 1; }
-  __host__ __device__ int sc() const { return y() + m; }  // 8 scalars
-  // lagged orthogonalisation: provisional column (m+1) and the update's 2 scalars;
-  // its coefficients a and c reuse h() and h2()
-  __host__ __device__ int hp() const { return sc() + 8; }
-  __host__ __device__ int lag() const { return hp() + m + 1; }
-  __host__ __device__ int size() const { return lag() + 2; }
-};
+using Layout = FgmresLayout;
 
 // sc[0] = beta = sqrt(sc[4]) ; g = beta e1
 __global__ void k_init_cycle(Layout L, double* __restrict__ sm) {
@@ -394,13 +378,6 @@ __global__ __launch_bounds__(kGsThreads) void k_lag_update(int k, double* __rest
   if (threadIdx.x == 0) part[blockIdx.x] = acc;
 }
 
-// c, s = the Givens rotation that zeroes b under a
-__device__ __forceinline__ void givens(double a, double b, double& c, double& s) {
-  if (b == 0.0) { c = 1.0; s = 0.0; }
-  else if (fabs(b) > fabs(a)) { const double t = a / b; s = 1.0 / sqrt(1.0 + t * t); c = s * t; }
-  else { const double t = b / a; c = 1.0 / sqrt(1.0 + t * t); s = c * t; }
-}
-
 // All 2j + 2 columns of partials fold at once: G lanes per column (the widest
 // power of two up to a wave with G * columns <= 1024 threads), each lane summing
 // every G-th partial, then the G lanes. The partials were written by other XCDs,
@@ -683,14 +660,28 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
   st.precision = precision;
   double* V = V_.p;
   double* Z = Z_.p;
+  // two passes over the basis per Arnoldi step (lagged reorthogonalisation) when
+  // a preconditioner stages the next V-cycle input and the basis fits the fused
+  // kernels; else CGS2's three passes and a normalisation
+  const bool lagged = M != nullptr && m <= kMaxFusedGs && !cgs2_;
+  // one workgroup per step where the system is small (fgmres_small.hip); its rows are
+  // walked by one lane each, so long CSR rows keep the kernels with lanes per row
+  const bool small = lagged && n <= kSmallRows && (A.stencil || A.csr.nnz <= kSmallRowNnz * n);
+  const SmallOperator So{A.stencil, A.st, A.csr, A.dinv, (int)n};
+  float* b32 = small && precision == 32 ? (float*)M->vcycle_in(32) : nullptr;
+  double* b64 = small && precision == 64 ? (double*)M->vcycle_in(64) : nullptr;
   // ||D^-1 b|| and the scaled initial residual r0 = D^-1 (b - A x0) in V, their
   // squared norms read back with one synchronisation
-  launch_scale_f64(bs_.p, A.dinv, b, n, s);
-  launch_dot_f64(bs_.p, bs_.p, n, sc + 5, work_.p, s);
-  if (!use_x0) launch_fill_f64(x, 0.0, n, s);
-  residual(A, x, b, V, s);
-  launch_dot_f64(V, V, n, sc + 4, work_.p, s);
-  IMPES_HIP_CHECK(hipMemcpyAsync(host_ + 4, sc + 4, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+  if (small) {
+    small_start(So, L, sm, b, x, use_x0, V, host_dev_, s);
+  } else {
+    launch_scale_f64(bs_.p, A.dinv, b, n, s);
+    launch_dot_f64(bs_.p, bs_.p, n, sc + 5, work_.p, s);
+    if (!use_x0) launch_fill_f64(x, 0.0, n, s);
+    residual(A, x, b, V, s);
+    launch_dot_f64(V, V, n, sc + 4, work_.p, s);
+    IMPES_HIP_CHECK(hipMemcpyAsync(host_ + 4, sc + 4, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+  }
   IMPES_HIP_CHECK(hipStreamSynchronize(s));
   const double bnorm = std::sqrt(host_[5]);
   double beta = std::sqrt(host_[4]);
@@ -743,15 +734,17 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
   const double ratio = std::max(err_ratio_[0], err_ratio_[1]);
   if (check && ratio > 0.0) target = std::min(tol, kErrTarget * etol_ / ratio * bnorm);
   bool ok = false;
-  // two passes over the basis per Arnoldi step (lagged reorthogonalisation) when
-  // a preconditioner stages the next V-cycle input and the basis fits the fused
-  // kernels; else CGS2's three passes and a normalisation
-  const bool lagged = M != nullptr && m <= kMaxFusedGs && !cgs2_;
+  bool staged = false;  // small: the error check's preconditioner input is S .* V already
   for (;;) {
     while (beta > target && its < maxit && std::isfinite(beta)) {
-      k_init_cycle<<<1, 1, 0, s>>>(L, sm);
-      IMPES_LAUNCH_CHECK();
-      normalize(V, V, sc + 0);
+      if (small) {
+        if (b32) small_begin(So.n, L, sm, V, M->in_scale(), b32, s);
+        else small_begin(So.n, L, sm, V, M->in_scale(), b64, s);
+      } else {
+        k_init_cycle<<<1, 1, 0, s>>>(L, sm);
+        IMPES_LAUNCH_CHECK();
+        normalize(V, V, sc + 0);
+      }
       int k = 0;
       const int its0 = its;
       // the estimate of iteration jj lands in pinned slot host_[2 + (jj & 1)]; its
@@ -771,7 +764,15 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
         double* vj = V + (long long)j * n;
         double* zj = Z + (long long)j * n;
         double* est = host_dev_ + 2 + (j & 1);
-        if (lagged) {
+        if (small) {
+          M->vcycle_only(precision, s);
+          if (b32)
+            small_step(So, L, j, sm, (const float*)M->vcycle_out(32), M->out_scale(), zj, V, M->in_scale(), b32, est, s);
+          else
+            small_step(So, L, j, sm, (const double*)M->vcycle_out(64), M->out_scale(), zj, V, M->in_scale(), b64, est,
+                       s);
+          final_cols = j;
+        } else if (lagged) {
           // z_j = M u (the V-cycle input S .* u was written by the previous update,
           // or by the cycle's normalisation for j = 0), w = D^-1 A z_j
           precondition_apply(vj, zj);
@@ -835,6 +836,15 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
         if (stops(j, e)) break;
       }
       its = its0 + k;
+      if (small) {
+        if (b32) small_end(So, L, k, final_cols < k, sm, Z, V, b, x, M->in_scale(), b32, host_dev_, s);
+        else small_end(So, L, k, final_cols < k, sm, Z, V, b, x, M->in_scale(), b64, host_dev_, s);
+        staged = true;
+        IMPES_HIP_CHECK(hipStreamSynchronize(s));
+        beta = std::sqrt(((volatile double*)host_)[4]);
+        ++st.restarts;
+        continue;
+      }
       if (lagged && final_cols < k) {
         // close column k-1: dots of u = V[:, k] against v_0..v_{k-1}, then its colA
         const double* uk = V + (long long)k * n;
@@ -857,15 +867,24 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
     }
     // error check: V holds the scaled residual D^-1 (b - A x); z = M V lands in
     // Z's first column (w receives D^-1 A z, unused)
-    launch_fill_f64(sc + 6, 1.0, 1, s);
-    normalize(w_.p, V, sc + 6);
-    precondition_apply(w_.p, Z);
-    launch_amax_f64(Z, n, sc + 6, work_.p, s);
-    launch_axpy_f64(x, 1.0, Z, n, s);
-    launch_amax_f64(x, n, sc + 7, work_.p, s);
-    residual(A, x, b, V, s);
-    launch_dot_f64(V, V, n, sc + 4, work_.p, s);
-    IMPES_HIP_CHECK(hipMemcpyAsync(host_ + 4, sc + 4, 4 * sizeof(double), hipMemcpyDeviceToHost, s));
+    if (small) {
+      if (!staged && b32) small_input(So.n, V, M->in_scale(), b32, s);
+      else if (!staged) small_input(So.n, V, M->in_scale(), b64, s);
+      staged = false;
+      M->vcycle_only(precision, s);
+      if (b32) small_check(So, L, sm, (const float*)M->vcycle_out(32), M->out_scale(), V, b, x, host_dev_, s);
+      else small_check(So, L, sm, (const double*)M->vcycle_out(64), M->out_scale(), V, b, x, host_dev_, s);
+    } else {
+      launch_fill_f64(sc + 6, 1.0, 1, s);
+      normalize(w_.p, V, sc + 6);
+      precondition_apply(w_.p, Z);
+      launch_amax_f64(Z, n, sc + 6, work_.p, s);
+      launch_axpy_f64(x, 1.0, Z, n, s);
+      launch_amax_f64(x, n, sc + 7, work_.p, s);
+      residual(A, x, b, V, s);
+      launch_dot_f64(V, V, n, sc + 4, work_.p, s);
+      IMPES_HIP_CHECK(hipMemcpyAsync(host_ + 4, sc + 4, 4 * sizeof(double), hipMemcpyDeviceToHost, s));
+    }
     IMPES_HIP_CHECK(hipStreamSynchronize(s));
     const double zmax = host_[6], xmax = host_[7];
     const double est = (zmax > 0.0) ? zmax / std::max(xmax, 1e-300) : 0.0;
