@@ -69,7 +69,8 @@ struct LevelInfo {
 // tiles of whole rows; nw == 0 when a row is too long for a tile
 struct Pad4 {
   int n = 0, nnz = 0, nw = 0;
-  DevBuf<int> rp4, ci4, wrow, wq;
+  DevBuf<int> rp4, ci4, wrow;
+  DevBuf<unsigned short> tag;
   DevBuf<float> v4;
 };
 
@@ -88,8 +89,9 @@ struct Level {
   int g4 = 1;
   DevBuf<int> rp4, ci4;  // ci4 released when the 16-bit offsets co4 fit
   DevBuf<short> co4;
-  int nw4 = 0;               // wave tiles of the padded operator (0: none)
-  DevBuf<int> wrow4, wq4;
+  int nw4 = 0;               // wave tiles of the padded operator (0: the plain form)
+  DevBuf<int> wrow4;
+  DevBuf<unsigned short> tag4;
   DevBuf<float> v4;
   DevBuf<signed char> cf;  // final C/F markers (non-coarsest levels)
   // interpolation / restriction to the next level
@@ -213,6 +215,8 @@ class Hierarchy {
   void build_coarsest(int l, hipStream_t s);
   void dense_inverse(Level& L, hipStream_t s);  // coarsest pin and inverse
   void refresh_f32(hipStream_t s);
+  // wave tiles of a matrix's rows (Csr4F32): their number, 0 when a row is too long
+  int build_tiles(int rows, const int* rp, DevBuf<int>& wrow, DevBuf<int>& rp4, hipStream_t s);
   void build_pad4(Level& L, hipStream_t s);
   void build_pad4_transfer(int rows, int nnz, const int* rp, const int* ci, const double* v, Pad4& T, hipStream_t s);
   void refresh_stencil(hipStream_t s);

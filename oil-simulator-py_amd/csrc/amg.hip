@@ -263,7 +263,7 @@ struct Sel<float> {
   }
   static Csr4F32 A4(const Level& L) {
     return Csr4F32{L.n, L.nnz, L.rp4.p, reinterpret_cast<const int4*>(L.ci4.p), reinterpret_cast<const float4*>(L.v4.p),
-                   reinterpret_cast<const short4*>(L.co4.p), L.nw4, L.wrow4.p, L.wq4.p};
+                   reinterpret_cast<const short4*>(L.co4.p), L.nw4, L.wrow4.p, L.tag4.p};
   }
   static void jacL(const Level& L, const float* xi, const float* b, double w, float* xo, hipStream_t s) {
     if (L.pad4) launch_jacobi4_f32(A4(L), L.g4, xi, b, L.ir32.p, (float)w, xo, s);
@@ -290,7 +290,7 @@ struct Sel<float> {
   // grid transfers of level L: restriction in the padded tiled form when built
   static Csr4F32 T4(const Pad4& T) {
     return Csr4F32{T.n, T.nnz, T.rp4.p, reinterpret_cast<const int4*>(T.ci4.p), reinterpret_cast<const float4*>(T.v4.p),
-                   nullptr, T.nw, T.wrow.p, T.wq.p};
+                   nullptr, T.nw, T.wrow.p, T.tag.p};
   }
   static void restrict_j0(const Level& L, const float* r, const float* irc, double w, float* bc, float* xc,
                           hipStream_t s) {
@@ -693,68 +693,68 @@ void Hierarchy::dense_inverse(Level& L, hipStream_t s) {
     launch_gauss_jordan_inverse(L.n, L.rp.p, L.ci.p, L.v.p, L.pin.p, L.gj_bad.p, L.aug.p, L.inv.p, s);
 }
 
-void Hierarchy::build_pad4(Level& L, hipStream_t s) {
+int Hierarchy::build_tiles(int rows, const int* rp, DevBuf<int>& wrow, DevBuf<int>& rp4, hipStream_t s) {
+  const int segs = div_up(rows, kTileSeg);
   DevBuf<int> cnt;
-  cnt.alloc(L.n);
-  L.rp4.alloc(L.n + 1);
-  launch_csr4_count(L.n, L.rp.p, cnt.p, s);
-  scan_i32_to_i32(cnt.p, L.rp4.p, L.n, s);
-  const long long nnz4 = read_scalar(L.rp4.p + L.n, s);
-  L.ci4.alloc(nnz4);
-  L.v4.alloc(nnz4);
-  launch_csr4_pattern(L.n, L.rp.p, L.ci.p, L.rp4.p, L.ci4.p, s);
-  launch_csr4_values(L.n, L.rp.p, L.v.p, L.rp4.p, L.v4.p, s);
-  L.g4 = csr4_group_for(L.n, nnz4);
-  L.pad4 = true;
+  DevBuf<long long> base;
+  cnt.alloc(segs);
+  base.alloc(segs + 1);
+  launch_tile4_count(rows, rp, cnt.p, s);
+  scan_i32_to_i64(cnt.p, base.p, segs, s);
+  const long long nw = read_scalar(base.p + segs, s);
+  if (nw >= kTileNone) return 0;
+  wrow.alloc(nw + 1);
+  rp4.alloc(rows);
+  launch_tile4_rows(rows, rp, base.p, wrow.p, rp4.p, s);
+  sync_before_release(s);
+  return (int)nw;
+}
+
+void Hierarchy::build_pad4(Level& L, hipStream_t s) {
   // 16-bit column offsets from the row where every entry is within 2^15 of it
   DevBuf<int> maxabs;
   maxabs.alloc(1);
   launch_fill_i32(maxabs.p, 0, 1, s);
-  L.co4.alloc(nnz4);
-  launch_csr4_offsets(L.n, L.rp4.p, L.ci4.p, L.co4.p, maxabs.p, s);
+  L.nw4 = build_tiles(L.n, L.rp.p, L.wrow4, L.rp4, s);
+  if (L.nw4 > 0) {
+    const size_t slots = (size_t)L.nw4 * kWave;
+    L.ci4.alloc(4 * slots);
+    L.co4.alloc(4 * slots);
+    L.v4.alloc(4 * slots);
+    L.tag4.alloc(slots);
+    launch_tile4_fill(L.nw4, L.wrow4.p, L.rp.p, L.ci.p, L.v.p, L.rp4.p, L.ci4.p, L.co4.p, L.v4.p, L.tag4.p, maxabs.p,
+                      true, s);
+  } else {
+    DevBuf<int> cnt;
+    cnt.alloc(L.n);
+    L.rp4.alloc(L.n + 1);
+    launch_csr4_count(L.n, L.rp.p, cnt.p, s);
+    scan_i32_to_i32(cnt.p, L.rp4.p, L.n, s);
+    const long long nnz4 = read_scalar(L.rp4.p + L.n, s);
+    L.ci4.alloc(nnz4);
+    L.v4.alloc(nnz4);
+    L.co4.alloc(nnz4);
+    launch_csr4_pattern(L.n, L.rp.p, L.ci.p, L.rp4.p, L.ci4.p, s);
+    launch_csr4_values(L.n, L.rp.p, L.v.p, L.rp4.p, L.v4.p, s);
+    L.g4 = csr4_group_for(L.n, nnz4);
+    launch_csr4_offsets(L.n, L.rp4.p, L.ci4.p, L.co4.p, maxabs.p, s);
+  }
+  L.pad4 = true;
   if (read_scalar(maxabs.p, s) <= 32767) L.ci4.release();  // 8.97 -> 8.88 ms per step at 1M cells
   else L.co4.release();
-  // wave tiles of whole rows (the pattern is fixed after setup)
-  std::vector<int> hrp(L.n + 1), wrow, wq;
-  IMPES_HIP_CHECK(hipMemcpyAsync(hrp.data(), L.rp4.p, sizeof(int) * (L.n + 1), hipMemcpyDeviceToHost, s));
-  IMPES_HIP_CHECK(hipStreamSynchronize(s));
-  L.nw4 = csr4_wave_tiles(L.n, hrp.data(), wrow, wq);
-  if (L.nw4 > 0) {
-    L.wrow4.alloc(L.nw4 + 1);
-    L.wq4.alloc(L.nw4 + 1);
-    IMPES_HIP_CHECK(hipMemcpyAsync(L.wrow4.p, wrow.data(), sizeof(int) * (L.nw4 + 1), hipMemcpyHostToDevice, s));
-    IMPES_HIP_CHECK(hipMemcpyAsync(L.wq4.p, wq.data(), sizeof(int) * (L.nw4 + 1), hipMemcpyHostToDevice, s));
-    IMPES_HIP_CHECK(hipStreamSynchronize(s));
-  }
 }
 
 void Hierarchy::build_pad4_transfer(int rows, int nnz, const int* rp, const int* ci, const double* v, Pad4& T,
                                     hipStream_t s) {
   T = Pad4{};
   if (rows <= 0) return;
-  DevBuf<int> cnt;
-  cnt.alloc(rows);
-  T.rp4.alloc(rows + 1LL);
-  launch_csr4_count(rows, rp, cnt.p, s);
-  scan_i32_to_i32(cnt.p, T.rp4.p, rows, s);
-  std::vector<int> hrp(rows + 1LL), wrow, wq;
-  IMPES_HIP_CHECK(hipMemcpyAsync(hrp.data(), T.rp4.p, sizeof(int) * (rows + 1LL), hipMemcpyDeviceToHost, s));
-  IMPES_HIP_CHECK(hipStreamSynchronize(s));
-  const int nw = csr4_wave_tiles(rows, hrp.data(), wrow, wq);
-  if (nw == 0) {  // a row longer than a tile: the CSR transfer kernels stay
-    T.rp4.release();
-    return;
-  }
-  const long long nnz4 = hrp[rows];
-  T.ci4.alloc(nnz4);
-  T.v4.alloc(nnz4);
-  launch_csr4_pattern(rows, rp, ci, T.rp4.p, T.ci4.p, s, false);
-  launch_csr4_values(rows, rp, v, T.rp4.p, T.v4.p, s);
-  T.wrow.alloc(nw + 1LL);
-  T.wq.alloc(nw + 1LL);
-  IMPES_HIP_CHECK(hipMemcpyAsync(T.wrow.p, wrow.data(), sizeof(int) * (nw + 1LL), hipMemcpyHostToDevice, s));
-  IMPES_HIP_CHECK(hipMemcpyAsync(T.wq.p, wq.data(), sizeof(int) * (nw + 1LL), hipMemcpyHostToDevice, s));
-  IMPES_HIP_CHECK(hipStreamSynchronize(s));
+  const int nw = build_tiles(rows, rp, T.wrow, T.rp4, s);
+  if (nw == 0) return;  // a row longer than a tile: the CSR transfer kernels stay
+  const size_t slots = (size_t)nw * kWave;
+  T.ci4.alloc(4 * slots);
+  T.v4.alloc(4 * slots);
+  T.tag.alloc(slots);
+  launch_tile4_fill(nw, T.wrow.p, rp, ci, v, T.rp4.p, T.ci4.p, nullptr, T.v4.p, T.tag.p, nullptr, false, s);
   T.n = rows;
   T.nnz = nnz;
   T.nw = nw;

@@ -97,7 +97,7 @@ __global__ void k_diag_relax_pad4(int n, const int* __restrict__ rp, const int* 
        i += (long long)gridDim.x * blockDim.x / kDiagLanes) {
     double d = 0.0, rs = 0.0;
     int dpos = 0x7fffffff;
-    const int e0 = rp[i], len = rp[i + 1] - e0, q0 = rp4[i], len4 = rp4[i + 1] - q0;
+    const int e0 = rp[i], len = rp[i + 1] - e0, q0 = rp4[i], len4 = len > 0 ? (len + 3) & ~3 : 4;
     for (int k = g; k < len4; k += kDiagLanes) {
       float out = 0.f;
       if (k < len) {

@@ -2,7 +2,6 @@
 // All launchers enqueue on the given stream and never synchronise.
 #pragma once
 
-#include <vector>
 
 #include "common.h"
 
@@ -59,10 +58,14 @@ template <class T>
 struct Stencil7 { int nx = 0, ny = 0, nz = 0; const T* d = nullptr; const T* ox = nullptr; const T* oy = nullptr; const T* oz = nullptr; };
 
 // FP32 CSR with every row padded to a multiple of 4 entries (value 0, column = the
-// row itself), 16-byte aligned: a lane reads 4 consecutive entries of its row with
-// one vector load, and the lanes of a wavefront read whole cache lines whatever
-// the row lengths. rp4 counts entries (multiples of 4); nnz is the unpadded count
-// (algorithmic bytes).
+// row itself), 16-byte aligned: a lane reads 4 consecutive entries (a chunk) of its
+// row with one vector load. nnz is the unpadded count (algorithmic bytes).
+// Tiled form (nw > 0): tile t is the 64 chunks from 64 t on, whole rows from wrow[t]
+// to wrow[t+1] - 1 in order, unused chunks at its end zero; tag[q] tells chunk q's
+// row within the tile (bits 0-5), its place within the row (6-11) and whether it is
+// the row's last (12). rp4[r]: first entry of row r.
+// Plain form (a row of more than 64 chunks): rows one after another, n + 1 entry
+// offsets rp4.
 struct Csr4F32 {
   int n = 0, nnz = 0;
   const int* rp4 = nullptr;
@@ -71,36 +74,38 @@ struct Csr4F32 {
   // when set (every |column - row| < 2^15): 16-bit column offsets from the row,
   // read instead of ci4 (8 bytes per 4 entries instead of 16)
   const short4* co4 = nullptr;
-  // when set: the rows cut into nw wave tiles of whole rows and at most 64 chunks
-  // (tile t = rows wrow[t] .. wrow[t+1]-1, chunks wq[t] .. wq[t+1]-1)
   int nw = 0;
   const int* wrow = nullptr;
-  const int* wq = nullptr;
+  const unsigned short* tag = nullptr;
 };
-// Wave tiles of a padded operator (see Csr4F32): rows packed greedily, in order,
-// into tiles of at most 64 four-entry chunks. Fills wrow and wq (nw + 1 entries
-// each) from the host copy of rp4 (n + 1 entry offsets); returns nw, or 0 when a
-// row has more than 64 chunks.
-int csr4_wave_tiles(int n, const int* rp4_host, std::vector<int>& wrow, std::vector<int>& wq);
-// lanes per row of the padded kernels from the padded entry count
+// Cutting n rows into tiles, in segments of kTileSeg rows: cnt[seg] = tiles of the
+// segment (kTileNone when a row has more than 64 chunks); then, from their exclusive
+// scan, wrow (the total + 1 entries) and rp4 (n).
+constexpr int kTileSeg = 512;
+constexpr int kTileNone = 1 << 30;
+void launch_tile4_count(int n, const int* rp, int* cnt, hipStream_t s);
+void launch_tile4_rows(int n, const int* rp, const long long* base, int* wrow, int* rp4, hipStream_t s);
+// Columns (ci4 and, clamped, their 16-bit offsets co4), tags and FP32 values of the
+// tiles; *maxabs (a device int, zero on entry) = the largest |column - row|. Padding
+// entries have value 0 and the column of the row itself (square) or of the row's
+// first entry (rectangular; 0 for an empty row). co4 and maxabs may be null.
+void launch_tile4_fill(int nw, const int* wrow, const int* rp, const int* ci, const double* v, const int* rp4,
+                       int* ci4, short* co4, float* v4, unsigned short* tag, int* maxabs, bool square, hipStream_t s);
+// Plain form: lanes per row of the padded kernels from the padded entry count;
 int csr4_group_for(int n_rows, long long nnz4);
-// padded row lengths: cnt[r] = rows' lengths rounded up to 4 (an empty row gets 4)
+// padded row lengths: cnt[r] = rows' lengths rounded up to 4 (an empty row gets 4);
 void launch_csr4_count(int n, const int* rp, int* cnt, hipStream_t s);
-// padded pattern (ci4 sized rp4[n]) and FP32 values (rounded from FP64) of a CSR
-// matrix; padding entries have value 0 and the column of the row itself (square)
-// or of the row's first entry (rectangular; 0 for an empty row)
-void launch_csr4_pattern(int n, const int* rp, const int* ci, const int* rp4, int* ci4, hipStream_t s,
-                         bool square = true);
+// padded pattern (ci4 sized rp4[n]) and FP32 values (rounded from FP64), padding as
+// above (square);
+void launch_csr4_pattern(int n, const int* rp, const int* ci, const int* rp4, int* ci4, hipStream_t s);
 void launch_csr4_values(int n, const int* rp, const double* v, const int* rp4, float* v4, hipStream_t s);
-// co4[e] = ci4[e] - row (16-bit) over nnz4 entries; *maxabs = the largest |ci4[e] - row|
-// (a device int, zero on entry)
+// co4[e] = ci4[e] - row (16-bit) over nnz4 entries, *maxabs as above
 void launch_csr4_offsets(int n, const int* rp4, const int* ci4, short* co4, int* maxabs, hipStream_t s);
 // r = b - A x and xo = xi + w inv_relax .* (b - A xi) on the padded form
 void launch_residual4_f32(const Csr4F32& A, int group, const float* x, const float* b, float* r, hipStream_t s);
 void launch_jacobi4_f32(const Csr4F32& A, int group, const float* xi, const float* b, const float* inv_relax, float w,
                         float* xo, hipStream_t s);
-// restriction on a padded operator with wave tiles (A.wrow set; column indices in
-// ci4): y = A x; and y = A x with y2 = w inv_relax2 .* y (fused with the coarse
+// restriction on a padded operator with wave tiles (A.nw > 0; column indices in ci4): y = A x; and y = A x with y2 = w inv_relax2 .* y (fused with the coarse
 // level's first sweep from zero)
 void launch_spmv4_f32(const Csr4F32& A, const float* x, float* y, hipStream_t s);
 void launch_restrict4_j0_f32(const Csr4F32& R, const float* r, const float* inv_relax_c, float w, float* bc, float* xc,

@@ -121,49 +121,41 @@ __global__ __launch_bounds__(kBlock) void k_csr4(int n, const int* __restrict__ 
   }
 }
 
-// Padded FP32 CSR over wave tiles (Csr4F32::wrow/wq): a wave takes one tile of
-// whole rows, one 4-entry chunk per lane, so no lane idles on a short row. A lane
-// finds its row by a binary search (shuffles) over the start chunks of the
-// tile's rows, sums its chunk, and the lanes of a row add up by a segmented
-// scan; the row's last lane applies the update. The sweeps are bound by each
-// wave's chain of dependent loads at full occupancy, so the number of waves sets
-// their time: on the 1M-cell hierarchy (4.6 chunks per row on level 1) G = 8
-// lanes per row left 43% of the lanes idle; the tiles took a step from
-// 8.25-8.27 to 7.86-7.87 ms.
+// Padded FP32 CSR over wave tiles: a wave takes one tile of 64 four-entry chunks, one
+// per lane, so no lane idles on a short row. A lane's row and its place in the row
+// come with the chunk (tag), and the tile's address from its number alone, so all of
+// a tile's operator loads issue at once and the gathers wait on nothing else; the
+// lanes of a row add up by a segmented scan of as many steps as the tile's longest
+// row needs, and the row's last lane applies the update.
+// What bounds it: the chain of dependent loads per wave at full occupancy
+// (operator -> gather -> update), then the gathers. The first tiled form (tiles of
+// whole rows packed without gaps) read each tile's bounds first, found the lane's row
+// by six dependent shuffles over a load of the row starts, and scanned six steps of
+// two shuffles: 8.6 -> 7.6 us per sweep over the 1M-cell hierarchy's levels (level 1,
+// 58 MB: 15.2 -> 13.7 us), 4.2 -> 3.6 us over the 200k-cell hierarchy's; the sums are
+// the same bits.
 template <int MODE, bool OFF16>
-__global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restrict__ wrow, const int* __restrict__ wq,
-                                                       const int* __restrict__ rp4, const int4* __restrict__ ci4,
-                                                       const short4* __restrict__ co4, const float4* __restrict__ v4,
-                                                       const float* __restrict__ x, const float* __restrict__ b,
-                                                       const float* __restrict__ aux, float w, float* __restrict__ y,
-                                                       float* __restrict__ y2) {
+__global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restrict__ wrow,
+                                                       const unsigned short* __restrict__ tag,
+                                                       const int4* __restrict__ ci4, const short4* __restrict__ co4,
+                                                       const float4* __restrict__ v4, const float* __restrict__ x,
+                                                       const float* __restrict__ b, const float* __restrict__ aux,
+                                                       float w, float* __restrict__ y, float* __restrict__ y2) {
   constexpr int WPB = kBlock / kWave;
   const int lane = threadIdx.x & (kWave - 1);
-  for (long long t = xcd_block() * WPB + threadIdx.x / kWave; t < nw; t += (long long)gridDim.x * WPB) {
-    const int r0 = wrow[t], nr = wrow[t + 1] - r0;
-    const int q0 = wq[t], q1 = wq[t + 1];
-    const int q = q0 + lane;
-    const bool valid = q < q1;
-    // start chunk, relative to the tile, of row r0 + 1 + lane (64: no such row)
-    const int ps = (lane + 1 < nr) ? (rp4[r0 + 1 + lane] >> 2) - q0 : kWave;
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    short4 o = make_short4(0, 0, 0, 0);
-    int4 c4 = make_int4(0, 0, 0, 0);
-    if (valid) {
-      a = v4[q];
-      if (OFF16) o = co4[q];
-      else c4 = ci4[q];
-    }
-    // rows of the tile that start at or before this lane's chunk
-    int lo = 0;
-#pragma unroll
-    for (int st = kWave / 2; st >= 1; st >>= 1) {
-      const int pc = __shfl(ps, lo + st - 1, kWave);
-      if (pc <= lane) lo += st;
-    }
-    const int row = r0 + lo;
-    const int rn = __shfl_down(row, 1, kWave);
-    const bool last = valid && (lane == kWave - 1 || q + 1 >= q1 || rn != row);
+  for (int t = (int)xcd_block() * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); t < nw;
+       t += gridDim.x * WPB) {
+    const long long q = (long long)t * kWave + lane;
+    const float4 a = v4[q];
+    const unsigned tg = tag[q];
+    int4 c;
+    short4 o;
+    if (OFF16) o = co4[q];
+    else c = ci4[q];
+    const int row = wrow[t] + (int)(tg & 63u);
+    const int pos = (int)(tg >> 6 & 63u);
+    const bool last = (tg >> 12) != 0;
+    if (OFF16) c = make_int4(row + o.x, row + o.y, row + o.z, row + o.w);
     float ob = 0.f, ox = 0.f, oa = 0.f;
     if (last) {
       if (MODE == kRes || MODE == kJac) ob = b[row];
@@ -171,20 +163,15 @@ __global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restr
       if (MODE == kJac || MODE == kRestrictJ0) oa = aux[row];
     }
     float sum = 0.f;
-    if (valid) {
-      int4 c;
-      if (OFF16) c = make_int4(row + o.x, row + o.y, row + o.z, row + o.w);
-      else c = c4;
-      sum += a.x * x[c.x];
-      sum += a.y * x[c.y];
-      sum += a.z * x[c.z];
-      sum += a.w * x[c.w];
-    }
+    sum += a.x * x[c.x];
+    sum += a.y * x[c.y];
+    sum += a.z * x[c.z];
+    sum += a.w * x[c.w];
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
+      if (!__any(pos >= d)) break;  // uniform
       const float u = __shfl_up(sum, d, kWave);
-      const int ru = __shfl_up(row, d, kWave);
-      if (lane >= d && ru == row) sum += u;
+      if (pos >= d) sum += u;
     }
     if (last) {
       if (MODE == kRes) y[row] = ob - sum;
@@ -198,12 +185,106 @@ __global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restr
   }
 }
 
+// chunks of row r (an empty row has one)
+__device__ __forceinline__ int row_chunks(const int* __restrict__ rp, int r) {
+  const int len = rp[r + 1] - rp[r];
+  return len > 0 ? (len + 3) >> 2 : 1;
+}
+
+// Greedy tiles of one segment, a wave each: per tile the wave looks at the next 64
+// rows and takes those whose chunks fit. FILL writes the tiles' first rows and the
+// rows' first entries, else the segment's tile count.
+template <bool FILL>
+__global__ __launch_bounds__(kBlock) void k_tile4_rows(int n, const int* __restrict__ rp,
+                                                       const long long* __restrict__ base, int* __restrict__ cnt,
+                                                       int* __restrict__ wrow, int* __restrict__ rp4) {
+  const int seg = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int r0 = seg * kTileSeg, r1 = min(n, r0 + kTileSeg);
+  if (r0 >= n) return;
+  long long t = FILL ? base[seg] : 0;
+  for (int r = r0; r < r1;) {
+    const int mine = r + lane;
+    const int c = mine < r1 ? row_chunks(rp, mine) : kWave + 1;
+    int sum = c;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int u = __shfl_up(sum, d, kWave);
+      if (lane >= d) sum += u;
+    }
+    const int take = __popcll(__ballot(mine < r1 && sum <= kWave));
+    if (take == 0) {  // a row longer than a tile
+      if (!FILL && lane == 0) cnt[seg] = kTileNone;
+      return;
+    }
+    if (FILL) {
+      if (lane == 0) wrow[t] = r;
+      if (lane < take) rp4[mine] = (int)((t * kWave + sum - c) * 4);
+    }
+    r += take;
+    ++t;
+  }
+  if (!FILL && lane == 0) cnt[seg] = (int)t;
+  if (FILL && r1 == n && lane == 0) wrow[t] = n;
+}
+
+// One tile per wave: every lane finds its chunk's row among the tile's row starts
+__global__ __launch_bounds__(kBlock) void k_tile4_fill(int nw, const int* __restrict__ wrow,
+                                                       const int* __restrict__ rp, const int* __restrict__ ci,
+                                                       const double* __restrict__ v, const int* __restrict__ rp4,
+                                                       int4* __restrict__ ci4, short4* __restrict__ co4,
+                                                       float4* __restrict__ v4, unsigned short* __restrict__ tag,
+                                                       int* __restrict__ maxabs, int square) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int far = 0;
+  for (int t = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; t < nw; t += gridDim.x * (kBlock / kWave)) {
+    const int r0 = wrow[t], nr = wrow[t + 1] - r0;
+    const int q0 = t * kWave;
+    // first chunk, relative to the tile, of row r0 + 1 + lane (64: no such row)
+    const int ps = (lane + 1 < nr) ? (rp4[r0 + 1 + lane] >> 2) - q0 : kWave;
+    int lo = 0;
+#pragma unroll
+    for (int st = kWave / 2; st >= 1; st >>= 1) {
+      const int pc = __shfl(ps, lo + st - 1, kWave);
+      if (pc <= lane) lo += st;
+    }
+    const int row = r0 + lo;
+    const int e0 = rp[row], len = rp[row + 1] - e0;
+    const int pos = q0 + lane - (rp4[row] >> 2), chunks = row_chunks(rp, row);
+    const bool used = pos < chunks;
+    const int pad = square ? row : (len > 0 ? ci[e0] : 0);
+    int c[4];
+    float a[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int k = 4 * pos + m;
+      const bool in = used && k < len;
+      c[m] = in ? ci[e0 + k] : pad;
+      a[m] = in ? (float)v[e0 + k] : 0.f;
+      far = max(far, abs(c[m] - row));
+    }
+    const long long q = (long long)q0 + lane;
+    ci4[q] = make_int4(c[0], c[1], c[2], c[3]);
+    v4[q] = make_float4(a[0], a[1], a[2], a[3]);
+    if (co4) {
+      short o[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) o[m] = (short)max(-32768, min(32767, c[m] - row));
+      co4[q] = make_short4(o[0], o[1], o[2], o[3]);
+    }
+    tag[q] = (unsigned short)(used ? (lo | pos << 6 | (pos + 1 == chunks ? 1 << 12 : 0)) : lo);
+  }
+  if (!maxabs) return;
+  far = wave_max(far);
+  if (lane == 0 && far > 0) atomicMax(maxabs, far);
+}
+
 template <int MODE, bool OFF16>
 void csr4_tile_launch(const Csr4F32& A, const float* x, const float* b, const float* aux, float w, float* y,
                       hipStream_t s, float* y2 = nullptr) {
   const int grid = grid_for(A.nw, kBlock / kWave, 1 << 18);
-  klaunch(k_csr4_tile<MODE, OFF16>, dim3(grid), dim3(kBlock), 0, s, A.nw, A.wrow, A.wq, A.rp4, A.ci4, A.co4, A.v4, x, b,
-          aux, w, y, y2);
+  klaunch(k_csr4_tile<MODE, OFF16>, dim3(grid), dim3(kBlock), 0, s, A.nw, A.wrow, A.tag, A.ci4, A.co4, A.v4, x, b, aux,
+          w, y, y2);
 }
 
 template <int MODE, bool OFF16>
@@ -237,7 +318,7 @@ void csr4_dispatch(const Csr4F32& A, int G, const float* x, const float* b, cons
   if (A.n <= 0) return;
   IMPES_REQUIRE(((uintptr_t)A.ci4 & 15) == 0 && ((uintptr_t)A.v4 & 15) == 0, "padded CSR: arrays not 16-byte aligned");
   if (A.co4) IMPES_REQUIRE(((uintptr_t)A.co4 & 7) == 0, "padded CSR: offsets not 8-byte aligned");
-  if (A.wrow) {
+  if (A.nw > 0) {
     if (A.co4) csr4_tile_launch<MODE, true>(A, x, b, aux, w, y, s);
     else csr4_tile_launch<MODE, false>(A, x, b, aux, w, y, s);
   } else if (A.co4) {
@@ -253,11 +334,10 @@ __global__ void k_csr4_count(int n, const int* __restrict__ rp, int* __restrict_
 }
 
 __global__ void k_csr4_pattern(int n, const int* __restrict__ rp, const int* __restrict__ ci,
-                               const int* __restrict__ rp4, int* __restrict__ ci4, int square) {
+                               const int* __restrict__ rp4, int* __restrict__ ci4) {
   for (long long r = blockIdx.x * (long long)blockDim.x + threadIdx.x; r < n; r += (long long)gridDim.x * blockDim.x) {
     const int e0 = rp[r], len = rp[r + 1] - e0, q0 = rp4[r], len4 = rp4[r + 1] - q0;
-    const int pad = square ? (int)r : (len > 0 ? ci[e0] : 0);
-    for (int k = 0; k < len4; ++k) ci4[q0 + k] = (k < len) ? ci[e0 + k] : pad;
+    for (int k = 0; k < len4; ++k) ci4[q0 + k] = (k < len) ? ci[e0 + k] : (int)r;
   }
 }
 
@@ -656,24 +736,6 @@ void launch_jacobi_f32(const CsrF32& A, const float* xi, const float* b, const f
   KScope ks("csr_jacobi_f32", csr_bytes(A.n_rows, A.nnz, 4, 3), s);
   csr_dispatch<float, float, kJac>(A.n_rows, A.rp, A.ci, A.v, xi, b, inv_relax, w, xo, G, s);
 }
-int csr4_wave_tiles(int n, const int* rp4, std::vector<int>& wrow, std::vector<int>& wq) {
-  wrow.assign(1, 0);
-  wq.assign(1, 0);
-  int cur = 0;
-  for (int r = 0; r < n; ++r) {
-    const int len = (rp4[r + 1] - rp4[r]) >> 2;
-    if (len > kWave) return 0;
-    if (cur + len > kWave) {
-      wrow.push_back(r);
-      wq.push_back(rp4[r] >> 2);
-      cur = 0;
-    }
-    cur += len;
-  }
-  wrow.push_back(n);
-  wq.push_back(rp4[n] >> 2);
-  return (int)wrow.size() - 1;
-}
 int csr4_group_for(int n_rows, long long nnz4) {
   if (n_rows <= 0) return 1;
   // at most one 4-entry chunk per lane on a row of mean length: the smallest power
@@ -689,9 +751,27 @@ void launch_csr4_count(int n, const int* rp, int* cnt, hipStream_t s) {
   k_csr4_count<<<grid_for(n, kBlock, 1 << 16), kBlock, 0, s>>>(n, rp, cnt);
   IMPES_LAUNCH_CHECK();
 }
-void launch_csr4_pattern(int n, const int* rp, const int* ci, const int* rp4, int* ci4, hipStream_t s, bool square) {
+void launch_tile4_count(int n, const int* rp, int* cnt, hipStream_t s) {
+  const int segs = div_up(n, kTileSeg);
+  k_tile4_rows<false><<<div_up(segs, kBlock / kWave), kBlock, 0, s>>>(n, rp, nullptr, cnt, nullptr, nullptr);
+  IMPES_LAUNCH_CHECK();
+}
+void launch_tile4_rows(int n, const int* rp, const long long* base, int* wrow, int* rp4, hipStream_t s) {
+  const int segs = div_up(n, kTileSeg);
+  k_tile4_rows<true><<<div_up(segs, kBlock / kWave), kBlock, 0, s>>>(n, rp, base, nullptr, wrow, rp4);
+  IMPES_LAUNCH_CHECK();
+}
+void launch_tile4_fill(int nw, const int* wrow, const int* rp, const int* ci, const double* v, const int* rp4,
+                       int* ci4, short* co4, float* v4, unsigned short* tag, int* maxabs, bool square, hipStream_t s) {
+  if (nw <= 0) return;
+  k_tile4_fill<<<grid_for(nw, kBlock / kWave, 1 << 16), kBlock, 0, s>>>(
+      nw, wrow, rp, ci, v, rp4, reinterpret_cast<int4*>(ci4), reinterpret_cast<short4*>(co4),
+      reinterpret_cast<float4*>(v4), tag, maxabs, square ? 1 : 0);
+  IMPES_LAUNCH_CHECK();
+}
+void launch_csr4_pattern(int n, const int* rp, const int* ci, const int* rp4, int* ci4, hipStream_t s) {
   if (n <= 0) return;
-  k_csr4_pattern<<<grid_for(n, kBlock, 1 << 16), kBlock, 0, s>>>(n, rp, ci, rp4, ci4, square ? 1 : 0);
+  k_csr4_pattern<<<grid_for(n, kBlock, 1 << 16), kBlock, 0, s>>>(n, rp, ci, rp4, ci4);
   IMPES_LAUNCH_CHECK();
 }
 void launch_csr4_values(int n, const int* rp, const double* v, const int* rp4, float* v4, hipStream_t s) {
@@ -714,14 +794,14 @@ void launch_jacobi4_f32(const Csr4F32& A, int G, const float* xi, const float* b
   csr4_dispatch<kJac>(A, G, xi, b, inv_relax, w, xo, s);
 }
 void launch_spmv4_f32(const Csr4F32& A, const float* x, float* y, hipStream_t s) {
-  IMPES_REQUIRE(A.wrow && !A.co4, "padded transfer: wave tiles and column indices required");
+  IMPES_REQUIRE(A.nw > 0 && !A.co4, "padded transfer: wave tiles and column indices required");
   if (A.n <= 0) return;
   csr4_tile_launch<kY, false>(A, x, nullptr, nullptr, 0.f, y, s);
   IMPES_LAUNCH_CHECK();
 }
 void launch_restrict4_j0_f32(const Csr4F32& R, const float* r, const float* inv_relax_c, float w, float* bc, float* xc,
                              hipStream_t s) {
-  IMPES_REQUIRE(R.wrow && !R.co4, "padded transfer: wave tiles and column indices required");
+  IMPES_REQUIRE(R.nw > 0 && !R.co4, "padded transfer: wave tiles and column indices required");
   if (R.n <= 0) return;
   csr4_tile_launch<kRestrictJ0, false>(R, r, nullptr, inv_relax_c, w, bc, s, xc);
   IMPES_LAUNCH_CHECK();
