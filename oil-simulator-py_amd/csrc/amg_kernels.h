@@ -6,6 +6,8 @@
 
 namespace impes {
 
+class Readback;  // prims.h
+
 constexpr signed char kC = 0;  // coarse point marker (reference: cf_marker 0 = C)
 constexpr signed char kF = 1;  // fine point marker
 
@@ -35,9 +37,10 @@ void launch_cf_split(int n, long long nnz, const int* rp, const int* ci, const u
 // iterated independent-set split on the symmetrised strong graph with the same
 // (deg, hash, index) order: rounds of local-max selection among undecided points,
 // whose undecided neighbours become F, until every point is decided (no lift needed)
+// first (may be null): values fetched with the first test of the rounds
 void launch_cf_split_iterated(int n, long long nnz, const int* rp, const int* ci, const unsigned char* strong,
                               const int* tpos, int* deg, signed char* newc, int* undecided, signed char* cf,
-                              hipStream_t s);
+                              Readback* first, hipStream_t s);
 // cf[i] = C where |a_ii| > ratio * sum_j!=i |a_ij| (Dirichlet-like rows)
 void launch_force_dominant(int n, const int* rp, const int* ci, const double* v, double ratio, signed char* cf,
                            hipStream_t s);
@@ -150,7 +153,7 @@ struct TailArgs {
   void* B = nullptr;  // float (precision 32) or double
 };
 int tail_slices(int n);
-void launch_tail_widths(int n, const int* rp, int* width, hipStream_t s);
+void launch_tail_slices(int n, const int* rp, int* so, hipStream_t s);  // tail_slices(n) + 1 offsets
 size_t tail_ell_bytes(long long lines, int precision);
 void launch_tail_pack(int precision, int n, const int* rp, const int* ci, const double* v, const int* so, void* ell,
                       hipStream_t s);

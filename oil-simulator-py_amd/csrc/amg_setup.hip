@@ -985,22 +985,36 @@ void launch_cf_split(int n, long long nnz, const int* rp, const int* ci, const u
 }
 void launch_cf_split_iterated(int n, long long nnz, const int* rp, const int* ci, const unsigned char* strong,
                               const int* tpos, int* deg, signed char* newc, int* undecided, signed char* cf,
-                              hipStream_t s) {
+                              Readback* first, hipStream_t s) {
   const bool wave = wave_rows_mis(n, nnz);
   if (wave) launch_waves(k_cf_deg_wave, n, s, n, rp, ci, strong, tpos, deg);
   else launch_rows(k_cf_deg, n, s, n, rp, ci, strong, tpos, deg);
   launch_rows(k_mis_init, n, s, n, cf);
+  DevBuf<long long> part;
+  part.alloc(kSumParts);
+  // Rounds until the next test (a round without undecided points changes nothing): a
+  // test waits for the device, about three rounds' time on a small level; 4-6 rounds
+  // decide a level.
+  int batch = n < 32768 ? 3 : 1;
   // the undecided point of highest rank is selected in every round, so at most n rounds
-  for (long long round = 0;; ++round) {
+  for (long long round = 0;; round += batch, batch = n < 32768 ? 2 : 1) {
     IMPES_REQUIRE(round <= n, "amg setup: independent-set split does not terminate");
-    if (wave) {
-      launch_waves(k_mis_select_wave, n, s, n, rp, ci, strong, tpos, (const int*)deg, (const signed char*)cf, newc);
-      launch_waves(k_mis_cover_wave, n, s, n, rp, ci, strong, tpos, (const signed char*)newc, cf, undecided);
-    } else {
-      launch_rows(k_mis_select, n, s, n, rp, ci, strong, tpos, (const int*)deg, (const signed char*)cf, newc);
-      launch_rows(k_mis_cover, n, s, n, rp, ci, strong, tpos, (const signed char*)newc, cf, undecided);
+    for (int q = 0; q < batch; ++q) {
+      if (wave) {
+        launch_waves(k_mis_select_wave, n, s, n, rp, ci, strong, tpos, (const int*)deg, (const signed char*)cf, newc);
+        launch_waves(k_mis_cover_wave, n, s, n, rp, ci, strong, tpos, (const signed char*)newc, cf, undecided);
+      } else {
+        launch_rows(k_mis_select, n, s, n, rp, ci, strong, tpos, (const int*)deg, (const signed char*)cf, newc);
+        launch_rows(k_mis_cover, n, s, n, rp, ci, strong, tpos, (const signed char*)newc, cf, undecided);
+      }
     }
-    if (sum_i32(undecided, n, s) == 0) break;
+    const int m = launch_sum_i32(undecided, n, part.p, s);
+    Readback own;
+    Readback& r = first ? *first : own;
+    const int left = r.sum(part.p, m);
+    r.fetch(s);
+    first = nullptr;
+    if (r[left] == 0) break;
   }
 }
 void launch_force_dominant(int n, const int* rp, const int* ci, const double* v, double ratio, signed char* cf,

@@ -31,11 +31,28 @@ struct EllEntry {
   int c;
 };
 
-// Slice widths of a level: the longest row of each 64 rows. One wave per slice.
-__global__ void k_tail_widths(int n, const int* __restrict__ rp, int* __restrict__ width) {
-  const int r = blockIdx.x * kWave + threadIdx.x;
-  const int len = wave_max(r < n ? rp[r + 1] - rp[r] : 0);
-  if (threadIdx.x == 0) width[blockIdx.x] = len;
+// Slice offsets of a level: the exclusive sums of the longest row of each 64 rows
+// (at most kTailMax / 64 slices) and, behind them, the total. One workgroup.
+__global__ __launch_bounds__(kTailThreads) void k_tail_slices(int n, const int* __restrict__ rp, int* __restrict__ so) {
+  __shared__ int width[kWave];
+  static_assert(kTailMax <= kWave * kWave, "one lane per slice");
+  const int lane = threadIdx.x & (kWave - 1), ns = (n + kWave - 1) / kWave;
+  for (int sl = threadIdx.x / kWave; sl < ns; sl += kTailThreads / kWave) {
+    const int r = sl * kWave + lane;
+    const int len = wave_max(r < n ? rp[r + 1] - rp[r] : 0);
+    if (lane == 0) width[sl] = len;
+  }
+  __syncthreads();
+  if (threadIdx.x >= kWave) return;
+  const int w = lane < ns ? width[lane] : 0;
+  int sum = w;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int u = __shfl_up(sum, d, kWave);
+    if (lane >= d) sum += u;
+  }
+  if (lane < ns) so[lane] = sum - w;
+  if (lane == ns - 1) so[ns] = sum;
 }
 
 // The sliced operator in the cycle's precision: padding entries have value 0 and
@@ -345,8 +362,8 @@ void form(const TailArgs& A, size_t lds, hipStream_t s) {
 
 int tail_slices(int n) { return div_up(n, kWave); }
 
-void launch_tail_widths(int n, const int* rp, int* width, hipStream_t s) {
-  k_tail_widths<<<tail_slices(n), kWave, 0, s>>>(n, rp, width);
+void launch_tail_slices(int n, const int* rp, int* so, hipStream_t s) {
+  k_tail_slices<<<1, kTailThreads, 0, s>>>(n, rp, so);
   IMPES_LAUNCH_CHECK();
 }
 

@@ -1,0 +1,55 @@
+"""The setup's device primitives through hierarchies whose sizes reach their edges
+(exact results: the hierarchy and V-cycle of the oracle): the median of the scaling
+decision in one workgroup and over the whole device, product rows longer than a
+sort's LDS classes, tiles at segment borders."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _csr(A, dev):
+    return (torch.tensor(A.indptr, dtype=torch.int32, device=dev), torch.tensor(A.indices, dtype=torch.int32, device=dev),
+            torch.tensor(A.data, dtype=torch.float64, device=dev))
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 64, 1000, 1025, 32767, 32768, 32769, 300001])
+def test_median_scaling(dev, n):
+    """dhalf_inv is 1/sqrt of the lower median of |a_ii| (spread over 30 orders)."""
+    import impes_hip as H
+
+    d = 10.0 ** np.random.default_rng(n).uniform(-32.0, -7.0, n)
+    d[:: max(1, n // 5)] = d[0]  # ties
+    A = sp.diags(d, format="csr")
+    h = H.AmgHierarchy(max_levels=1, dense_max=1)
+    h.setup_csr(*_csr(A, dev))
+    mid = np.sort(np.maximum(np.abs(d), 1e-30))[(n - 1) // 2]
+    assert float(h.dhalf_inv()[0]) == 1.0 / np.sqrt(mid)
+
+
+@pytest.mark.parametrize("n", [511, 512, 513, 1024, 4097, 6000])
+def test_long_rows_and_segment_borders(dev, n):
+    """A hub coupled to every 13th row: product rows of thousands of terms, above and
+    below the size at which a sort bins its segments."""
+    import impes_hip as H
+    from oracle import amg as oa
+
+    A = sp.lil_matrix(sp.diags([np.full(n, 2.1), np.full(n - 1, -1.0), np.full(n - 1, -1.0)], [0, 1, -1]))
+    hub = n // 2
+    for j in range(0, n, 13):
+        if abs(j - hub) > 1:
+            A[hub, j] = A[j, hub] = -0.6
+            A[j, j] = A[j, j] + 0.6
+            A[hub, hub] = A[hub, hub] + 0.6
+    A = sp.csr_matrix(A)
+    A.sort_indices()
+    kw = dict(coarsest_size=40)
+    ho, h = oa.Hierarchy(A, **kw), H.AmgHierarchy(**kw)
+    h.setup_csr(*_csr(A, dev))
+    assert h.num_levels == len(ho.levels)
+    b = np.random.default_rng(1).standard_normal(n)
+    x = h.vcycle(torch.tensor(b, device=dev)).cpu().numpy()
+    y = ho.vcycle(b)
+    assert np.linalg.norm(x - y) <= 1e-11 * np.linalg.norm(y)
