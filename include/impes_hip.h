@@ -99,6 +99,9 @@ void impes_amg_default_params(impes_amg_params* p);
 /* Replaces ClassicalAMG.__init__ (hierarchy build), src/solver/classical_amg.py:699-938. */
 int impes_amg_create(const impes_amg_params* params, impes_amg** out);
 int impes_amg_destroy(impes_amg* amg);
+/* Device memory of hierarchy builds is kept for the next build when its handle is
+ * destroyed or set up again (at most 4 GiB per device). Gives it back to the device. */
+int impes_release_cached_memory(void);
 int impes_amg_setup_csr(impes_amg* amg, int n, int nnz, const int* rowptr, const int* col, const double* val,
                         void* stream);
 /* Same, from the 7-point stencil; level 0 then runs index-free. */

@@ -346,7 +346,10 @@ Hierarchy::Hierarchy(const AmgParams& p) : prm_(p) {
   graphs_ = !(g && g[0] == '0');
 }
 
-Hierarchy::~Hierarchy() { drop_graphs(); }
+Hierarchy::~Hierarchy() {
+  drop_graphs();
+  pool_->retire();
+}
 
 namespace {
 // Capture-only stream (nothing runs on it): one per thread and device, created on

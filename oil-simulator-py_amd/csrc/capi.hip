@@ -217,6 +217,10 @@ int impes_amg_destroy(impes_amg* amg) {
   return guarded(__func__, [&] { delete amg; });
 }
 
+int impes_release_cached_memory(void) {
+  return guarded(__func__, [&] { release_cached_memory(); });
+}
+
 int impes_amg_setup_csr(impes_amg* amg, int n, int nnz, const int* rowptr, const int* col, const double* val,
                         void* stream) {
   return guarded(__func__, [&] {

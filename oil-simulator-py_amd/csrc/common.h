@@ -157,9 +157,10 @@ __device__ __forceinline__ T block_max(T v, T* lds, T init) {
 // large one becomes a spare that a later allocation of the scope may take (at
 // most twice the size asked for). A spare's previous users were enqueued
 // earlier, so the scope's owner must put all device work of the scope on one
-// stream, and close the scope after synchronising it: closing frees the spares
-// and every slab without live blocks. Outside a scope, blocks of the pool are
-// released at once (hipFree, or the slab when it empties).
+// stream, and close the scope after synchronising it: closing gives the spares and
+// every slab without live blocks to a bounded cache of idle blocks (pool.hip), from
+// which new blocks come. Outside a scope, blocks of the pool are released at once
+// (hipFree, or the slab when it empties), after retire() into the cache.
 class SetupPool {
  public:
   static constexpr size_t kPoolSmall = size_t(1) << 20;
@@ -172,6 +173,9 @@ class SetupPool {
   void release(void* p);
   void open();
   void close();
+  // The owner gives up its blocks: waits for the device once, so that the releases
+  // that follow need not (each hipFree would).
+  void retire();
   size_t slab_bytes() const;  // device memory held in slabs
 
  private:
@@ -179,6 +183,9 @@ class SetupPool {
   Impl* impl();
   std::unique_ptr<Impl> impl_;
 };
+
+// Gives the cached idle blocks of every device back to it.
+void release_cached_memory();
 
 // The pool that DevBuf allocations use on this thread (null outside a scope).
 std::shared_ptr<SetupPool> current_setup_pool();

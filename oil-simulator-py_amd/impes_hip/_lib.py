@@ -114,6 +114,7 @@ SIGNATURES = {
     "impes_amg_default_params": [C.POINTER(AmgParams)],
     "impes_amg_create": [C.POINTER(AmgParams), C.POINTER(_P)],
     "impes_amg_destroy": [_P],
+    "impes_release_cached_memory": [],
     "impes_amg_setup_csr": [_P, _I, _I, _P, _P, _P, _P],
     "impes_amg_setup_st7": [_P, _I, _I, _I, _P, _P, _P, _P, _P],
     "impes_amg_update_csr": [_P, _P, _P],

@@ -14,7 +14,7 @@ from ._lib import AmgParams, ImpesError, SolveStats, call, load, ptr, stream_ptr
 __all__ = [
     "spmv_csr", "spmv_st7", "l1jacobi_csr", "dot", "AmgHierarchy", "FgmresSolver", "amg_default_params",
     "ktimer_reset", "ktimer_read", "copy_f64",
-    "ImpesModel", "csr_diagonal",
+    "ImpesModel", "csr_diagonal", "release_cached_memory",
 ]
 
 
@@ -72,6 +72,11 @@ def copy_f64(y, x):
     assert x.numel() == y.numel() and x.dtype == y.dtype == torch.float64
     call("impes_copy_f64", x.numel(), ptr(x), ptr(y), stream_ptr())
     return y
+
+
+def release_cached_memory():
+    """Give the device memory kept between hierarchy builds (at most 4 GiB) back."""
+    call("impes_release_cached_memory")
 
 
 _KT = {"name": ""}

@@ -1,11 +1,16 @@
 """The setup's device primitives through hierarchies whose sizes reach their edges
 (exact results: the hierarchy and V-cycle of the oracle): the median of the scaling
 decision in one workgroup and over the whole device, product rows longer than a
-sort's LDS classes, tiles at segment borders."""
+sort's LDS classes, tiles at segment borders; and the reuse of a destroyed
+hierarchy's memory by the next build, also from other threads and streams."""
+import threading
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
 import torch
+
+from matrices import impes_like, laplacian_2d
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +58,63 @@ def test_long_rows_and_segment_borders(dev, n):
     x = h.vcycle(torch.tensor(b, device=dev)).cpu().numpy()
     y = ho.vcycle(b)
     assert np.linalg.norm(x - y) <= 1e-11 * np.linalg.norm(y)
+
+
+def test_memory_of_destroyed_hierarchies(dev):
+    """Build, use and drop hierarchies from several threads on streams of their own:
+    every result equals the first one's bits; the kept memory is given back."""
+    import impes_hip as H
+
+    sizes = [(20, 18, 9), (30, 20, 11), (25, 25, 4)]
+    want = {}
+
+    def once(dims):
+        A, *_ = impes_like(*dims, seed=3)
+        b = torch.tensor(np.random.default_rng(2).standard_normal(A.shape[0]), device=dev)
+        h = H.AmgHierarchy()
+        h.setup_csr(*_csr(A, dev))
+        x = h.precondition(b, precision=32)
+        h.close()
+        return x
+
+    for d in sizes:
+        want[d] = once(d).cpu()
+    bad = []
+
+    def work(k):
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            for q in range(6):
+                d = sizes[(k + q) % len(sizes)]
+                x = once(d)
+                st.synchronize()
+                if not torch.equal(x.cpu(), want[d]):
+                    bad.append((k, q, d))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not bad
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    H.release_cached_memory()
+    assert torch.cuda.mem_get_info()[0] > before
+
+
+def test_update_after_a_reused_build(dev):
+    """A numeric update of a hierarchy in reused memory equals a fresh one's."""
+    import impes_hip as H
+
+    A = laplacian_2d(70)
+    A = (A + sp.identity(A.shape[0]) * 1e-3).tocsr()
+    A.sort_indices()
+    out = []
+    for _ in range(2):
+        h = H.AmgHierarchy()
+        h.setup_csr(*_csr(A, dev))
+        h.update_csr(_csr(A * 1.5, dev)[2])
+        out.append(h.vcycle(torch.ones(A.shape[0], dtype=torch.float64, device=dev)))
+        h.close()
+    assert torch.equal(*out)
