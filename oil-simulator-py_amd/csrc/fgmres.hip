@@ -22,7 +22,7 @@ namespace impes {
 
 namespace {
 
-constexpr int kGsThreads = 256;
+constexpr int kGsThreads = 512;
 using Layout = FgmresLayout;
 
 // sc[0] = beta = sqrt(sc[4]) ; g = beta e1
@@ -150,15 +150,19 @@ __global__ void k_fold_cols(const double* __restrict__ part, int nb, double* __r
   if (threadIdx.x == 0) out[c] = s;
 }
 
-// Workgroups of a Gram-Schmidt pass: each folds its rows' k products per column
-// with wavefront shuffles, so more rows per thread amortise the folds (1024: 1%
-// faster per time step than 2048 at 1M cells; 512 and 256 no better).
-constexpr int kGsBlocks = 1024;
+// Workgroups of a Gram-Schmidt pass over n rows: at least two rows per thread (each
+// workgroup folds its rows' products and leaves one partial per column, which the
+// Hessenberg kernels read), at most kGsBlocks of 512 threads (1024 of 256 keep as many
+// waves and leave twice the partials). With the halving fold (wave_fold) a dots pass
+// of 8 columns takes 12.9 us at 1M rows and 5.4 us at 200,000, where 1024 workgroups
+// at every size and six shuffles per sum and lane took 18.0 and 12.0 us.
+constexpr int kGsBlocks = 512;
 static_assert(kGsBlocks <= kMultiDotBlocks, "the partials workspace is sized for kMultiDotBlocks");
+int gs_blocks(long long n) { return grid_for(n, 2 * kGsThreads, kGsBlocks); }
 
 template <int PASS>
 void launch_gs_pass(int k, double* w, const double* V, long long n, const double* h, double* part, hipStream_t s) {
-  const int nb = kGsBlocks;
+  const int nb = gs_blocks(n);
   if (k <= 4)
     k_gs_pass<4, PASS><<<nb, kGsThreads, 0, s>>>(k, w, V, n, h, part);
   else if (k <= 8)
@@ -201,13 +205,6 @@ __global__ void k_arnoldi(Layout L, int j, double* __restrict__ sm, const double
 // stops after step j).
 // P lanes share a row (P = 1 or 2), lane h of the pair taking columns t = h + P m:
 // the accumulators (and coefficients) per thread fall from 2K to 2K/P doubles.
-template <int P, class T>
-__device__ __forceinline__ T pair_sum(T v) {  // sum over the lanes of one column set (xor offsets >= P)
-#pragma unroll
-  for (int off = kWave / 2; off >= P; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
-}
-
 template <int K, int P, int R>
 __global__ __launch_bounds__(kGsThreads) void k_lag_dots(int k, const double* __restrict__ V, long long n,
                                                          const double* __restrict__ u, const double* __restrict__ w,
@@ -260,23 +257,19 @@ __global__ __launch_bounds__(kGsThreads) void k_lag_dots(int k, const double* __
     }
   }
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  {  // all columns at once: aa then cc, lane set h = lane % P holding columns h + P m
+    double f[2 * KP];
 #pragma unroll
-  for (int m = 0; m < KP; ++m) {
-    if (P * m < k) {
-      const double x = pair_sum<P>(aa[m]), y = pair_sum<P>(cc[m]);
-      const int t = lane + P * m;  // lanes 0..P-1 hold the sums of columns P m .. P m + P - 1
-      if (lane < P && t < k) {
-        lds[wid * NC + t] = x;
-        lds[wid * NC + K + t] = y;
-      }
+    for (int m = 0; m < KP; ++m) {
+      f[m] = aa[m];
+      f[KP + m] = cc[m];
     }
-  }
-  {
-    const double x = wave_sum(ss), y = wave_sum(dd);
-    if (lane == 0) {
-      lds[wid * NC + 2 * K] = x;
-      lds[wid * NC + 2 * K + 1] = y;
-    }
+    const double v = wave_fold<2 * KP, P>(f);
+    const int q = fold_index<2 * KP>(lane), t = h + P * (q % KP);
+    if (lane % (kWave / (2 * KP)) < P && t < k) lds[wid * NC + (q < KP ? 0 : K) + t] = v;
+    double g[2] = {ss, dd};
+    const double w2 = wave_fold<2>(g);
+    if (lane % (kWave / 2) == 0) lds[wid * NC + 2 * K + fold_index<2>(lane)] = w2;
   }
   __syncthreads();
   // partial columns: a_t -> t, c_t -> k + t, s -> 2k, d -> 2k + 1
@@ -514,21 +507,21 @@ void launch_lag_pair(int k, double* V, long long n, const double* w, double* sm,
   auto a16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   const bool two = n % 2 == 0 && a16(V) && a16(w) && (dots_only ? a16(u) : (a16(S) && bout != nullptr));
   if (dots_only) {
-    if (two) k_lag_dots<K, P, 2><<<kGsBlocks, kGsThreads, 0, s>>>(k, V, n, u, w, part);
-    else k_lag_dots<K, P, 1><<<kGsBlocks, kGsThreads, 0, s>>>(k, V, n, u, w, part);
+    if (two) k_lag_dots<K, P, 2><<<gs_blocks(n), kGsThreads, 0, s>>>(k, V, n, u, w, part);
+    else k_lag_dots<K, P, 1><<<gs_blocks(n), kGsThreads, 0, s>>>(k, V, n, u, w, part);
   } else if (precision == 32) {
     if (two)
-      k_lag_update<K, P, float, 2><<<kGsBlocks, kGsThreads, 0, s>>>(k, V, n, w, sm + L.h(), sm + L.h2(), sm + L.lag(),
+      k_lag_update<K, P, float, 2><<<gs_blocks(n), kGsThreads, 0, s>>>(k, V, n, w, sm + L.h(), sm + L.h2(), sm + L.lag(),
                                                                     S, (float*)bout, part);
     else
-      k_lag_update<K, P, float, 1><<<kGsBlocks, kGsThreads, 0, s>>>(k, V, n, w, sm + L.h(), sm + L.h2(), sm + L.lag(),
+      k_lag_update<K, P, float, 1><<<gs_blocks(n), kGsThreads, 0, s>>>(k, V, n, w, sm + L.h(), sm + L.h2(), sm + L.lag(),
                                                                     S, (float*)bout, part);
   } else {
     if (two)
-      k_lag_update<K, P, double, 2><<<kGsBlocks, kGsThreads, 0, s>>>(k, V, n, w, sm + L.h(), sm + L.h2(),
+      k_lag_update<K, P, double, 2><<<gs_blocks(n), kGsThreads, 0, s>>>(k, V, n, w, sm + L.h(), sm + L.h2(),
                                                                      sm + L.lag(), S, (double*)bout, part);
     else
-      k_lag_update<K, P, double, 1><<<kGsBlocks, kGsThreads, 0, s>>>(k, V, n, w, sm + L.h(), sm + L.h2(),
+      k_lag_update<K, P, double, 1><<<gs_blocks(n), kGsThreads, 0, s>>>(k, V, n, w, sm + L.h(), sm + L.h2(),
                                                                      sm + L.lag(), S, (double*)bout, part);
   }
   IMPES_LAUNCH_CHECK();
@@ -777,12 +770,12 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
           // or by the cycle's normalisation for j = 0), w = D^-1 A z_j
           precondition_apply(vj, zj);
           launch_lag(j, V, n, w_.p, sm, L, nullptr, nullptr, precision, work_.p, true, vj, s);
-          k_lag_colA<<<1, kColAThreads, 0, s>>>(L, j, sm, work_.p, kGsBlocks);
+          k_lag_colA<<<1, kColAThreads, 0, s>>>(L, j, sm, work_.p, gs_blocks(n));
           IMPES_LAUNCH_CHECK();
           final_cols = j;
           launch_lag(j, V, n, w_.p, sm, L, M->in_scale(), M->vcycle_in(precision), precision, work_.p, false,
                      nullptr, s);
-          k_lag_colB<<<1, kColAThreads, 0, s>>>(L, j, sm, work_.p, kGsBlocks, est);
+          k_lag_colB<<<1, kColAThreads, 0, s>>>(L, j, sm, work_.p, gs_blocks(n), est);
           IMPES_LAUNCH_CHECK();
         } else {
         precondition_apply(vj, zj);
@@ -791,10 +784,10 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
         const int kj = j + 1;
         if (kj <= kMaxFusedGs) {
           launch_gs_pass<0>(kj, w_.p, V, n, nullptr, work_.p, s);
-          k_fold_cols<<<kj, kGsThreads, 0, s>>>(work_.p, kGsBlocks, sm + L.h());
+          k_fold_cols<<<kj, kGsThreads, 0, s>>>(work_.p, gs_blocks(n), sm + L.h());
           IMPES_LAUNCH_CHECK();
           launch_gs_pass<1>(kj, w_.p, V, n, sm + L.h(), work_.p, s);
-          k_fold_cols<<<kj, kGsThreads, 0, s>>>(work_.p, kGsBlocks, sm + L.h2());
+          k_fold_cols<<<kj, kGsThreads, 0, s>>>(work_.p, gs_blocks(n), sm + L.h2());
           IMPES_LAUNCH_CHECK();
           launch_gs_pass<2>(kj, w_.p, V, n, sm + L.h2(), work_.p, s);
         } else {
@@ -804,7 +797,7 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
           launch_gs_update_f64(w_.p, V, n, kj, sm + L.h2(), n, s);
           launch_dot_partial_f64(w_.p, w_.p, n, work_.p, kMultiDotBlocks, s);
         }
-        k_arnoldi<<<1, kGsThreads, 0, s>>>(L, j, sm, work_.p, kj <= kMaxFusedGs ? kGsBlocks : kMultiDotBlocks, est);
+        k_arnoldi<<<1, kGsThreads, 0, s>>>(L, j, sm, work_.p, kj <= kMaxFusedGs ? gs_blocks(n) : kMultiDotBlocks, est);
         IMPES_LAUNCH_CHECK();
         normalize(V + (long long)(j + 1) * n, w_.p, sc + 3);
         }
@@ -849,7 +842,7 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
         // close column k-1: dots of u = V[:, k] against v_0..v_{k-1}, then its colA
         const double* uk = V + (long long)k * n;
         launch_lag(k, V, n, uk, sm, L, nullptr, nullptr, precision, work_.p, true, uk, s);
-        k_lag_colA<<<1, kColAThreads, 0, s>>>(L, k, sm, work_.p, kGsBlocks);
+        k_lag_colA<<<1, kColAThreads, 0, s>>>(L, k, sm, work_.p, gs_blocks(n));
         IMPES_LAUNCH_CHECK();
       }
       if (k <= kBackLanes) k_backsolve_wave<<<1, kBackLanes, 0, s>>>(L, k, sm);

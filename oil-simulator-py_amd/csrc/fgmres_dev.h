@@ -33,25 +33,29 @@ __device__ __forceinline__ void givens(double a, double b, double& c, double& s)
   else { const double t = b / a; c = 1.0 / sqrt(1.0 + t * t); s = c * t; }
 }
 
-// Sums of NV values (a power of two up to 64) over the wave's lanes: each step sends
-// half of a lane's values to its partner, so NV values take NV - 1 + log2(64 / NV)
-// shuffles instead of 6 NV. Returns the sum of value fold_index<NV>(lane).
-template <int NV>
-__device__ __forceinline__ double wave_fold(double (&v)[NV]) {
-  const int lane = threadIdx.x & (kWave - 1);
-  int off = kWave / 2;
+// Sums of NV values (a power of two, NV P <= 64) over the wave's lanes of equal
+// lane % P: each step sends half of a lane's values to its partner, so NV values take
+// NV - 1 + log2(64 / (NV P)) shuffles instead of NV log2(64 / P). Returns the sum of
+// value fold_index<NV>(lane).
+template <int M, int OFF, int P, int NV>
+__device__ __forceinline__ void fold_steps(double (&v)[NV], int lane) {
+  if constexpr (M >= 1) {
+    const bool hi = (lane & OFF) != 0;
 #pragma unroll
-  for (int m = NV / 2; m >= 1; m /= 2) {
-    const bool hi = (lane & off) != 0;
-#pragma unroll
-    for (int q = 0; q < m; ++q) {
-      const double send = hi ? v[q] : v[q + m], keep = hi ? v[q + m] : v[q];
-      v[q] = keep + __shfl_xor(send, off, kWave);
+    for (int q = 0; q < M; ++q) {
+      const double send = hi ? v[q] : v[q + M], keep = hi ? v[q + M] : v[q];
+      v[q] = keep + __shfl_xor(send, OFF, kWave);
     }
-    off /= 2;
+    fold_steps<M / 2, OFF / 2, P>(v, lane);
+  } else if constexpr (OFF >= P) {
+    v[0] += __shfl_xor(v[0], OFF, kWave);
+    fold_steps<0, OFF / 2, P>(v, lane);
   }
-#pragma unroll
-  for (; off >= 1; off /= 2) v[0] += __shfl_xor(v[0], off, kWave);
+}
+template <int NV, int P = 1>
+__device__ __forceinline__ double wave_fold(double (&v)[NV]) {
+  static_assert(NV * P <= kWave, "one value per lane at the end");
+  fold_steps<NV / 2, kWave / 2, P>(v, threadIdx.x & (kWave - 1));
   return v[0];
 }
 template <int NV>
