@@ -35,7 +35,7 @@ enum WellSlot {
   kWellSlots = 16,
 };
 
-constexpr int kWellScratch = 9;  // per-well scratch row of the transport step's well loop
+constexpr int kWellScratch = 3;  // per-well scratch row of the well kernels (wells that share a cell)
 
 struct Grid {
   int nx, ny, nz;
@@ -122,6 +122,8 @@ class Model {
   bool gravity_ = false;
   DevBuf<double> pvt_P_, pvt_col_, pvt_slope_;
   DevBuf<WellDesc> wells_;
+  DevBuf<int> well_link_;  // chains of the wells that share a cell (2 per well)
+  int wells_shared_ = 0;   // whether one does
   // pinned staging of the well descriptors; `ev` marks when the last upload has
   // left it
   struct Staging {

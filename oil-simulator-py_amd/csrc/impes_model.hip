@@ -1,9 +1,11 @@
 // IMPES step kernels and their host orchestration.
+#include "fgmres_dev.h"
 #include "impes_model.h"
 #include "model_dev.h"
 
 #include <cstring>
 
+#include <algorithm>
 #include <cmath>
 
 // Products and sums are rounded separately (no fused multiply-add), as in the
@@ -15,6 +17,21 @@ namespace impes {
 
 namespace {
 using namespace model_dev;
+// Sums of NV values (a power of two) over the workgroup, in a fixed order: a wave folds
+// all its values by halving (wave_fold), LDS joins the waves. Thread q < NV returns the
+// sum of value q. `lds`: NV slots per wave.
+template <int NV>
+__device__ __forceinline__ double block_fold(double (&v)[NV], double* lds) {
+  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  const double s = wave_fold(v);
+  if (lane % (kWave / NV) == 0) lds[wid * NV + fold_index<NV>(lane)] = s;
+  __syncthreads();
+  double r = 0.0;
+  if (threadIdx.x < NV)
+    for (int w = 0; w < (int)(blockDim.x / kWave); ++w) r += lds[w * NV + threadIdx.x];
+  return r;
+}
+
 constexpr int kLedgerQ = 10;  // mass(6) + volume dV_w, dV_g, clamp_w, clamp_g
 
 // ---------------------------------------------------------------- transmissibility
@@ -143,15 +160,25 @@ __global__ void k_assemble(GridDev G, FluidParams F, const double* __restrict__ 
   }
 }
 
-// _calculate_well_terms (:1622-1660), applied in well order by one thread.
-// One thread per well computes its diagonal and right-hand-side increments (into
-// ws[2 w], ws[2 w + 1]) and report slots; one thread then adds the increments in
-// well order (the serial loop's accumulation, bit for bit). One workgroup.
+// Wells of one cell form a chain: link[2 w] is the cell's first well, link[2 w + 1] the
+// next one after w (-1: none). Several wells of a cell add to it in well order (the
+// serial loop's accumulation, bit for bit), by the thread of the first; wells of
+// different cells are independent, so nothing else is serial.
+__device__ __forceinline__ bool well_lone(const int* __restrict__ link, int w) {
+  return link[2 * w] == w && link[2 * w + 1] < 0;
+}
+
+// _calculate_well_terms (:1622-1660). One thread per well computes its diagonal and
+// right-hand-side increments and report slots and, where the well has its cell to
+// itself (every well unless `shared`), adds them; the others leave them in
+// ws[2 w], ws[2 w + 1] for the first well's thread. One workgroup: latency is all it
+// costs (a serial thread over the wells took 128 us for 256 wells, 3.2 us).
 __global__ __launch_bounds__(256) void k_wells_pressure(FluidParams F, int nw, const WellDesc* __restrict__ W,
                                                         const double* __restrict__ p, const double* __restrict__ mt,
                                                         double* __restrict__ diag, double* __restrict__ b,
                                                         double* __restrict__ dinv, double* __restrict__ rep,
-                                                        double* __restrict__ ws) {
+                                                        double* __restrict__ ws, const int* __restrict__ link,
+                                                        int shared) {
   for (int w = threadIdx.x; w < nw; w += blockDim.x) {
     double* R = rep + kReportHead + kWellSlots * w;
     const WellDesc& d = W[w];
@@ -187,17 +214,30 @@ __global__ __launch_bounds__(256) void k_wells_pressure(FluidParams F, int nw, c
       dd = term;
       db = term * (d.value * 1e6);
     }
-    ws[2 * w] = dd;
-    ws[2 * w + 1] = db;
+    if (!shared || well_lone(link, w)) {
+      const double a = diag[c] + dd;
+      diag[c] = a;
+      b[c] += db;
+      dinv[c] = 1.0 / a;
+    } else {
+      ws[2 * w] = dd;
+      ws[2 * w + 1] = db;
+    }
   }
+  if (!shared) return;
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int w = 0; w < nw; ++w) {
+  for (int w = threadIdx.x; w < nw; w += blockDim.x) {
+    if (link[2 * w] != w || link[2 * w + 1] < 0) continue;
     const int c = W[w].cell;
-    diag[c] += ws[2 * w];
-    b[c] += ws[2 * w + 1];
+    double a = diag[c], r = b[c];
+    for (int v = w; v >= 0; v = link[2 * v + 1]) {
+      a += ws[2 * v];
+      r += ws[2 * v + 1];
+    }
+    diag[c] = a;
+    b[c] = r;
+    dinv[c] = 1.0 / a;
   }
-  for (int w = 0; w < nw; ++w) dinv[W[w].cell] = 1.0 / diag[W[w].cell];
 }
 
 // ---------------------------------------------------------------- transport
@@ -281,6 +321,8 @@ struct SatWellCtx {
   double dt;
   int nw;
   const WellDesc* W;
+  const int* link;  // wells of one cell (well_lone)
+  int shared;       // some cell holds several wells
   const double* p_prev;
   const double* p;
   const double* sw;
@@ -316,20 +358,21 @@ __device__ double row_balance(const SatWellCtx& X, int c, double q_rate) {
 
 // The per-well loop of the transport step (simulation.py:1051-1347). Each well's
 // terms depend only on its cell's state and on the pressure step's report, so one
-// thread per well computes them into its scratch row ws[9 w ..] (cell increments
-// of qw, qg, qo; oil in/out, gas in/out; volume sums of qw, qg); then one thread
-// adds the rows in well order, which gives the sums and the per-cell accumulation
-// of the serial loop bit for bit. One workgroup.
-enum WellScratch { kWsQW = 0, kWsQG, kWsQO, kWsOilIn, kWsOilOut, kWsGasIn, kWsGasOut, kWsSumQW, kWsSumQG,
-                   kWsLen };
-static_assert(kWsLen == kWellScratch, "well scratch row length");
-
+// thread per well computes them: the increments of qw, qg, qo go to the cell (or, for
+// wells that share one, through the scratch row ws[3 w ..] to the first well's thread,
+// which adds them in well order), and the oil in/out, gas in/out and volume sums are
+// folded over the workgroup in a fixed order. One workgroup: latency is all it costs (a
+// serial thread adding up 256 wells took 125 us, this 12 us: dependent loads that miss).
 __global__ __launch_bounds__(256) void k_wells_sat(SatWellCtx X, double* __restrict__ qw, double* __restrict__ qg,
                                                    double* __restrict__ qo, double* __restrict__ rep,
                                                    double* __restrict__ ws) {
+  __shared__ double lds[8 * (256 / kWave)];
   const FluidParams& F = X.F;
   const bool pvt = X.T.n > 0;
   const double dt = X.dt;
+  const int* __restrict__ link = X.link;
+  // oil in, oil out, gas in, gas out, sums of qw and qg (a power of two of slots)
+  double tot[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   for (int w = threadIdx.x; w < X.nw; w += blockDim.x) {
     double dqw = 0.0, dqg = 0.0, dqo = 0.0;
     double oil_in = 0.0, oil_out = 0.0, gas_in = 0.0, gas_out = 0.0, sum_qw = 0.0, sum_qg = 0.0;
@@ -435,8 +478,7 @@ __global__ __launch_bounds__(256) void k_wells_sat(SatWellCtx X, double* __restr
       // well with a pressure-equation diagonal term in the cell
       int nterm = 0;
       double q_rate = 0.0;
-      for (int v = 0; v < X.nw; ++v) {
-        if (X.W[v].cell != c) continue;
+      for (int v = link[2 * w]; v >= 0; v = link[2 * v + 1]) {
         const double* Rv = rep + kReportHead + kWellSlots * v;
         if (Rv[kWTerm] != 0.0) ++nterm;
         q_rate += Rv[kWQRate];
@@ -486,39 +528,43 @@ __global__ __launch_bounds__(256) void k_wells_sat(SatWellCtx X, double* __restr
         }
       }
     }
-    double* r = ws + (long long)kWsLen * w;
-    r[kWsQW] = dqw;
-    r[kWsQG] = dqg;
-    r[kWsQO] = dqo;
-    r[kWsOilIn] = oil_in;
-    r[kWsOilOut] = oil_out;
-    r[kWsGasIn] = gas_in;
-    r[kWsGasOut] = gas_out;
-    r[kWsSumQW] = sum_qw;
-    r[kWsSumQG] = sum_qg;
+    if (!X.shared || well_lone(link, w)) {
+      qw[c] += dqw;
+      qg[c] += dqg;
+      qo[c] += dqo;
+    } else {
+      double* r = ws + (long long)kWellScratch * w;
+      r[0] = dqw;
+      r[1] = dqg;
+      r[2] = dqo;
+    }
+    tot[0] += oil_in;
+    tot[1] += oil_out;
+    tot[2] += gas_in;
+    tot[3] += gas_out;
+    tot[4] += sum_qw;
+    tot[5] += sum_qg;
   }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  double oil_in = 0.0, oil_out = 0.0, gas_in = 0.0, gas_out = 0.0, sum_qw = 0.0, sum_qg = 0.0;
-  for (int w = 0; w < X.nw; ++w) {
-    const double* r = ws + (long long)kWsLen * w;
-    const int c = X.W[w].cell;
-    qw[c] += r[kWsQW];
-    qg[c] += r[kWsQG];
-    qo[c] += r[kWsQO];
-    oil_in += r[kWsOilIn];
-    oil_out += r[kWsOilOut];
-    gas_in += r[kWsGasIn];
-    gas_out += r[kWsGasOut];
-    sum_qw += r[kWsSumQW];
-    sum_qg += r[kWsSumQG];
+  const double f = block_fold(tot, lds);  // also the barrier before the rows of ws are read
+  if (X.shared) {
+    for (int w = threadIdx.x; w < X.nw; w += blockDim.x) {
+      if (link[2 * w] != w || link[2 * w + 1] < 0) continue;
+      const int c = X.W[w].cell;
+      double a = qw[c], g = qg[c], o = qo[c];
+      for (int v = w; v >= 0; v = link[2 * v + 1]) {
+        const double* r = ws + (long long)kWellScratch * v;
+        a += r[0];
+        g += r[1];
+        o += r[2];
+      }
+      qw[c] = a;
+      qg[c] = g;
+      qo[c] = o;
+    }
   }
-  rep[kCompOIn] = oil_in;
-  rep[kCompOOut] = oil_out;
-  rep[kCompGIn] = gas_in;
-  rep[kCompGOut] = gas_out;
-  rep[kVolQW] = dt * sum_qw;
-  rep[kVolQG] = dt * sum_qg;
+  const int t = threadIdx.x;
+  if (t < 4) rep[kCompOIn + t] = f;
+  else if (t < 6) rep[kVolQW + t - 4] = dt * f;
 }
 
 // NaN/inf-propagating max (torch.max semantics)
@@ -693,7 +739,7 @@ __global__ void k_ledger_fold(int nb, const double* __restrict__ part, double* _
 __global__ __launch_bounds__(256) void k_substep_ledger(SatWellCtx X, const double* __restrict__ dsw,
                                                         const double* __restrict__ dsg, double* __restrict__ rep,
                                                         const double* __restrict__ nsub, long long env_cells) {
-  __shared__ double lds[256 / kWave];
+  __shared__ double lds[4 * (256 / kWave)];
   const FluidParams& F = X.F;
   const int N_all = (int)rep[kNSub];
   // stacked reservoirs: each well uses its own reservoir's count, at most max_substeps
@@ -764,22 +810,15 @@ __global__ __launch_bounds__(256) void k_substep_ledger(SatWellCtx X, const doub
       }
     }
   }
-  oil_in = block_sum(oil_in, lds);
-  oil_out = block_sum(oil_out, lds);
-  gas_in = block_sum(gas_in, lds);
-  gas_out = block_sum(gas_out, lds);
-  if (threadIdx.x == 0) {
-    rep[kCompOIn] += oil_in;
-    rep[kCompOOut] += oil_out;
-    rep[kCompGIn] += gas_in;
-    rep[kCompGOut] += gas_out;
-  }
+  double tot[4] = {oil_in, oil_out, gas_in, gas_out};
+  const double f = block_fold(tot, lds);
+  if (threadIdx.x < 4) rep[kCompOIn + threadIdx.x] += f;
 }
 
 __global__ void k_reset_wells(int nw, const WellDesc* __restrict__ W, double* __restrict__ qw, double* __restrict__ qg,
                               double* __restrict__ qo) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  for (int w = 0; w < nw; ++w) {
+  const int w = blockIdx.x * blockDim.x + threadIdx.x;
+  if (w < nw) {
     const int c = W[w].cell;
     qw[c] = 0.0;
     qg[c] = 0.0;
@@ -855,11 +894,34 @@ Model::Staging::~Staging() {
   if (p) (void)hipHostFree(p);
 }
 
+namespace {
+// Chains of the wells that share a cell (k_wells_pressure); returns whether one does.
+int link_wells(const std::vector<WellDesc>& w, int* link) {
+  const int n = (int)w.size();
+  std::vector<int> order(n);
+  for (int i = 0; i < n; ++i) {
+    order[i] = link[2 * i] = i;
+    link[2 * i + 1] = -1;
+  }
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return w[a].cell < w[b].cell; });
+  int shared = 0;
+  for (int i = 1; i < n; ++i) {
+    const int a = order[i - 1], b = order[i];
+    if (w[a].cell != w[b].cell) continue;
+    link[2 * a + 1] = b;
+    link[2 * b] = link[2 * a];
+    shared = 1;
+  }
+  return shared;
+}
+}  // namespace
+
 void Model::set_wells(const std::vector<WellDesc>& w, hipStream_t s) {
   for (const auto& d : w) IMPES_REQUIRE(d.cell >= 0 && d.cell < N_, "model: well outside the grid");
   nw_ = (int)w.size();
   if (nw_ > 0) {
     wells_.reserve(nw_);
+    well_link_.reserve(2 * (size_t)nw_);
     well_sc_.reserve((size_t)kWellScratch * nw_);
     if (!stage_.ev) IMPES_HIP_CHECK(hipEventCreateWithFlags(&stage_.ev, hipEventDisableTiming));
     IMPES_HIP_CHECK(hipEventSynchronize(stage_.ev));  // the last upload has left the staging
@@ -867,11 +929,15 @@ void Model::set_wells(const std::vector<WellDesc>& w, hipStream_t s) {
       if (stage_.p) IMPES_HIP_CHECK(hipHostFree(stage_.p));
       stage_.p = nullptr;
       stage_.cap = 0;
-      IMPES_HIP_CHECK(hipHostMalloc((void**)&stage_.p, sizeof(WellDesc) * nw_, hipHostMallocDefault));
+      IMPES_HIP_CHECK(hipHostMalloc((void**)&stage_.p, (sizeof(WellDesc) + 2 * sizeof(int)) * nw_,
+                                    hipHostMallocDefault));
       stage_.cap = nw_;
     }
     std::memcpy(stage_.p, w.data(), sizeof(WellDesc) * nw_);
+    int* link = reinterpret_cast<int*>(stage_.p + nw_);
+    wells_shared_ = link_wells(w, link);
     IMPES_HIP_CHECK(hipMemcpyAsync(wells_.p, stage_.p, sizeof(WellDesc) * nw_, hipMemcpyHostToDevice, s));
+    IMPES_HIP_CHECK(hipMemcpyAsync(well_link_.p, link, 2 * sizeof(int) * nw_, hipMemcpyHostToDevice, s));
     IMPES_HIP_CHECK(hipEventRecord(stage_.ev, s));
   }
   report_.reserve(report_len());
@@ -914,7 +980,8 @@ void Model::assemble(double dt, const double* p, const double* sw, const double*
                                    rho_o_.p, rho_g_.p, pc_.p, acc.p, diag.p, ox.p, oy.p, oz.p, b.p, extra.p, dinv.p);
   IMPES_LAUNCH_CHECK();
   if (nw_ > 0) {
-    k_wells_pressure<<<1, 256, 0, s>>>(F, nw_, wells_.p, p, mob_t.p, diag.p, b.p, dinv.p, report_.p, well_sc_.p);
+    k_wells_pressure<<<1, 256, 0, s>>>(F, nw_, wells_.p, p, mob_t.p, diag.p, b.p, dinv.p, report_.p, well_sc_.p,
+                                       well_link_.p, wells_shared_);
     IMPES_LAUNCH_CHECK();
   }
 }
@@ -982,7 +1049,7 @@ void Model::saturation(double dt, const double* p_prev, const double* p_new, con
   k_flux<<<gr, kBlock, 0, s>>>(G, F, p_new, tx.p, ty.p, tz.p, mob_w_.p, mob_g_.p, rho_w_.p, rho_g_.p, pcog_.p,
                                div_w_.p, div_g_.p);
   IMPES_LAUNCH_CHECK();
-  SatWellCtx X{G, F, pvt, dt, nw_, wells_.p, p_prev, p_new, sw, sg, pv.p, mob_w_.p, mob_o_.p, mob_g_.p, mob_t.p,
+  SatWellCtx X{G, F, pvt, dt, nw_, wells_.p, well_link_.p, wells_shared_, p_prev, p_new, sw, sg, pv.p, mob_w_.p, mob_o_.p, mob_g_.p, mob_t.p,
                ox.p, oy.p, oz.p, acc.p, extra.p};
   // head slots written below must start from zero each step
   k_wells_sat<<<1, 256, 0, s>>>(X, qw_.p, qg_.p, qo_.p, report_.p, well_sc_.p);
@@ -1007,7 +1074,7 @@ void Model::saturation(double dt, const double* p_prev, const double* p_new, con
     IMPES_LAUNCH_CHECK();
   }
   if (nw_ > 0) {
-    k_reset_wells<<<1, 1, 0, s>>>(nw_, wells_.p, qw_.p, qg_.p, qo_.p);
+    k_reset_wells<<<grid_for(nw_, kBlock), kBlock, 0, s>>>(nw_, wells_.p, qw_.p, qg_.p, qo_.p);
     IMPES_LAUNCH_CHECK();
   }
   IMPES_HIP_CHECK(hipMemcpyAsync(host_report, report_.p, sizeof(double) * report_len(), hipMemcpyDeviceToHost, s));
@@ -1024,7 +1091,7 @@ void Model::transport_forward(double dt, const double* p_prev, const double* p_n
   k_flux<<<gr, kBlock, 0, s>>>(G, F, p_new, tx.p, ty.p, tz.p, mob_w_.p, mob_g_.p, rho_w_.p, rho_g_.p, pcog_.p,
                                div_w_.p, div_g_.p);
   IMPES_LAUNCH_CHECK();
-  SatWellCtx X{G, F, pvt, dt, nw_, wells_.p, p_prev, p_new, sw, sg, pv.p, mob_w_.p, mob_o_.p, mob_g_.p, mob_t.p,
+  SatWellCtx X{G, F, pvt, dt, nw_, wells_.p, well_link_.p, wells_shared_, p_prev, p_new, sw, sg, pv.p, mob_w_.p, mob_o_.p, mob_g_.p, mob_t.p,
                ox.p, oy.p, oz.p, acc.p, extra.p};
   k_wells_sat<<<1, 256, 0, s>>>(X, qw_.p, qg_.p, qo_.p, report_.p, well_sc_.p);
   IMPES_LAUNCH_CHECK();
@@ -1034,7 +1101,7 @@ void Model::transport_forward(double dt, const double* p_prev, const double* p_n
   k_nsub<<<1, kBlock, 0, s>>>(kRedBlocks, F, part_.p, report_.p);
   IMPES_LAUNCH_CHECK();
   if (nw_ > 0) {
-    k_reset_wells<<<1, 1, 0, s>>>(nw_, wells_.p, qw_.p, qg_.p, qo_.p);
+    k_reset_wells<<<grid_for(nw_, kBlock), kBlock, 0, s>>>(nw_, wells_.p, qw_.p, qg_.p, qo_.p);
     IMPES_LAUNCH_CHECK();
   }
 }
