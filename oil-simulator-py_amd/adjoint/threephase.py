@@ -298,7 +298,7 @@ def _faces(t):
 
 
 def _div(fx, fy, fz):
-    """Net outflow per cell of face fluxes (oracle div / k_flux)."""
+    """Net outflow per cell of face fluxes (oracle div / k_flux_rat)."""
     return (_px(fx, 0, 1) - _px(fx, 1, 0)) + (_py(fy, 0, 1) - _py(fy, 1, 0)) + (_pz(fz, 0, 1) - _pz(fz, 1, 0))
 
 

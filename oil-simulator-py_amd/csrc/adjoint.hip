@@ -364,7 +364,7 @@ __global__ void k_sat_vjp(GridDev G, FluidParams F, double dt, const double* __r
   }
 }
 
-// Phase fluxes (k_flux): for a face (lo, hi) with T = T[lo], dp = P1[lo] - P1[hi],
+// Phase fluxes (k_flux_rat): for a face (lo, hi) with T = T[lo], dp = P1[lo] - P1[hi],
 // u = dp > 0 ? lo : hi, pot = dp (+ g rho_mean dz on z faces),
 // fw = T mw[u] pot_w, fg = T mg[u] (pot_g - (pcog[hi] - pcog[lo])); div[lo] += f,
 // div[hi] -= f. Each cell gathers the cotangents of its own inputs over its six
@@ -484,7 +484,7 @@ struct WellOut {
   WD obs[3];      // surface oil, water, gas rates of producers (m3/day)
 };
 
-// One well of k_wells_sat on duals. `bal` is the row balance (the BHP rate form
+// One well of wells_sat on duals. `bal` is the row balance (the BHP rate form
 // used when row_form), mt_pres the pressure step's total mobility at the cell.
 __device__ WellOut well_sat_d(const FluidParams& F, const PvtDev& T, double dt, const WellDesc& d, double P_v,
                               double mw_v, double mo_v, double mg_v, double sw_v, double sg_v, double pvc, bool row_form,

@@ -42,6 +42,8 @@ struct Grid {
   double dx, dy, dz;
 };
 
+struct SatWellCtx;
+
 class Model {
  public:
   Model(const Grid& g, const FluidParams& f, int pvt_n, const double* pvt_host, const std::vector<WellDesc>& wells);
@@ -137,8 +139,21 @@ class Model {
   } stage_;
   DevBuf<double> well_sc_;  // per-well terms of the transport step (kWellScratch doubles per well)
   DevBuf<double> mob_w_, mob_o_, mob_g_, rho_w_, rho_o_, rho_g_, pc_;
-  DevBuf<double> pcog_, div_w_, div_g_, dsw_, dsg_, qw_, qg_, qo_;
+  DevBuf<double> pcog_, dsw_, dsg_, qw_, qg_, qo_;
   DevBuf<double> part_, report_;
+  // the report of a step in mapped host memory (k_step_end)
+  struct HostReport {
+    double* p = nullptr;
+    double* dev = nullptr;
+    size_t cap = 0;
+    HostReport() = default;
+    HostReport(const HostReport&) = delete;
+    HostReport& operator=(const HostReport&) = delete;
+    ~HostReport();
+    void reserve(size_t n);
+  } report_host_;
+  SatWellCtx sat_ctx(double dt, const double* p_prev, const double* p_new, const double* sw, const double* sg) const;
+  int transport_increments(const SatWellCtx& X, double* mo, double* rat, hipStream_t s);
   AmgParams amg_prm_;
   std::unique_ptr<Hierarchy> amg_;
   Fgmres fgmres_;

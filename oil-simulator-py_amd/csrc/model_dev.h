@@ -21,10 +21,11 @@ struct GridDev {
 #define CELL_LOOP(c, n) for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < (n); c += (long long)gridDim.x * blockDim.x)
 
 __device__ __forceinline__ void ijk(const GridDev& G, long long c, int& i, int& j, int& k) {
-  k = (int)(c % G.nz);
-  const long long t = c / G.nz;
-  j = (int)(t % G.ny);
-  i = (int)(t / G.ny);
+  // a grid has fewer than 2^30 cells (Model): 32-bit divisions
+  const unsigned u = (unsigned)c, t = u / (unsigned)G.nz;
+  k = (int)(u - t * (unsigned)G.nz);
+  i = (int)(t / (unsigned)G.ny);
+  j = (int)(t - (unsigned)i * (unsigned)G.ny);
 }
 
 inline GridDev grid_dev(const Grid& g, bool gravity, int env_nx) {
@@ -41,4 +42,28 @@ inline GridDev grid_dev(const Grid& g, bool gravity, int env_nx) {
 __device__ __forceinline__ double mx12(double a) { return fmax(a, 1e-12); }
 
 }  // namespace model_dev
+
+// State and operands of the transport step's wells.
+struct SatWellCtx {
+  model_dev::GridDev G;
+  FluidParams F;
+  PvtDev T;
+  double dt;
+  int nw;
+  const WellDesc* W;
+  const int* link;  // wells of one cell (well_lone)
+  int shared;       // some cell holds several wells
+  const double* p_prev;
+  const double* p;
+  const double* sw;
+  const double* sg;
+  const double* pv;
+  const double* mt_pres;
+  const double* ox;
+  const double* oy;
+  const double* oz;
+  const double* acc;
+  const double* extra;
+};
+
 }  // namespace impes
