@@ -206,11 +206,11 @@ __device__ __forceinline__ Dual<K> mx12d(const Dual<K>& a) {
 // PVT column at a located pressure; x = p / 1e6 as a dual
 template <int K>
 __device__ __forceinline__ Dual<K> pvt_d(const PvtDev& T, int key, const PvtAt& a, const Dual<K>& x) {
-  const double* fp = T.col + key * T.n;
-  if (a.side == 2) return x;
-  if (a.side == -1) return cst<K>(fp[0]);
-  if (a.side == 1) return cst<K>(fp[T.n - 1]);
-  return T.slope[key * (T.n - 1) + a.lo] * (x - T.P[a.lo]) + fp[a.lo];
+  const double slope = T.tab[a.row * kPvtKeys + key].x;
+  Dual<K> r;
+  r.v = pvt_at(T, key, a);
+  for (int q = 0; q < K; ++q) r.d[q] = slope * x.d[q];
+  return r;
 }
 
 // ---------------------------------------------------------------- physics on duals
@@ -287,15 +287,16 @@ __device__ Dual<K> ct_d(const FluidParams& F, const PvtDev& T, const Dual<K>& p,
   if (T.n == 0) return cst<K>(F.cf);
   const Dual<K> pm = p / 1e6;
   const Dual<K> p0 = pm * 1e6, pp = (pm + 0.1) * 1e6, pn = (pm - 0.1) * 1e6;
-  const PvtAt a0 = pvt_locate(T, p0.v);
-  const PvtAt ap = pvt_locate_near(T, pp.v, a0), am = pvt_locate_near(T, pn.v, a0);
+  const double at[3] = {p0.v, pp.v, pn.v};
+  PvtAt a[3];
+  pvt_locate(T, at, a);
   const Dual<K> x0 = p0 / 1e6, xp = pp / 1e6, xn = pn / 1e6;
   const int keys[3] = {kBw, kBo, kBg};
   Dual<K> c[3];
   for (int q = 0; q < 3; ++q) {
-    const Dual<K> b0 = pvt_d(T, keys[q], a0, x0);
-    const Dual<K> bp = pvt_d(T, keys[q], ap, xp);
-    const Dual<K> bm = pvt_d(T, keys[q], am, xn);
+    const Dual<K> b0 = pvt_d(T, keys[q], a[0], x0);
+    const Dual<K> bp = pvt_d(T, keys[q], a[1], xp);
+    const Dual<K> bm = pvt_d(T, keys[q], a[2], xn);
     const Dual<K> dB = (bp - bm) / (2 * 0.1);
     c[q] = -(dB / (b0 + 1e-12)) / 1e6;
   }

@@ -122,7 +122,8 @@ class Model {
   long long env_cells_ = 0;          // cells per stacked reservoir
   DevBuf<double> rat_, nsub_;        // per-cell substep demand, per-reservoir substep count
   bool gravity_ = false;
-  DevBuf<double> pvt_P_, pvt_col_, pvt_slope_;
+  DevBuf<double> pvt_P_;
+  DevBuf<double2> pvt_tab_;
   DevBuf<WellDesc> wells_;
   DevBuf<int> well_link_;  // chains of the wells that share a cell (2 per well)
   int wells_shared_ = 0;   // whether one does
@@ -138,7 +139,7 @@ class Model {
     ~Staging();
   } stage_;
   DevBuf<double> well_sc_;  // per-well terms of the transport step (kWellScratch doubles per well)
-  DevBuf<double> mob_w_, mob_o_, mob_g_, rho_w_, rho_o_, rho_g_, pc_;
+  DevBuf<double> mob_w_, mob_o_, mob_g_, rho_w_, rho_o_, rho_g_, grav_, pc_;
   DevBuf<double> pcog_, dsw_, dsg_, qw_, qg_, qo_;
   DevBuf<double> part_, report_;
   // the report of a step in mapped host memory (k_step_end)

@@ -69,89 +69,117 @@ __global__ void k_trans(GridDev G, const double* __restrict__ kx, const double* 
 
 // ---------------------------------------------------------------- pressure step
 // simulation.py:871-882 + fluid properties at the previous pressure
-__global__ void k_props_pressure(GridDev G, FluidParams F, PvtDev T, double dt, const double* __restrict__ p,
-                                 const double* __restrict__ sw, const double* __restrict__ sg,
-                                 const double* __restrict__ pv, double* __restrict__ mw, double* __restrict__ mo,
-                                 double* __restrict__ mg, double* __restrict__ mt, double* __restrict__ rw,
-                                 double* __restrict__ ro, double* __restrict__ rg, double* __restrict__ pc,
-                                 double* __restrict__ acc) {
+// acc and mt always; grav = mw rw + mo ro + mg rg and pc, mo are what the assembly
+// reads (with gravity, with capillarity); the phases' own mobilities and densities only
+// where they are asked for (the reverse sweep; nullptr otherwise). At 1M
+// cells 42 us; 61 us with all of them written and one table search after the other.
+struct PressureProps {
+  double *mt, *acc, *grav, *pc, *mo;
+  double *mw, *mg, *rw, *ro, *rg;
+};
+__global__ __launch_bounds__(kBlock) void k_props_pressure(GridDev G, FluidParams F, PvtDev T, double dt,
+                                                           const double* __restrict__ p,
+                                                           const double* __restrict__ sw,
+                                                           const double* __restrict__ sg,
+                                                           const double* __restrict__ pv, PressureProps Q) {
   const long long n = (long long)G.nx * G.ny * G.nz;
   CELL_LOOP(c, n) {
     const double pp = p[c], s_w = sw[c], s_g = sg[c];
     double kro, krw, krg, muo, muw, mug;
     relperms(F, s_w, s_g, kro, krw, krg);
-    PvtAt at{};
-    if (T.n > 0) at = pvt_locate(T, pp);
-    viscosities(F, T, pp, muo, muw, mug, &at);
+    PvtAt at[4] = {};
+    if (T.n > 0) {
+      double q[4], ct[3];
+      ct_pressures(pp, ct);
+      q[0] = pp;
+      for (int i = 0; i < 3; ++i) q[i + 1] = ct[i];
+      pvt_locate(T, q, at);
+    }
+    viscosities(F, T, pp, muo, muw, mug, at);
     const double a = krw / muw, o = kro / muo, g = krg / mug;
-    mw[c] = a;
-    mo[c] = o;
-    mg[c] = g;
-    mt[c] = a + o + g;
+    Q.mt[c] = a + o + g;
+    if (Q.mo) Q.mo[c] = o;
+    if (Q.mw) {
+      Q.mw[c] = a;
+      Q.mg[c] = g;
+    }
     if (G.gravity) {
       double r1, r2, r3;
-      densities(F, T, pp, r1, r2, r3, &at);
-      rw[c] = r1;
-      ro[c] = r2;
-      rg[c] = r3;
+      densities(F, T, pp, r1, r2, r3, at);
+      Q.grav[c] = a * r1 + o * r2 + g * r3;
+      if (Q.rw) {
+        Q.rw[c] = r1;
+        Q.ro[c] = r2;
+        Q.rg[c] = r3;
+      }
     }
-    if (F.pc_scale > 0.0) pc[c] = pc_ow(F, s_w);
-    acc[c] = pv[c] * total_compressibility(F, T, pp, s_w, s_g, &at) / dt;
+    if (F.pc_scale > 0.0) Q.pc[c] = pc_ow(F, s_w);
+    Q.acc[c] = pv[c] * total_compressibility(F, T, pp, s_w, s_g, at + 1) / dt;
   }
 }
 
 // _build_pressure_matrix_vectorized (:1546-1580) + _build_pressure_rhs (:1582-1620) in face form:
 // each cell visits its six faces (coefficients recomputed on both sides, no atomics).
-__global__ void k_assemble(GridDev G, FluidParams F, const double* __restrict__ p, const double* __restrict__ tx,
-                           const double* __restrict__ ty, const double* __restrict__ tz,
-                           const double* __restrict__ mw, const double* __restrict__ mo,
-                           const double* __restrict__ mg, const double* __restrict__ mt,
-                           const double* __restrict__ rw, const double* __restrict__ ro,
-                           const double* __restrict__ rg, const double* __restrict__ pc,
-                           const double* __restrict__ acc, double* __restrict__ diag, double* __restrict__ ox,
-                           double* __restrict__ oy, double* __restrict__ oz, double* __restrict__ b,
-                           double* __restrict__ extra, double* __restrict__ dinv) {
+// Every load is made whether its face exists or not (a missing neighbour reads the cell
+// itself), so that a wave waits for them once and not face after face; each XCD takes
+// one run of cells. At 1M cells 31 us; 52 us with a wait per face.
+__global__ __launch_bounds__(kBlock) void k_assemble(
+    GridDev G, FluidParams F, const double* __restrict__ p, const double* __restrict__ tx,
+    const double* __restrict__ ty, const double* __restrict__ tz, const double* __restrict__ mt,
+    const double* __restrict__ grav, const double* __restrict__ mo, const double* __restrict__ pc,
+    const double* __restrict__ acc, double* __restrict__ diag, double* __restrict__ ox, double* __restrict__ oy,
+    double* __restrict__ oz, double* __restrict__ b, double* __restrict__ extra, double* __restrict__ dinv) {
   const long long n = (long long)G.nx * G.ny * G.nz;
-  const bool with_pc = F.pc_scale > 0.0;
-  CELL_LOOP(c, n) {
+  const bool with_pc = F.pc_scale > 0.0, with_g = G.gravity != 0;
+  for (long long c = xcd_block() * kBlock + threadIdx.x; c < n; c += (long long)gridDim.x * kBlock) {
     int i, j, k;
     ijk(G, c, i, j, k);
-    const double pcc = p[c];
-    double d = 0.0, qg = 0.0, qpc = 0.0;
-    const double* T[3] = {tx, ty, tz};
+    const bool up[3] = {i < G.nx - 1, j < G.ny - 1, k < G.nz - 1}, dn[3] = {i > 0, j > 0, k > 0};
     const long long st[3] = {G.sx, G.sy, 1};
-    const int idx[3] = {i, j, k};
-    const int dim[3] = {G.nx, G.ny, G.nz};
+    const double* const T[3] = {tx, ty, tz};
+    // face f: axis f / 2, to the upper (even) or the lower (odd) neighbour
+    double pn[6], tn[6], mn[6], on[6], cn[6], gn[2] = {0.0, 0.0}, gc = 0.0;
+    const double pcc = p[c], mc = mt[c], a = acc[c];
+    const double oc = with_pc ? mo[c] : 0.0, cc = with_pc ? pc[c] : 0.0;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+      const int ax = f >> 1;
+      const long long o = f & 1 ? (dn[ax] ? c - st[ax] : c) : (up[ax] ? c + st[ax] : c);
+      pn[f] = p[o];
+      mn[f] = mt[o];
+      tn[f] = T[ax][f & 1 ? o : c];
+      on[f] = with_pc ? mo[o] : 0.0;
+      cn[f] = with_pc ? pc[o] : 0.0;
+    }
+    if (with_g) {
+      gc = grav[c];
+      gn[0] = grav[up[2] ? c + 1 : c];
+      gn[1] = grav[dn[2] ? c - 1 : c];
+    }
+    double d = 0.0, qg = 0.0, qpc = 0.0;
     double o_plus[3] = {0.0, 0.0, 0.0};
-    for (int ax = 0; ax < 3; ++ax) {
-      // face to the upper neighbour: this cell is the lower one
-      if (idx[ax] < dim[ax] - 1) {
-        const long long nb = c + st[ax];
-        const bool up_self = (pcc - p[nb]) > 0;
-        const long long u = up_self ? c : nb;
-        const double tl = T[ax][c] * mt[u];
-        o_plus[ax] = -tl;
-        d += tl;
-        if (ax == 2 && G.gravity)
-          qg -= T[2][c] * F.g * G.dz * (mw[u] * rw[u] + mo[u] * ro[u] + mg[u] * rg[u]);
-        if (with_pc) qpc -= T[ax][c] * mo[u] * (pc[nb] - pc[c]);
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+      const int ax = f >> 1;
+      const bool low = f & 1;
+      if (!(low ? dn[ax] : up[ax])) continue;
+      // the flow leaves this cell: over its upper face, or not in over its lower one
+      const bool self = low ? !((pn[f] - pcc) > 0) : (pcc - pn[f]) > 0;
+      const double tl = tn[f] * (self ? mc : mn[f]);
+      if (!low) o_plus[ax] = -tl;
+      d += tl;
+      if (ax == 2 && with_g) {
+        const double q = tn[f] * F.g * G.dz * (self ? gc : gn[f & 1]);
+        qg = low ? qg + q : qg - q;
       }
-      // face to the lower neighbour: this cell is the upper one
-      if (idx[ax] > 0) {
-        const long long nb = c - st[ax];
-        const bool up_nb = (p[nb] - pcc) > 0;
-        const long long u = up_nb ? nb : c;
-        const double tl = T[ax][nb] * mt[u];
-        d += tl;
-        if (ax == 2 && G.gravity)
-          qg += T[2][nb] * F.g * G.dz * (mw[u] * rw[u] + mo[u] * ro[u] + mg[u] * rg[u]);
-        if (with_pc) qpc += T[ax][nb] * mo[u] * (pc[c] - pc[nb]);
+      if (with_pc) {
+        const double q = tn[f] * (self ? oc : on[f]) * (low ? cc - cn[f] : cn[f] - cc);
+        qpc = low ? qpc + q : qpc - q;
       }
     }
     ox[c] = o_plus[0];
     oy[c] = o_plus[1];
     oz[c] = o_plus[2];
-    const double a = acc[c];
     const double dd = d + a;
     diag[c] = dd;
     dinv[c] = 1.0 / dd;
@@ -477,7 +505,8 @@ __device__ void wells_sat(const SatWellCtx& X, double* __restrict__ qw, double* 
 // simulation.py:973-1006: mobilities at the new pressure, densities, o-g capillarity,
 // and, in the first workgroup, the wells. mo: nullptr where nobody reads the oil
 // mobility (the reverse sweep does). A streaming pass: at 1M cells 24 MB read, 32 MB
-// (40 with mo) written, 34.5 us; as two launches 26 + 15 us and their gap.
+// (40 with mo) written, 22 us; as two launches 26 + 15 us and their gap (34.5 us as one
+// with a branch per table lookup).
 __global__ __launch_bounds__(kBlock) void k_props_wells(SatWellCtx X, double* __restrict__ mw,
                                                         double* __restrict__ mo, double* __restrict__ mg,
                                                         double* __restrict__ rw, double* __restrict__ rg,
@@ -565,7 +594,7 @@ inline int trans_blocks(long long n) {
 // One pass, so the divergences stay in registers; and every load is made whether its
 // face exists or not (a missing neighbour reads the cell itself), both sides of an
 // upwind choice included, so that a wave waits for them once and not face after face.
-// At 1M cells 27.3 us; 29.9 us (fluxes) + 16.0 us (increments) as two passes with a
+// At 1M cells 27 us; 29.9 us (fluxes) + 16.0 us (increments) as two passes with a
 // wait per face.
 __global__ __launch_bounds__(kBlock) void k_flux_rat(
     GridDev G, FluidParams F, double dt, int per, const double* __restrict__ p, const double* __restrict__ tx,
@@ -708,7 +737,7 @@ __device__ __forceinline__ void substep(const FluidParams& F, double dsw_sub, do
 // new pressure and the volume ledger sum PV dS vs dt sum q + clamp corrections. Every
 // workgroup first folds the demand's partials into the substep count by itself: about
 // 1 us, where a launch for it took 4.5 us and its gap. At 1M cells (48 MB read, 24 MB
-// written) 36.5 us; 49 us with 512 workgroups, two per CU, and ten block sums at the
+// written) 33 us; 49 us with 512 workgroups, two per CU, and ten block sums at the
 // end.
 __global__ __launch_bounds__(kBlock) void k_substeps(
     GridDev G, FluidParams F, PvtDev T, int per, double* __restrict__ rep, int n_rat,
@@ -727,6 +756,7 @@ __global__ __launch_bounds__(kBlock) void k_substeps(
     rep[kNSub] = Nd;
   }
   const int N_all = (int)Nd;
+  const double r_all = 1.0 / N_all;
   double acc[kFoldQ];
 #pragma unroll
   for (int q = 0; q < kFoldQ; ++q) acc[q] = 0.0;
@@ -735,7 +765,8 @@ __global__ __launch_bounds__(kBlock) void k_substeps(
     if (c >= n) break;
     const int N = nsub ? (int)nsub[c / env_cells] : N_all;  // this cell's reservoir
     const double w0 = sw[c], g0 = sg[c];
-    const double a = dsw[c] / N, b = dsg[c] / N;
+    const double rN = nsub ? 1.0 / N : r_all;
+    const double a = div_by(dsw[c], N, rN), b = div_by(dsg[c], N, rN);
     double w = w0, g = g0, cw = 0.0, cg = 0.0;
     const double v = pv[c];
     for (int s = 0; s < N; ++s) {
@@ -853,7 +884,7 @@ __device__ void substep_ledger(const SatWellCtx& X, const double* __restrict__ d
 // component ledger over the wells' substeps, zeroes the wells' sources and hands the
 // report out. Report and ledgers are written to `host` (mapped host memory) as well:
 // the caller waits for the stream and reads them there, with no copy to queue (at 1M
-// cells and 9 wells 10.8 us in all; the three launches it replaces took 22 us, the copy
+// cells and 9 wells 9 us in all; the three launches it replaces took 22 us, the copy
 // on top).
 __global__ __launch_bounds__(kBlock) void k_step_end(SatWellCtx X, int nb, const double* __restrict__ part,
                                                      const double* __restrict__ dsw, const double* __restrict__ dsg,
@@ -917,25 +948,25 @@ Model::Model(const Grid& g, const FluidParams& f, int pvt_n, const double* pvt_h
     IMPES_REQUIRE(pvt_n >= 2 && pvt_host, "model: PVT table needs >= 2 rows");
     std::vector<double> P(pvt_host, pvt_host + pvt_n), cols(pvt_host + pvt_n, pvt_host + 9 * pvt_n);
     for (int i = 0; i + 1 < pvt_n; ++i) IMPES_REQUIRE(P[i + 1] > P[i], "model: PVT pressures must increase");
-    std::vector<double> slope(8 * (pvt_n - 1));
-    for (int k = 0; k < 8; ++k)
-      for (int i = 0; i + 1 < pvt_n; ++i)
-        slope[k * (pvt_n - 1) + i] = (cols[k * pvt_n + i + 1] - cols[k * pvt_n + i]) / (P[i + 1] - P[i]);
+    std::vector<double2> tab(8 * (size_t)(pvt_n + 1));
+    for (int k = 0; k < 8; ++k) {
+      const double* col = cols.data() + k * pvt_n;
+      for (int i = 0; i + 1 < pvt_n; ++i) tab[8 * i + k] = double2{(col[i + 1] - col[i]) / (P[i + 1] - P[i]), col[i]};
+      tab[8 * (pvt_n - 1) + k] = double2{0.0, col[pvt_n - 1]};
+      tab[8 * pvt_n + k] = double2{0.0, col[0]};
+    }
     pvt_P_.alloc(pvt_n);
-    pvt_col_.alloc(8 * pvt_n);
-    pvt_slope_.alloc(8 * (pvt_n - 1));
+    pvt_tab_.alloc(tab.size());
     IMPES_HIP_CHECK(hipMemcpy(pvt_P_.p, P.data(), sizeof(double) * pvt_n, hipMemcpyHostToDevice));
-    IMPES_HIP_CHECK(hipMemcpy(pvt_col_.p, cols.data(), sizeof(double) * 8 * pvt_n, hipMemcpyHostToDevice));
-    IMPES_HIP_CHECK(hipMemcpy(pvt_slope_.p, slope.data(), sizeof(double) * slope.size(), hipMemcpyHostToDevice));
+    IMPES_HIP_CHECK(hipMemcpy(pvt_tab_.p, tab.data(), sizeof(double2) * tab.size(), hipMemcpyHostToDevice));
     pvt.n = pvt_n;
     pvt.P = pvt_P_.p;
-    pvt.col = pvt_col_.p;
-    pvt.slope = pvt_slope_.p;
+    pvt.tab = pvt_tab_.p;
   }
   const long long n = N_;
   for (auto* b : {&tx, &ty, &tz, &pv, &diag, &ox, &oy, &oz, &this->b, &dinv, &acc, &extra, &mob_t}) b->alloc(n);
   for (auto* b : {&mob_w_, &mob_o_, &mob_g_, &dsw_, &dsg_, &qw_, &qg_, &qo_}) b->alloc(n);
-  if (gravity_) for (auto* b : {&rho_w_, &rho_o_, &rho_g_}) b->alloc(n);
+  if (gravity_) for (auto* b : {&rho_w_, &rho_o_, &rho_g_, &grav_}) b->alloc(n);
   if (F.pc_scale > 0.0) pc_.alloc(n);
   if (F.pcog_scale > 0.0) pcog_.alloc(n);
   IMPES_HIP_CHECK(hipMemset(qw_.p, 0, n * sizeof(double)));
@@ -1049,11 +1080,13 @@ void Model::assemble(double dt, const double* p, const double* sw, const double*
   dt_ = dt;
   GridDev G = grid_dev(grid, gravity_, env_nx_);
   const int gr = grid_for(N_, kBlock, 1 << 16);
-  k_props_pressure<<<gr, kBlock, 0, s>>>(G, F, pvt, dt, p, sw, sg, pv.p, mob_w_.p, mob_o_.p, mob_g_.p, mob_t.p,
-                                         rho_w_.p, rho_o_.p, rho_g_.p, pc_.p, acc.p);
+  // the mobility of the oil is read for the capillary fluxes alone
+  const PressureProps Q{mob_t.p, acc.p, grav_.p, pc_.p, F.pc_scale > 0.0 ? mob_o_.p : nullptr,
+                        nullptr, nullptr, nullptr, nullptr, nullptr};
+  k_props_pressure<<<gr, kBlock, 0, s>>>(G, F, pvt, dt, p, sw, sg, pv.p, Q);
   IMPES_LAUNCH_CHECK();
-  k_assemble<<<gr, kBlock, 0, s>>>(G, F, p, tx.p, ty.p, tz.p, mob_w_.p, mob_o_.p, mob_g_.p, mob_t.p, rho_w_.p,
-                                   rho_o_.p, rho_g_.p, pc_.p, acc.p, diag.p, ox.p, oy.p, oz.p, b.p, extra.p, dinv.p);
+  k_assemble<<<gr, kBlock, 0, s>>>(G, F, p, tx.p, ty.p, tz.p, mob_t.p, grav_.p, mob_o_.p, pc_.p, acc.p, diag.p, ox.p,
+                                   oy.p, oz.p, b.p, extra.p, dinv.p);
   IMPES_LAUNCH_CHECK();
   if (nw_ > 0) {
     k_wells_pressure<<<1, 256, 0, s>>>(F, nw_, wells_.p, p, mob_t.p, diag.p, b.p, dinv.p, report_.p, well_sc_.p,
@@ -1164,9 +1197,8 @@ void Model::transport_forward(double dt, const double* p_prev, const double* p_n
 
 void Model::pressure_props(double dt, const double* p, const double* sw, const double* sg, hipStream_t s) {
   GridDev G = grid_dev(grid, gravity_, env_nx_);
-  k_props_pressure<<<grid_for(N_, kBlock, 1 << 16), kBlock, 0, s>>>(G, F, pvt, dt, p, sw, sg, pv.p, mob_w_.p,
-                                                                    mob_o_.p, mob_g_.p, mob_t.p, rho_w_.p, rho_o_.p,
-                                                                    rho_g_.p, pc_.p, acc.p);
+  const PressureProps Q{mob_t.p, acc.p, grav_.p, pc_.p, mob_o_.p, mob_w_.p, mob_g_.p, rho_w_.p, rho_o_.p, rho_g_.p};
+  k_props_pressure<<<grid_for(N_, kBlock, 1 << 16), kBlock, 0, s>>>(G, F, pvt, dt, p, sw, sg, pv.p, Q);
   IMPES_LAUNCH_CHECK();
 }
 

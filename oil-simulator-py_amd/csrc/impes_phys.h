@@ -23,12 +23,14 @@ struct FluidParams {
   double rate_scale;                  // global_rate_scale
 };
 
-// PVT table (pvt.py): pressure in MPa, 8 columns, slopes precomputed on the host.
+// PVT table (pvt.py): pressure in MPa, 8 columns. Row r < n of tab holds, for every
+// column, the slope of the segment above node r and the value at the node (row n - 1:
+// slope 0), row n slope 0 and the value at node 0: one 128-byte line for all the
+// columns of a pressure, and no case split for pressures outside the table.
 struct PvtDev {
   int n = 0;
   const double* P = nullptr;
-  const double* col = nullptr;    // 8 x n
-  const double* slope = nullptr;  // 8 x (n-1)
+  const double2* tab = nullptr;  // (n + 1) x 8, {slope, value}
 };
 
 // One well (well.py:10-55 + the branch flags of simulation.py:1051-1347,1622-1660).
@@ -47,73 +49,69 @@ struct WellDesc {
   double lim[4];           // m3/day
 };
 
+// x / d, correctly rounded, from r = 1/d (rounded): Markstein's quotient correction
+// (P. W. Markstein, IBM J. Res. Dev. 34, 1990). 3 operations where the general division
+// takes about 10; x = +-inf keeps its quotient.
+__device__ __forceinline__ double div_by(double x, double d, double r) {
+  const double q = x * r;
+  const double e = fma(-q, d, x);
+  return e == e ? fma(e, r, q) : q;
+}
+__device__ __forceinline__ double mega(double p_pa) { return div_by(p_pa, 1e6, 1.0 / 1e6); }
+
 // np.interp(p/1e6, P, col, left=col[0], right=col[-1]); products and sums are
-// rounded separately, as numpy does. The table segment depends only on the
-// pressure, so it is located once (pvt_locate) and read for every column that
-// pressure needs (pvt_at): one binary search per pressure instead of one per
-// property.
+// rounded separately, as numpy does. The table row depends only on the pressure, so it
+// is located once (pvt_locate) and read for every column that pressure needs
+// (pvt_at): one search per pressure instead of one per property.
 struct PvtAt {
-  double x;  // p / 1e6
-  int lo;    // segment (inside the table)
-  int side;  // 0 inside, -1 below the first node, 1 at or above the last, 2 NaN
+  double dx;  // p / 1e6 less its node (0 outside the table, NaN for a NaN)
+  int row;    // of PvtDev::tab
 };
 
-__device__ __forceinline__ PvtAt pvt_locate(const PvtDev& T, double p_pa) {
-  PvtAt a;
-  a.x = p_pa / 1e6;
-  a.lo = 0;
-  const double* xp = T.P;
+// K pressures at once: each step of the searches is one load and no branch (the number
+// of steps depends on the table alone), and the K chains of dependent loads overlap.
+template <int K>
+__device__ __forceinline__ void pvt_locate(const PvtDev& T, const double (&p_pa)[K], PvtAt (&a)[K]) {
+  const double* __restrict__ xp = T.P;
   const int n = T.n;
-  if (!(a.x >= xp[0])) {
-    a.side = (a.x != a.x) ? 2 : -1;
-    return a;
+  const double first = xp[0], last = xp[n - 1];
+  double x[K], node[K];
+  int lo[K];
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    x[q] = mega(p_pa[q]);
+    lo[q] = 0;
+    node[q] = first;
   }
-  if (a.x >= xp[n - 1]) {
-    a.side = 1;
-    return a;
+  for (int len = n - 1; len > 1;) {
+    const int half = len >> 1;
+#pragma unroll
+    for (int q = 0; q < K; ++q) {
+      const double v = xp[lo[q] + half];
+      const bool up = v <= x[q];
+      lo[q] = up ? lo[q] + half : lo[q];
+      node[q] = up ? v : node[q];
+    }
+    len -= half;
   }
-  int lo = 0, hi = n - 1;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (xp[mid] <= a.x) lo = mid; else hi = mid;
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    const bool below = x[q] < first, above = x[q] >= last;
+    a[q].row = below ? n : above ? n - 1 : lo[q];
+    a[q].dx = below || above ? 0.0 : x[q] - node[q];
   }
-  a.lo = lo;
-  a.side = 0;
-  return a;
 }
-
-// The same location found by walking from a nearby located pressure (a few table
-// nodes away): the segment with xp[lo] <= x < xp[lo + 1] is unique in the
-// increasing node list, so the walk ends where the binary search does.
-__device__ __forceinline__ PvtAt pvt_locate_near(const PvtDev& T, double p_pa, const PvtAt& near) {
-  if (near.side != 0) return pvt_locate(T, p_pa);
-  PvtAt a;
-  a.x = p_pa / 1e6;
-  a.lo = 0;
-  const double* xp = T.P;
-  const int n = T.n;
-  if (!(a.x >= xp[0])) {
-    a.side = (a.x != a.x) ? 2 : -1;
-    return a;
-  }
-  if (a.x >= xp[n - 1]) {
-    a.side = 1;
-    return a;
-  }
-  int lo = near.lo;
-  while (lo > 0 && xp[lo] > a.x) --lo;
-  while (lo < n - 2 && xp[lo + 1] <= a.x) ++lo;
-  a.lo = lo;
-  a.side = 0;
-  return a;
+__device__ __forceinline__ PvtAt pvt_locate(const PvtDev& T, double p_pa) {
+  const double p[1] = {p_pa};
+  PvtAt a[1];
+  pvt_locate(T, p, a);
+  return a[0];
 }
 
 __device__ __forceinline__ double pvt_at(const PvtDev& T, int key, const PvtAt& a) {
-  const double* fp = T.col + key * T.n;
-  if (a.side == 2) return a.x;
-  if (a.side == -1) return fp[0];
-  if (a.side == 1) return fp[T.n - 1];
-  return __dadd_rn(__dmul_rn(T.slope[key * (T.n - 1) + a.lo], __dsub_rn(a.x, T.P[a.lo])), fp[a.lo]);
+#pragma clang fp contract(off)
+  const double2 e = T.tab[a.row * kPvtKeys + key];
+  return e.x * a.dx + e.y;
 }
 
 __device__ __forceinline__ double pvt_eval(const PvtDev& T, int key, double p_pa) {
@@ -182,23 +180,36 @@ __device__ __forceinline__ void viscosities(const FluidParams& F, const PvtDev& 
   }
 }
 
-// fluid.py:190-222 (central difference of B over +-0.1 MPa); fluid.py:47-48 without PVT
-// `at`: the located pressure p when the caller has it
+// The pressures whose formation volume factors the compressibility takes: its own and
+// the two +-0.1 MPa away (fluid.py:190-222).
+__device__ __forceinline__ void ct_pressures(double p, double (&q)[3]) {
+  const double pm = mega(p);
+  q[0] = pm * 1e6;
+  q[1] = (pm + 0.1) * 1e6;
+  q[2] = (pm - 0.1) * 1e6;
+}
+
+// fluid.py:190-222 (central difference of B over +-0.1 MPa); fluid.py:47-48 without PVT.
+// `at`: the located ct_pressures when the caller has them
 __device__ __forceinline__ double total_compressibility(const FluidParams& F, const PvtDev& T, double p, double sw,
                                                         double sg, const PvtAt* at = nullptr) {
   if (T.n == 0) return F.cf;
-  const double pm = p / 1e6;
+  PvtAt a[3];
+  if (at) {
+    for (int q = 0; q < 3; ++q) a[q] = at[q];
+  } else {
+    double pq[3];
+    ct_pressures(p, pq);
+    pvt_locate(T, pq, a);
+  }
   double c[3];
   const int keys[3] = {kBw, kBo, kBg};
-  const double p0 = pm * 1e6;
-  const PvtAt a0 = (at && p0 == p) ? *at : pvt_locate(T, p0);
-  const PvtAt ap = pvt_locate_near(T, (pm + 0.1) * 1e6, a0), am = pvt_locate_near(T, (pm - 0.1) * 1e6, a0);
   for (int q = 0; q < 3; ++q) {
-    const double b0 = pvt_at(T, keys[q], a0);
-    const double bp = pvt_at(T, keys[q], ap);
-    const double bm = pvt_at(T, keys[q], am);
-    const double dB = (bp - bm) / (2 * 0.1);
-    c[q] = -(dB / (b0 + 1e-12)) / 1e6;
+    const double b0 = pvt_at(T, keys[q], a[0]);
+    const double bp = pvt_at(T, keys[q], a[1]);
+    const double bm = pvt_at(T, keys[q], a[2]);
+    const double dB = div_by(bp - bm, 2 * 0.1, 1.0 / (2 * 0.1));
+    c[q] = mega(-(dB / (b0 + 1e-12)));
   }
   const double so = 1.0 - sw - sg;
   return F.c_r + sw * c[0] + so * c[1] + sg * c[2];
