@@ -102,7 +102,6 @@ struct Level {
   Pad4 r4;  // FP32 restriction in the padded tiled form (read instead of rv32 when set)
   // Galerkin product data: AP = A*P (values refreshed on update), next A = R*AP
   int apnnz = 0;
-  int ap_group = 1, ac_group = 1;  // lanes per output entry of the numeric products
   DevBuf<int> aprp, apci;
   DevBuf<double> apv;
   DevBuf<long long> ap_seg, ac_seg;
