@@ -28,13 +28,6 @@ void d2d(T* dst, const T* src, size_t n, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------- stencil kernels
-__device__ __forceinline__ void cell_ijk(long long c, int ny, int nz, int& i, int& j, int& k) {
-  k = (int)(c % nz);
-  const long long t = c / nz;
-  j = (int)(t % ny);
-  i = (int)(t / ny);
-}
-
 __global__ void k_st7_count(int nx, int ny, int nz, int* __restrict__ cnt) {
   const long long n = (long long)nx * ny * nz;
   for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < n; c += (long long)gridDim.x * blockDim.x) {

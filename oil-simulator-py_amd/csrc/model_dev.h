@@ -21,11 +21,7 @@ struct GridDev {
 #define CELL_LOOP(c, n) for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < (n); c += (long long)gridDim.x * blockDim.x)
 
 __device__ __forceinline__ void ijk(const GridDev& G, long long c, int& i, int& j, int& k) {
-  // a grid has fewer than 2^30 cells (Model): 32-bit divisions
-  const unsigned u = (unsigned)c, t = u / (unsigned)G.nz;
-  k = (int)(u - t * (unsigned)G.nz);
-  i = (int)(t / (unsigned)G.ny);
-  j = (int)(t - (unsigned)i * (unsigned)G.ny);
+  cell_ijk(c, G.ny, G.nz, i, j, k);
 }
 
 inline GridDev grid_dev(const Grid& g, bool gravity, int env_nx) {

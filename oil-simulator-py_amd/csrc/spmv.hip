@@ -386,61 +386,54 @@ void csr_dispatch(int n, const int* rp, const int* ci, const T* v, const T* x, c
 }
 
 // ---------------------------------------------------------------- stencil 7
-template <class T>
-struct St7Row {
-  // sum_j A[c,j] x[j] in the column order of the CSR form (c-sx, c-nz, c-1, c, c+1, c+nz, c+sx)
-  __device__ __forceinline__ static T apply(const Stencil7<T>& S, const T* __restrict__ x, long long c, int i, int j,
-                                            int k) {
-    const long long sy = S.nz;
-    const long long sx = (long long)S.ny * S.nz;
-    T s = T(0);
-    if (i > 0) s += S.ox[c - sx] * x[c - sx];
-    if (j > 0) s += S.oy[c - sy] * x[c - sy];
-    if (k > 0) s += S.oz[c - 1] * x[c - 1];
-    s += S.d[c] * x[c];
-    if (k < S.nz - 1) s += S.oz[c] * x[c + 1];
-    if (j < S.ny - 1) s += S.oy[c] * x[c + sy];
-    if (i < S.nx - 1) s += S.ox[c] * x[c + sx];
-    return s;
-  }
-  // the same sum with x[q] given by xv(q)
-  template <class F>
-  __device__ __forceinline__ static T apply_f(const Stencil7<T>& S, F xv, long long c, int i, int j, int k) {
-    const long long sy = S.nz;
-    const long long sx = (long long)S.ny * S.nz;
-    T s = T(0);
-    if (i > 0) s += S.ox[c - sx] * xv(c - sx);
-    if (j > 0) s += S.oy[c - sy] * xv(c - sy);
-    if (k > 0) s += S.oz[c - 1] * xv(c - 1);
-    s += S.d[c] * xv(c);
-    if (k < S.nz - 1) s += S.oz[c] * xv(c + 1);
-    if (j < S.ny - 1) s += S.oy[c] * xv(c + sy);
-    if (i < S.nx - 1) s += S.ox[c] * xv(c + sx);
-    return s;
-  }
-};
+// sum_j A[c,j] x[j] in the column order of the CSR form (c-sx, c-nz, c-1, c, c+1, c+nz,
+// c+sx), x[q] given by xv(q). A missing neighbour is read as the cell itself and left
+// out of the sum: with the loads under the boundary conditions instead, a wave waited
+// for memory once per neighbour (FP32 sweeps of 76,800 rows 3.5 us, now 2.5; the FP64 operator apply 4.8 and 3.8).
+template <class T, class F>
+__device__ __forceinline__ T st7_row(const Stencil7<T>& S, F xv, long long c, int i, int j, int k) {
+  const long long sy = S.nz;
+  const long long sx = (long long)S.ny * S.nz;
+  const bool w = i > 0, e = i < S.nx - 1, o = j > 0, n = j < S.ny - 1, b = k > 0, t = k < S.nz - 1;
+  const long long qw = w ? c - sx : c, qo = o ? c - sy : c, qb = b ? c - 1 : c;
+  const T fw = S.ox[qw], fo = S.oy[qo], fb = S.oz[qb], d = S.d[c], ft = S.oz[c], fn = S.oy[c], fe = S.ox[c];
+  const T xw = xv(qw), xo = xv(qo), xb = xv(qb), xc = xv(c);
+  const T xt = xv(t ? c + 1 : c), xn = xv(n ? c + sy : c), xe = xv(e ? c + sx : c);
+  T s = T(0);
+  s = w ? s + fw * xw : s;
+  s = o ? s + fo * xo : s;
+  s = b ? s + fb * xb : s;
+  s += d * xc;
+  s = t ? s + ft * xt : s;
+  s = n ? s + fn * xn : s;
+  s = e ? s + fe * xe : s;
+  return s;
+}
 
 template <class T, class TA, int MODE>
 __global__ __launch_bounds__(kBlock) void k_st7(Stencil7<T> S, const T* __restrict__ x, const T* __restrict__ b,
                                                 const TA* __restrict__ aux, T w, T* __restrict__ y) {
   const long long n = (long long)S.nx * S.ny * S.nz;
   for (long long c = xcd_block() * blockDim.x + threadIdx.x; c < n; c += (long long)gridDim.x * blockDim.x) {
-    const int k = (int)(c % S.nz);
-    const long long t = c / S.nz;
-    const int j = (int)(t % S.ny);
-    const int i = (int)(t / S.ny);
+    int i, j, k;
+    cell_ijk(c, S.ny, S.nz, i, j, k);
     if constexpr (MODE == kJacZ0) {
       auto xv = [&](long long q) { return w * (T)aux[q] * b[q]; };
-      const T sum = St7Row<T>::apply_f(S, xv, c, i, j, k);
-      y[c] = xv(c) + w * (T)aux[c] * (b[c] - sum);
+      const T bc = b[c], ac = (T)aux[c];
+      const T sum = st7_row(S, xv, c, i, j, k);
+      y[c] = xv(c) + w * ac * (bc - sum);
       continue;
     }
-    const T sum = St7Row<T>::apply(S, x, c, i, j, k);
+    // the row's own operands are loaded with the row's
+    constexpr bool uses_b = MODE == kRes || MODE == kJac || MODE == kRowScaledRes;
+    constexpr bool uses_aux = MODE == kJac || MODE == kRowScaled || MODE == kRowScaledRes;
+    const T bc = uses_b ? b[c] : T(0), ac = uses_aux ? (T)aux[c] : T(0);
+    const T sum = st7_row(S, [&](long long q) { return x[q]; }, c, i, j, k);
     if (MODE == kY) y[c] = sum;
-    else if (MODE == kRes) y[c] = b[c] - sum;
-    else if (MODE == kJac) y[c] = x[c] + w * (T)aux[c] * (b[c] - sum);
-    else if (MODE == kRowScaled) y[c] = (T)aux[c] * sum;
-    else if (MODE == kRowScaledRes) y[c] = (T)aux[c] * (b[c] - sum);
+    else if (MODE == kRes) y[c] = bc - sum;
+    else if (MODE == kJac) y[c] = x[c] + w * ac * (bc - sum);
+    else if (MODE == kRowScaled) y[c] = ac * sum;
+    else if (MODE == kRowScaledRes) y[c] = ac * (bc - sum);
   }
 }
 
@@ -448,7 +441,7 @@ __global__ __launch_bounds__(kBlock) void k_st7(Stencil7<T> S, const T* __restri
 // consecutive cells of one z-column (same i, j) and reads every coefficient and
 // x array with 16-byte loads (the +-x and +-y neighbours of V aligned cells are
 // V aligned cells), plus oz[c-1], x[c-1] and x[c+V] for the column ends. Each
-// cell's sum is formed in St7Row's order, so the results equal k_st7's.
+// cell's sum is formed in st7_row's order, so the results equal k_st7's.
 template <class T>
 struct Wide;
 template <>
@@ -478,10 +471,8 @@ __global__ __launch_bounds__(kBlock) void k_st7_wide(Stencil7<T> S, const T* __r
   const long long sx = (long long)S.ny * S.nz;
   for (long long q = xcd_block() * blockDim.x + threadIdx.x; q * V < n; q += (long long)gridDim.x * blockDim.x) {
     const long long c = q * V;
-    const int k0 = (int)(c % S.nz);
-    const long long t = c / S.nz;
-    const int j = (int)(t % S.ny);
-    const int i = (int)(t / S.ny);
+    int i, j, k0;
+    cell_ijk(c, S.ny, S.nz, i, j, k0);
     T xc[V], dd[V], fz[V], fy[V], fx[V];
     T fw[V] = {}, xw[V] = {}, fs[V] = {}, xs[V] = {}, xn[V] = {}, xe[V] = {}, bb[V] = {}, aa[V] = {};
     // x at V aligned cells: read, or (kJacZ0) the first sweep w * aux .* b formed in place
@@ -505,13 +496,17 @@ __global__ __launch_bounds__(kBlock) void k_st7_wide(Stencil7<T> S, const T* __r
     ld_wide(S.oz + c, fz);
     ld_wide(S.oy + c, fy);
     ld_wide(S.ox + c, fx);
-    if (i > 0) { ld_wide(S.ox + c - sx, fw); xg(c - sx, xw); }
-    if (j > 0) { ld_wide(S.oy + c - sy, fs); xg(c - sy, xs); }
-    if (j < S.ny - 1) xg(c + sy, xn);
-    if (i < S.nx - 1) xg(c + sx, xe);
-    const T zb = k0 > 0 ? S.oz[c - 1] : T(0);
-    const T xb = k0 > 0 ? x1(c - 1) : T(0);
-    const T xa = k0 + V < S.nz ? x1(c + V) : T(0);
+    // a missing neighbour is read as the cells themselves and left out of the sum
+    const long long qw = i > 0 ? c - sx : c, qs = j > 0 ? c - sy : c, qb = k0 > 0 ? c - 1 : c;
+    ld_wide(S.ox + qw, fw);
+    xg(qw, xw);
+    ld_wide(S.oy + qs, fs);
+    xg(qs, xs);
+    xg(j < S.ny - 1 ? c + sy : c, xn);
+    xg(i < S.nx - 1 ? c + sx : c, xe);
+    const T zb = S.oz[qb];
+    const T xb = x1(qb);
+    const T xa = x1(k0 + V < S.nz ? c + V : c);
     if (MODE == kRes || MODE == kJac || MODE == kRowScaledRes || MODE == kJacZ0) ld_wide(b + c, bb);
     if (MODE == kJac || MODE == kRowScaled || MODE == kRowScaledRes || MODE == kJacZ0) ld_wide(aux + c, aa);
     T out[V];
@@ -549,22 +544,13 @@ __global__ __launch_bounds__(kBlock) void k_st7_rowscaled_z(Stencil7<double> S, 
   const long long sy = S.nz;
   const long long sx = (long long)S.ny * S.nz;
   for (long long c = xcd_block() * blockDim.x + threadIdx.x; c < n; c += (long long)gridDim.x * blockDim.x) {
-    const int k = (int)(c % S.nz);
-    const long long t = c / S.nz;
-    const int j = (int)(t % S.ny);
-    const int i = (int)(t / S.ny);
+    int i, j, k;
+    cell_ijk(c, S.ny, S.nz, i, j, k);
     auto zv = [&](long long q) { return sout[q] * (double)x[q]; };
-    const double zc = zv(c);
-    double s = 0.0;
-    if (i > 0) s += S.ox[c - sx] * zv(c - sx);
-    if (j > 0) s += S.oy[c - sy] * zv(c - sy);
-    if (k > 0) s += S.oz[c - 1] * zv(c - 1);
-    s += S.d[c] * zc;
-    if (k < S.nz - 1) s += S.oz[c] * zv(c + 1);
-    if (j < S.ny - 1) s += S.oy[c] * zv(c + sy);
-    if (i < S.nx - 1) s += S.ox[c] * zv(c + sx);
-    z[c] = zc;
-    y[c] = dinv[c] * s;
+    const double di = dinv[c];
+    const double s = st7_row(S, zv, c, i, j, k);
+    z[c] = zv(c);
+    y[c] = di * s;
   }
 }
 
@@ -595,10 +581,8 @@ __global__ __launch_bounds__(kBlock) void k_st7_rowscaled_z_wide(Stencil7<double
   const long long sx = (long long)S.ny * S.nz;
   for (long long q = xcd_block() * blockDim.x + threadIdx.x; q * 2 < n; q += (long long)gridDim.x * blockDim.x) {
     const long long c = q * 2;
-    const int k0 = (int)(c % S.nz);
-    const long long t = c / S.nz;
-    const int j = (int)(t % S.ny);
-    const int i = (int)(t / S.ny);
+    int i, j, k0;
+    cell_ijk(c, S.ny, S.nz, i, j, k0);
     // z = sout .* x at the cell pair and at each neighbour pair
     auto zpair = [&](long long p0, double (&zz)[2]) {
       TX xx[2];
@@ -616,13 +600,18 @@ __global__ __launch_bounds__(kBlock) void k_st7_rowscaled_z_wide(Stencil7<double
     ld_pair(S.oy + c, fy);
     ld_pair(S.ox + c, fx);
     ld_pair(dinv + c, di);
-    if (i > 0) { ld_pair(S.ox + c - sx, fw); zpair(c - sx, zw); }
-    if (j > 0) { ld_pair(S.oy + c - sy, fs); zpair(c - sy, zs); }
-    if (j < S.ny - 1) zpair(c + sy, zn);
-    if (i < S.nx - 1) zpair(c + sx, ze);
-    const double fb = k0 > 0 ? S.oz[c - 1] : 0.0;
-    const double zb = k0 > 0 ? sout[c - 1] * (double)x[c - 1] : 0.0;
-    const double za = k0 + 2 < S.nz ? sout[c + 2] * (double)x[c + 2] : 0.0;
+    // a missing neighbour is read as the cells themselves and left out of the sum
+    const long long qw = i > 0 ? c - sx : c, qs = j > 0 ? c - sy : c, qb = k0 > 0 ? c - 1 : c;
+    const long long qa = k0 + 2 < S.nz ? c + 2 : c;
+    ld_pair(S.ox + qw, fw);
+    zpair(qw, zw);
+    ld_pair(S.oy + qs, fs);
+    zpair(qs, zs);
+    zpair(j < S.ny - 1 ? c + sy : c, zn);
+    zpair(i < S.nx - 1 ? c + sx : c, ze);
+    const double fb = S.oz[qb];
+    const double zb = sout[qb] * (double)x[qb];
+    const double za = sout[qa] * (double)x[qa];
     double out[2];
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
