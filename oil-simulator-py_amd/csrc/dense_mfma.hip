@@ -42,13 +42,16 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 // 16w..16w+15 as four 16 x 16 output tiles t (columns 16t..16t+15).
 // v_mfma_f64_16x16x4_f64 lane layout (measured on gfx950): A[i][k] at lane i + 16k,
 // B[k][j] at lane j + 16k, D[i][j] at lane j + 16 (i % 4), element i / 4.
-__device__ __forceinline__ void tile_mma(const double* __restrict__ As, const double* __restrict__ Bs, v4d (&acc)[4]) {
+// kDepth: how many of the 64 inner indices count (the rest add zeros)
+template <int kDepth>
+__device__ __forceinline__ void tile_mma_depth(const double* __restrict__ As, const double* __restrict__ Bs,
+                                               v4d (&acc)[4]) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i = lane & 15, kk = lane >> 4;
 #pragma unroll
   for (int t = 0; t < 4; ++t) acc[t] = v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll 4
-  for (int k0 = 0; k0 < kB; k0 += 4) {
+  for (int k0 = 0; k0 < kDepth; k0 += 4) {
     const double a = As[(16 * w + i) * kLdA + k0 + kk];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -56,6 +59,14 @@ __device__ __forceinline__ void tile_mma(const double* __restrict__ As, const do
       acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[t], 0, 0, 0);
     }
   }
+}
+
+// rows: the inner indices that belong to the matrix
+__device__ __forceinline__ void tile_mma(const double* __restrict__ As, const double* __restrict__ Bs, int rows,
+                                         v4d (&acc)[4]) {
+  if (rows <= kB / 4) tile_mma_depth<kB / 4>(As, Bs, acc);
+  else if (rows <= kB / 2) tile_mma_depth<kB / 2>(As, Bs, acc);
+  else tile_mma_depth<kB>(As, Bs, acc);
 }
 
 // (row, column) within the 64 x 64 tile of element e of output tile t
@@ -152,10 +163,13 @@ __device__ __forceinline__ M2 mul2(const M2& x, const M2& y) {
 // cycles). The launch with one block: 31 -> 20 us against vector updates from one
 // thread column each with four divisions per step.
 // A pivot not above tol times its diagonal entry of dg (or above zero when dg is
-// null) clears the return value.
+// null) clears the return value. rows: the block's rows that belong to the matrix; the
+// padding behind them is an identity and needs no step (at 83 rows 21 steps in all
+// instead of 32, 60 -> 46 us for the whole inverse; 142 -> 134 us at 275).
 constexpr int kGjLds = 2 * 4 * kB + 2 * kB * 4;
-__device__ __forceinline__ bool invert_block(v4d (&acc)[4], double* __restrict__ lds, const double* __restrict__ dg,
-                                             double tol) {
+template <bool kPartial>
+__device__ __forceinline__ bool invert_block_rows(v4d (&acc)[4], double* __restrict__ lds, const double* __restrict__ dg,
+                                             double tol, int rows) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i = lane & 15, kk = lane >> 4;
   double* rowb = lds;               // [2][4][64]
@@ -165,6 +179,7 @@ __device__ __forceinline__ bool invert_block(v4d (&acc)[4], double* __restrict__
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int p0 = 16 * q4 + 4 * e;
+      if (kPartial && p0 >= rows) return ok;  // uniform
       double* rb = rowb + (e & 1) * 4 * kB;
       double* cb = colb + (e & 1) * kB * 4;
       if (w == q4) {
@@ -229,6 +244,12 @@ __device__ __forceinline__ bool invert_block(v4d (&acc)[4], double* __restrict__
   }
   return ok;
 }
+// The exit test inside the unrolled steps costs a full block 3 us: two forms.
+__device__ __forceinline__ bool invert_block(v4d (&acc)[4], double* __restrict__ lds, const double* __restrict__ dg,
+                                             double tol, int rows) {
+  return rows >= kB ? invert_block_rows<false>(acc, lds, dg, tol, rows)
+                    : invert_block_rows<true>(acc, lds, dg, tol, rows);
+}
 
 // Block 0: the inverse of the first 64 x 64 pivot block, into P (leading dimension
 // 64; straight into the result, with its transpose PT, when the matrix has no other
@@ -237,7 +258,7 @@ __device__ __forceinline__ bool invert_block(v4d (&acc)[4], double* __restrict__
 // sqrt(a_ii a_jj) (the rounding asymmetry of a Galerkin product passes, a
 // non-symmetric operator does not; well rows can exceed interior rows by 15 orders,
 // so the scale is per entry), and for a positive diagonal, and keeps the diagonal.
-__global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n_pad, int sym_rows, const double* __restrict__ M,
+__global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n, int n_pad, int sym_rows, const double* __restrict__ M,
                                                           double* __restrict__ P, double* __restrict__ PT,
                                                           double* __restrict__ dg, double tol,
                                                           int* __restrict__ bad) {
@@ -271,7 +292,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n_pad, int sym_row
       acc[t][e] = M[(long long)r * n_pad + c];
     }
   __syncthreads();
-  if (!invert_block(acc, lds, dg ? d0 : nullptr, tol)) *bad = 1;
+  if (!invert_block(acc, lds, dg ? d0 : nullptr, tol, min(n, kB))) *bad = 1;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -290,8 +311,8 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n_pad, int sym_row
 // also inverts the next pivot block (fetches, two products of 1.7 us, the inverse);
 // every tile it needs is fetched before the first product. The last block column
 // also writes the transposed inverse (AnT). One launch per block
-// column: 47-49 -> 18-25 us at 128-576 rows.
-__global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, const double* __restrict__ A,
+// column: 47-49 -> 13-24 us at 83-576 rows.
+__global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n, int n_pad, const double* __restrict__ A,
                                                           double* __restrict__ An, const double* __restrict__ P,
                                                           double* __restrict__ Pn, double* __restrict__ AnT,
                                                           const double* __restrict__ dg, double tol,
@@ -311,13 +332,16 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, cons
   }
   v4d acc[4];
   TileRegs ta, tb;
+  // inner indices past the matrix's last row meet zeros: of A_ik, and of P left of its
+  // identity
+  const int depth = n - k * kB;
   if (j == k) {  // A'_ik = -A_ik P
     tile_fetch(blk, n_pad, ta);
     tile_fetch(P, kB, tb);
     tile_put<kLdA>(ta, As);
     tile_put<kLdB>(tb, Bs);
     __syncthreads();
-    tile_mma(As, Bs, acc);
+    tile_mma(As, Bs, depth, acc);
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -335,7 +359,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, cons
     tile_put<kLdA>(ta, As);
     tile_put<kLdB>(tb, Bs);
     __syncthreads();
-    tile_mma(As, Bs, acc);  // P A_kj
+    tile_mma(As, Bs, depth, acc);  // P A_kj
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -363,7 +387,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, cons
   tile_put<kLdB>(tb, Bs);
   tile_put<kLdA>(tc, Cs);
   __syncthreads();
-  tile_mma(As, Bs, acc);  // P A_kj
+  tile_mma(As, Bs, depth, acc);  // P A_kj
   __syncthreads();        // every wave is done reading Bs
 #pragma unroll
   for (int t = 0; t < 4; ++t)
@@ -374,7 +398,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, cons
       Bs[r * kLdB + c] = acc[t][e];
     }
   __syncthreads();
-  tile_mma(Cs, Bs, acc);  // A_ik (P A_kj)
+  tile_mma(Cs, Bs, depth, acc);  // A_ik (P A_kj)
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -388,7 +412,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n_pad, cons
   if (i != k + 1 || j != k + 1 || Pn == nullptr) return;
   // this block is the next step's pivot block: its inverse goes to step k + 1 in Pn
   // (As is free: every wave has passed the barrier behind its last read of it)
-  if (!invert_block(own, As, dg ? d0 : nullptr, tol)) *bad = 1;
+  if (!invert_block(own, As, dg ? d0 : nullptr, tol, min(n - i * kB, kB))) *bad = 1;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -448,14 +472,14 @@ void launch_dense_inverse_mfma(int n, const int* rp, const int* ci, const double
   // P holds two 64 x 64 pivot inverses: step k reads P_k and its block (k+1, k+1)
   // workgroup writes P_{k+1} into the other half. With one block its inverse is the
   // result (n_pad = 64 = the leading dimension of P).
-  k_gj_diag<<<1 + (strict ? n : 0), kGemmThreads, 0, s>>>(n_pad, strict ? n : 0, cur, nb == 1 ? M : P,
+  k_gj_diag<<<1 + (strict ? n : 0), kGemmThreads, 0, s>>>(n, n_pad, strict ? n : 0, cur, nb == 1 ? M : P,
                                                               nb == 1 ? MT : nullptr, dg, tol, bad);
   IMPES_LAUNCH_CHECK();
   if (nb == 1) return;
   for (int k = 0; k < nb; ++k) {
     double* Pk = P + (k & 1) * kB * kB;
     double* Pn = (k + 1 < nb) ? P + ((k + 1) & 1) * kB * kB : nullptr;
-    k_gj_step<<<dim3(nb, nb), kGemmThreads, 0, s>>>(k, n_pad, cur, nxt, Pk, Pn, k + 1 == nb ? MT : nullptr, dg, tol, bad);
+    k_gj_step<<<dim3(nb, nb), kGemmThreads, 0, s>>>(k, n, n_pad, cur, nxt, Pk, Pn, k + 1 == nb ? MT : nullptr, dg, tol, bad);
     IMPES_LAUNCH_CHECK();
     std::swap(cur, nxt);
   }
