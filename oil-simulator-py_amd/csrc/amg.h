@@ -100,6 +100,7 @@ struct Level {
   DevBuf<double> pv, rv;
   DevBuf<float> pv32, rv32;
   Pad4 r4;  // FP32 restriction in the padded tiled form (read instead of rv32 when set)
+  Pad4 s4;  // P - omega D_relax^-1 AP in the same form: prolongation and first post-sweep in one pass
   // Galerkin product data: AP = A*P (values refreshed on update), next A = R*AP
   int apnnz = 0;
   DevBuf<int> aprp, apci;
@@ -226,6 +227,8 @@ class Hierarchy {
   void vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done = false,
                     bool tail = false);
   void choose_tail(hipStream_t s);
+  void build_prolong_sweeps(hipStream_t s);
+  void fill_prolong_sweep(Level& L, int* miss, hipStream_t s);  // values, after every numeric change
   void ensure_tail(int precision, hipStream_t s);
   template <class T>
   void smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& zero, hipStream_t s);

@@ -416,6 +416,7 @@ void Hierarchy::setup_impl(int n, int nnz, const int* rp, const int* ci, const d
   if (stencil_) refresh_stencil(s);
   alloc_vectors();
   choose_tail(s);
+  build_prolong_sweeps(s);
   IMPES_HIP_CHECK(hipStreamSynchronize(s));
   }
   last_setup_seconds = wall() - t0;
@@ -833,6 +834,7 @@ void Hierarchy::update_levels(bool fine_done, hipStream_t s) {
       else launch_pin_decide(L.n, L.rp.p, L.ci.p, L.v.p, L.pin_mode, L.pin.p, L.gj_bad.p, s);
     }
   }
+  for (auto& L : levels_) fill_prolong_sweep(L, nullptr, s);
   if (stencil_ && !fine_done) refresh_stencil(s);
 }
 
@@ -866,6 +868,41 @@ bool Hierarchy::coarse_pinned(hipStream_t s) const {
 LevelInfo Hierarchy::info(int l) const {
   const Level& L = levels_.at(l);
   return LevelInfo{L.n, L.nnz, L.coarsest ? 0 : L.pnnz, L.coarsest ? 1 : 0, L.dense ? 1 : 0};
+}
+
+// ---------------------------------------------------------------- prolongation and sweep
+// After the coarse correction e the first post-sweep is x + P e + w D^-1 (b - A (x + P
+// e)) = x + w D^-1 r + (P - w D^-1 A P) e, with the residual r that the restriction has
+// left: one pass over a matrix with the pattern of AP (already formed for the Galerkin
+// product) instead of one over P and one over A. FP32 cycle, in tiles.
+// Measured, the pass and its share of the refresh against the two passes and the gap
+// between them: CSR levels of 16,000 rows 3.6 against 7.6 us, of 82,000 rows 5.9 against
+// 9.3, of 409,000 rows 19.2 against 21.4. A stencil level's sweep is cheaper than its
+// matrix (7 values a cell, no columns): 76,800 cells 4.1 against 6.4 us, 200,000 cells
+// 7.9 against 8.4, beyond that the two passes.
+constexpr int kSweepStencilMax = 1 << 18;
+void Hierarchy::build_prolong_sweeps(hipStream_t s) {
+  for (auto& L : levels_) L.s4 = Pad4{};
+  if (prm_.post_smooth < 1 && prm_.pre_smooth < 1) return;
+  const int end = tail_ >= 0 ? tail_ : (int)levels_.size() - 1;
+  DevBuf<int> miss;
+  if (end < 1) return;
+  miss.alloc(1);
+  launch_fill_i32(miss.p, 0, 1, s);
+  for (int l = 0; l < end; ++l) {
+    Level& L = levels_[l];
+    if (L.coarsest || (l == 0 && stencil_ && L.n > kSweepStencilMax)) continue;
+    build_pad4_transfer(L.n, L.apnnz, L.aprp.p, L.apci.p, L.apv.p, L.s4, s);
+    fill_prolong_sweep(L, miss.p, s);
+  }
+  // a matrix with a row without a diagonal entry keeps the two passes
+  if (read_scalar(miss.p, s) != 0)
+    for (auto& L : levels_) L.s4 = Pad4{};
+}
+
+void Hierarchy::fill_prolong_sweep(Level& L, int* miss, hipStream_t s) {
+  launch_tile4_prolong_sweep(L.s4.nw, L.s4.wrow.p, L.s4.tag.p, L.s4.rp4.p, L.s4.ci4.p, L.aprp.p, L.apv.p, L.prp.p, L.pci.p,
+                             L.pv.p, L.ir64.p, prm_.omega, L.s4.v4.p, miss, s);
 }
 
 // ---------------------------------------------------------------- coarse tail
@@ -1057,9 +1094,15 @@ double Hierarchy::level_bytes(int l, int precision) const {
   b += (prm_.pre_smooth == 0) ? 2.0 * n * vb : sweep(2.0);  // residual (a copy without pre-smoothing)
   const bool fused = !C.coarsest && prm_.pre_smooth > 0;
   b += csr(C.n, L.pnnz, n, fused ? 3.0 : 1.0);  // restriction (+ the coarse first sweep: inv_relax, b_c, x_c)
-  b += csr(n, L.pnnz, C.n, 2.0);                 // prolongation: x + P e_c
-  b += prm_.post_smooth * sweep(3.0);
-  if (prm_.post_smooth % 2) b += 2.0 * n * vb;  // the final copy back into x
+  int post = prm_.post_smooth;
+  if (precision == 32 && L.s4.nw && post > 0 && prm_.pre_smooth > 0) {
+    b += csr(n, L.apnnz, C.n, 4.0);  // prolongation and a sweep: r, inv_relax, x before and after
+    --post;
+  } else {
+    b += csr(n, L.pnnz, C.n, 2.0);  // prolongation: x + P e_c
+  }
+  b += post * sweep(3.0);
+  if (post == prm_.post_smooth && post % 2) b += 2.0 * n * vb;  // the final copy back into x
   return b;
 }
 
@@ -1154,6 +1197,18 @@ void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s
   segment(l, m0, mark(s));
   vcycle_level<T>(l + 1, Sel<T>::b(C), Sel<T>::x(C), true, s, fused, tail);
   const int m1 = mark(s);
+  if constexpr (sizeof(T) == 4) {
+    if (!zero && prm_.post_smooth > 0 && L.s4.nw) {
+      // the sweeps after the fused one alternate between x and t and end in x
+      float* out = (prm_.post_smooth % 2 == 1) ? x : L.t32.p;
+      launch_prolong_sweep4_f32(Sel<T>::T4(L.s4), C.x32.p, r, L.ir32.p, (float)prm_.omega, cur, out, s);
+      cur = out;
+      other = (cur == x) ? L.t32.p : x;
+      smooth<T>(l, b, cur, other, prm_.post_smooth - 1, zero, s);
+      segment(l, m1, mark(s));
+      return;
+    }
+  }
   // Post-smoothing alternates between x and t: prolongate into the buffer from
   // which post_smooth sweeps end in x, so the cycle needs no final copy.
   T* target = (prm_.post_smooth % 2 == 0) ? x : Sel<T>::t(L);

@@ -108,6 +108,14 @@ void launch_jacobi4_f32(const Csr4F32& A, int group, const float* xi, const floa
 // restriction on a padded operator with wave tiles (A.nw > 0; column indices in ci4): y = A x; and y = A x with y2 = w inv_relax2 .* y (fused with the coarse
 // level's first sweep from zero)
 void launch_spmv4_f32(const Csr4F32& A, const float* x, float* y, hipStream_t s);
+// prolongation and the sweep after it, S = P - w diag(inv_relax) AP in tiles: x = x0 +
+// w inv_relax .* r + S e (r = b - A x0; x may be x0); and the values of S, with the count of P's entries outside
+// its pattern added to *miss (or null)
+void launch_prolong_sweep4_f32(const Csr4F32& S, const float* e, const float* r, const float* inv_relax, float w,
+                               float* x0, float* x, hipStream_t s);
+void launch_tile4_prolong_sweep(int nw, const int* wrow, const unsigned short* tag, const int* rp4, const int* ci4,
+                                const int* aprp, const double* apv, const int* prp, const int* pci, const double* pv, const double* ir,
+                                double w, float* v4, int* miss, hipStream_t s);
 void launch_restrict4_j0_f32(const Csr4F32& R, const float* r, const float* inv_relax_c, float w, float* bc, float* xc,
                              hipStream_t s);
 

@@ -27,8 +27,12 @@ constexpr int kBlock = 256;
 // kJacZ0 (stencil): two L1-Jacobi sweeps from a zero guess in one pass: the first
 // sweep's x = w * aux .* b is formed at every stencil point instead of being read
 // (the expression of k_jacobi0), then y = x + w * aux .* (b - A x) as kJac
+// kProlongJac (padded tiles): y = y2 + w * aux .* b + A x, the prolongation and the first
+// L1-Jacobi sweep after it with A = P - w diag(aux) (A_l P), x the coarse correction, b
+// the residual and y2 the iterate before the correction (y may be y2)
 enum Mode {
-  kY = 0, kYAdd = 1, kRes = 2, kJac = 3, kRowScaled = 4, kRowScaledRes = 5, kRestrictJ0 = 6, kYPlusB = 7, kJacZ0 = 8
+  kY = 0, kYAdd = 1, kRes = 2, kJac = 3, kRowScaled = 4, kRowScaledRes = 5, kRestrictJ0 = 6, kYPlusB = 7, kJacZ0 = 8,
+  kProlongJac = 9
 };
 
 template <int G, class T, class TA, int MODE>
@@ -140,7 +144,7 @@ __global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restr
                                                        const int4* __restrict__ ci4, const short4* __restrict__ co4,
                                                        const float4* __restrict__ v4, const float* __restrict__ x,
                                                        const float* __restrict__ b, const float* __restrict__ aux,
-                                                       float w, float* __restrict__ y, float* __restrict__ y2) {
+                                                       float w, float* y, float* y2) {
   constexpr int WPB = kBlock / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   for (int t = (int)xcd_block() * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); t < nw;
@@ -158,9 +162,10 @@ __global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restr
     if (OFF16) c = make_int4(row + o.x, row + o.y, row + o.z, row + o.w);
     float ob = 0.f, ox = 0.f, oa = 0.f;
     if (last) {
-      if (MODE == kRes || MODE == kJac) ob = b[row];
+      if (MODE == kRes || MODE == kJac || MODE == kProlongJac) ob = b[row];
       if (MODE == kJac) ox = x[row];
-      if (MODE == kJac || MODE == kRestrictJ0) oa = aux[row];
+      if (MODE == kProlongJac) ox = y2[row];
+      if (MODE == kJac || MODE == kRestrictJ0 || MODE == kProlongJac) oa = aux[row];
     }
     float sum = 0.f;
     sum += a.x * x[c.x];
@@ -176,6 +181,7 @@ __global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restr
     if (last) {
       if (MODE == kRes) y[row] = ob - sum;
       else if (MODE == kJac) y[row] = ox + w * oa * (ob - sum);
+      else if (MODE == kProlongJac) y[row] = (ox + w * oa * ob) + sum;
       else if (MODE == kY) y[row] = sum;
       else if (MODE == kRestrictJ0) {
         y[row] = sum;
@@ -277,6 +283,53 @@ __global__ __launch_bounds__(kBlock) void k_tile4_fill(int nw, const int* __rest
   if (!maxabs) return;
   far = wave_max(far);
   if (lane == 0 && far > 0) atomicMax(maxabs, far);
+}
+
+// Values of a tiled P - w diag(ir) AP on AP's pattern (P's is part of it: A has its
+// diagonal): a lane per chunk, its row's few entries of P compared with the chunk's four
+// columns. Formed in FP64, rounded once. miss (or null): adds the entries of P that AP's
+// pattern lacks (a row without a diagonal entry).
+__global__ __launch_bounds__(kBlock) void k_tile4_prolong_sweep(int nw, const int* __restrict__ wrow,
+                                                                const unsigned short* __restrict__ tag,
+                                                                const int* __restrict__ rp4,
+                                                                const int4* __restrict__ ci4,
+                                                                const int* __restrict__ aprp,
+                                                                const double* __restrict__ apv,
+                                                                const int* __restrict__ prp,
+                                                                const int* __restrict__ pci,
+                                                                const double* __restrict__ pv,
+                                                                const double* __restrict__ ir, double w,
+                                                                float4* __restrict__ v4, int* __restrict__ miss) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int lack = 0;
+  for (int t = (int)xcd_block() * (kBlock / kWave) + threadIdx.x / kWave; t < nw; t += gridDim.x * (kBlock / kWave)) {
+    const long long q = (long long)t * kWave + lane;
+    const unsigned tg = tag[q];
+    const int4 c4 = ci4[q];
+    const int row = wrow[t] + (int)(tg & 63u), pos = (int)(tg >> 6 & 63u);
+    const bool used = (rp4[row] >> 2) + pos == q;  // not a spare chunk at the tile's end
+    const int e0 = aprp[row] + 4 * pos, e1 = used ? aprp[row + 1] : 0, p0 = prp[row], p1 = prp[row + 1];
+    const double s = w * ir[row];
+    const int c[4] = {c4.x, c4.y, c4.z, c4.w};
+    double a[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) a[m] = e0 + m < e1 ? -s * apv[e0 + m] : 0.0;
+    for (int e = p0; e < p1; ++e) {
+      const int col = pci[e];
+      const double v = pv[e];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const bool hit = e0 + m < e1 && c[m] == col;
+        a[m] += hit ? v : 0.0;
+        lack -= hit ? 1 : 0;
+      }
+    }
+    if (tg >> 12) lack += p1 - p0;
+    v4[q] = make_float4((float)a[0], (float)a[1], (float)a[2], (float)a[3]);
+  }
+  if (!miss) return;
+  lack = wave_sum(lack);
+  if (lane == 0 && lack != 0) atomicAdd(miss, lack);
 }
 
 template <int MODE, bool OFF16>
@@ -793,6 +846,23 @@ void launch_restrict4_j0_f32(const Csr4F32& R, const float* r, const float* inv_
   IMPES_REQUIRE(R.nw > 0 && !R.co4, "padded transfer: wave tiles and column indices required");
   if (R.n <= 0) return;
   csr4_tile_launch<kRestrictJ0, false>(R, r, nullptr, inv_relax_c, w, bc, s, xc);
+  IMPES_LAUNCH_CHECK();
+}
+void launch_prolong_sweep4_f32(const Csr4F32& S, const float* e, const float* r, const float* inv_relax, float w,
+                               float* x0, float* x, hipStream_t s) {
+  IMPES_REQUIRE(S.nw > 0 && !S.co4, "padded transfer: wave tiles and column indices required");
+  if (S.n <= 0) return;
+  KScope ks("csr_prolong_sweep_f32", csr_bytes(S.n, S.nnz, 4, 4), s);
+  csr4_tile_launch<kProlongJac, false>(S, e, r, inv_relax, w, x, s, x0);
+  IMPES_LAUNCH_CHECK();
+}
+void launch_tile4_prolong_sweep(int nw, const int* wrow, const unsigned short* tag, const int* rp4, const int* ci4,
+                                const int* aprp, const double* apv, const int* prp, const int* pci, const double* pv, const double* ir,
+                                double w, float* v4, int* miss, hipStream_t s) {
+  if (nw <= 0) return;
+  k_tile4_prolong_sweep<<<grid_for(nw, kBlock / kWave, 1 << 18), kBlock, 0, s>>>(
+      nw, wrow, tag, rp4, reinterpret_cast<const int4*>(ci4), aprp, apv, prp, pci, pv, ir, w, reinterpret_cast<float4*>(v4),
+      miss);
   IMPES_LAUNCH_CHECK();
 }
 void launch_restrict_j0_f64(const CsrF64& R, const double* r, const double* inv_relax_c, double w, double* bc,
