@@ -72,6 +72,7 @@ struct Pad4 {
   DevBuf<int> rp4, ci4, wrow;
   DevBuf<unsigned short> tag;
   DevBuf<float> v4;
+  DevBuf<double> v8;  // FP64 values (Hierarchy::ensure_tiles64)
 };
 
 struct Level {
@@ -93,6 +94,7 @@ struct Level {
   DevBuf<int> wrow4;
   DevBuf<unsigned short> tag4;
   DevBuf<float> v4;
+  DevBuf<double> v8;         // FP64 values of the tiles (ensure_tiles64)
   DevBuf<signed char> cf;  // final C/F markers (non-coarsest levels)
   // interpolation / restriction to the next level
   int nc = 0, pnnz = 0, pgroup = 1, rgroup = 1;
@@ -228,10 +230,12 @@ class Hierarchy {
                     bool tail = false);
   void choose_tail(hipStream_t s);
   void build_prolong_sweeps(hipStream_t s);
+  void ensure_sweeps32(hipStream_t s);
+  void ensure_tiles64(hipStream_t s);
   void fill_prolong_sweep(Level& L, int* miss, hipStream_t s);  // values, after every numeric change
   void ensure_tail(int precision, hipStream_t s);
   template <class T>
-  void smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& zero, hipStream_t s);
+  void smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& zero, hipStream_t s, bool tiles = false);
   template <class T>
   void coarse_solve(int l, const T* b, T* x, hipStream_t s);
   void drop_graphs();
@@ -261,6 +265,8 @@ class Hierarchy {
   int tail_ = -1;
   bool tail_ready_[2] = {false, false};
   int tail_ld_ = 0;
+  bool sweeps32_ready_ = false;  // the fused sweeps' FP32 values are those of the operators
+  bool tiles64_ready_ = false;  // the levels' FP64 tile values are those of the operators
   std::vector<long long> tail_at_;   // per level from tail_: first slice offset in tail_so_
   std::vector<long long> tail_line_; // per level from tail_: first line in tail_ell_ (last: the total)
   DevBuf<int> tail_so_;

@@ -200,11 +200,29 @@ struct Sel<double> {
   static void jac0(const double* b, const double* ir, double w, double* xo, int n, hipStream_t s) {
     launch_jacobi0_f64(b, ir, w, xo, n, s);
   }
-  static void jacL(const Level& L, const double* xi, const double* b, double w, double* xo, hipStream_t s) {
-    launch_jacobi_f64(A(L), xi, b, L.ir64.p, w, xo, L.group, s);
+  // the patterns of the padded tiled forms (their FP64 values are in v8)
+  static Csr4F32 A4(const Level& L) {
+    Csr4F32 A;
+    A.n = L.n;
+    A.nnz = L.nnz;
+    A.rp4 = L.rp4.p;
+    A.ci4 = reinterpret_cast<const int4*>(L.ci4.p);
+    A.co4 = reinterpret_cast<const short4*>(L.co4.p);
+    A.nw = L.nw4;
+    A.wrow = L.wrow4.p;
+    A.tag = L.tag4.p;
+    return A;
   }
-  static void resL(const Level& L, const double* x, const double* b, double* r, hipStream_t s) {
-    launch_residual_f64(A(L), x, b, r, L.group, s);
+  static Csr4F32 T4(const Pad4& T) {
+    return Csr4F32{T.n, T.nnz, T.rp4.p, reinterpret_cast<const int4*>(T.ci4.p), nullptr, nullptr, T.nw, T.wrow.p, T.tag.p};
+  }
+  static void jacL(const Level& L, const double* xi, const double* b, double w, double* xo, hipStream_t s, bool tiles) {
+    if (tiles && L.v8.p) launch_jacobi4_f64(A4(L), L.v8.p, xi, b, L.ir64.p, w, xo, s);
+    else launch_jacobi_f64(A(L), xi, b, L.ir64.p, w, xo, L.group, s);
+  }
+  static void resL(const Level& L, const double* x, const double* b, double* r, hipStream_t s, bool tiles) {
+    if (tiles && L.v8.p) launch_residual4_f64(A4(L), L.v8.p, x, b, r, s);
+    else launch_residual_f64(A(L), x, b, r, L.group, s);
   }
   static void res(const CsrF64& A, const double* x, const double* b, double* r, int g, hipStream_t s) {
     launch_residual_f64(A, x, b, r, g, s);
@@ -222,9 +240,19 @@ struct Sel<double> {
   static void pin0(const int* pin, double* b, hipStream_t s) { launch_pin_rhs_f64(pin, b, s); }
   // grid transfers of level L (P: n x nc, R: nc x n)
   static void restrict_j0(const Level& L, const double* r, const double* irc, double w, double* bc, double* xc,
-                          hipStream_t s) { launch_restrict_j0_f64(R(L), r, irc, w, bc, xc, L.rgroup, s); }
-  static void restrict_to(const Level& L, const double* r, double* bc, hipStream_t s) {
-    launch_spmv_f64(R(L), r, bc, L.rgroup, s);
+                          hipStream_t s, bool tiles) {
+    if (tiles && L.r4.v8.p) launch_restrict4_j0_f64(T4(L.r4), L.r4.v8.p, r, irc, w, bc, xc, s);
+    else launch_restrict_j0_f64(R(L), r, irc, w, bc, xc, L.rgroup, s);
+  }
+  static void restrict_to(const Level& L, const double* r, double* bc, hipStream_t s, bool tiles) {
+    if (tiles && L.r4.v8.p) launch_spmv4_f64(T4(L.r4), L.r4.v8.p, r, bc, s);
+    else launch_spmv_f64(R(L), r, bc, L.rgroup, s);
+  }
+  static bool prolong_sweep(const Level& L, const double* e, const double* r, double w, double* x0, double* x,
+                            hipStream_t s, bool tiles) {
+    if (!tiles || !L.s4.v8.p) return false;
+    launch_prolong_sweep4_f64(T4(L.s4), L.s4.v8.p, e, r, L.ir64.p, w, x0, x, s);
+    return true;
   }
   static void prolong(const Level& L, const double* e, double* y, hipStream_t s) {
     launch_spmv_f64(P(L), e, y, L.pgroup, s);
@@ -258,11 +286,11 @@ struct Sel<float> {
     return Csr4F32{L.n, L.nnz, L.rp4.p, reinterpret_cast<const int4*>(L.ci4.p), reinterpret_cast<const float4*>(L.v4.p),
                    reinterpret_cast<const short4*>(L.co4.p), L.nw4, L.wrow4.p, L.tag4.p};
   }
-  static void jacL(const Level& L, const float* xi, const float* b, double w, float* xo, hipStream_t s) {
+  static void jacL(const Level& L, const float* xi, const float* b, double w, float* xo, hipStream_t s, bool) {
     if (L.pad4) launch_jacobi4_f32(A4(L), L.g4, xi, b, L.ir32.p, (float)w, xo, s);
     else launch_jacobi_f32(A(L), xi, b, L.ir32.p, (float)w, xo, L.group, s);
   }
-  static void resL(const Level& L, const float* x, const float* b, float* r, hipStream_t s) {
+  static void resL(const Level& L, const float* x, const float* b, float* r, hipStream_t s, bool) {
     if (L.pad4) launch_residual4_f32(A4(L), L.g4, x, b, r, s);
     else launch_residual_f32(A(L), x, b, r, L.group, s);
   }
@@ -286,13 +314,19 @@ struct Sel<float> {
                    nullptr, T.nw, T.wrow.p, T.tag.p};
   }
   static void restrict_j0(const Level& L, const float* r, const float* irc, double w, float* bc, float* xc,
-                          hipStream_t s) {
+                          hipStream_t s, bool) {
     if (L.r4.nw) launch_restrict4_j0_f32(T4(L.r4), r, irc, (float)w, bc, xc, s);
     else launch_restrict_j0_f32(R(L), r, irc, (float)w, bc, xc, L.rgroup, s);
   }
-  static void restrict_to(const Level& L, const float* r, float* bc, hipStream_t s) {
+  static void restrict_to(const Level& L, const float* r, float* bc, hipStream_t s, bool) {
     if (L.r4.nw) launch_spmv4_f32(T4(L.r4), r, bc, s);
     else launch_spmv_f32(R(L), r, bc, L.rgroup, s);
+  }
+  static bool prolong_sweep(const Level& L, const float* e, const float* r, double w, float* x0, float* x,
+                            hipStream_t s, bool) {
+    if (!L.s4.nw) return false;
+    launch_prolong_sweep4_f32(T4(L.s4), e, r, L.ir32.p, (float)w, x0, x, s);
+    return true;
   }
   static void prolong(const Level& L, const float* e, float* y, hipStream_t s) {
     launch_spmv_f32(P(L), e, y, L.pgroup, s);
@@ -808,6 +842,7 @@ void Hierarchy::update_csr_values(const double* v, hipStream_t s) {
 
 void Hierarchy::update_levels(bool fine_done, hipStream_t s) {
   tail_ready_[0] = tail_ready_[1] = false;
+  tiles64_ready_ = false;
   for (int l = 0; l + 1 < (int)levels_.size(); ++l) {
     Level& A = levels_[l];
     if (A.coarsest) break;
@@ -834,7 +869,7 @@ void Hierarchy::update_levels(bool fine_done, hipStream_t s) {
       else launch_pin_decide(L.n, L.rp.p, L.ci.p, L.v.p, L.pin_mode, L.pin.p, L.gj_bad.p, s);
     }
   }
-  for (auto& L : levels_) fill_prolong_sweep(L, nullptr, s);
+  sweeps32_ready_ = false;
   if (stencil_ && !fine_done) refresh_stencil(s);
 }
 
@@ -898,11 +933,44 @@ void Hierarchy::build_prolong_sweeps(hipStream_t s) {
   // a matrix with a row without a diagonal entry keeps the two passes
   if (read_scalar(miss.p, s) != 0)
     for (auto& L : levels_) L.s4 = Pad4{};
+  sweeps32_ready_ = true;
+}
+
+// the FP32 values, when a cycle first needs them after a numeric update
+void Hierarchy::ensure_sweeps32(hipStream_t s) {
+  if (sweeps32_ready_) return;
+  for (auto& L : levels_) fill_prolong_sweep(L, nullptr, s);
+  sweeps32_ready_ = true;
 }
 
 void Hierarchy::fill_prolong_sweep(Level& L, int* miss, hipStream_t s) {
   launch_tile4_prolong_sweep(L.s4.nw, L.s4.wrow.p, L.s4.tag.p, L.s4.rp4.p, L.s4.ci4.p, L.aprp.p, L.apv.p, L.prp.p, L.pci.p,
-                             L.pv.p, L.ir64.p, prm_.omega, L.s4.v4.p, miss, s);
+                             L.pv.p, L.ir64.p, prm_.omega, L.s4.v4.p, nullptr, miss, s);
+}
+
+// FP64 values of the tiles above the tail, when the FP64 preconditioner first needs them
+// after a numeric change (262,000 cells: 65 us a refresh, against about 30 us saved per cycle)
+void Hierarchy::ensure_tiles64(hipStream_t s) {
+  if (tiles64_ready_) return;
+  const int end = tail_ >= 0 ? tail_ : (int)levels_.size() - 1;
+  for (int l = 0; l < end; ++l) {
+    Level& L = levels_[l];
+    if (L.coarsest) break;
+    if (L.pad4 && L.nw4 > 0) {
+      L.v8.alloc(4 * (size_t)L.nw4 * kWave);
+      launch_tile4_values_f64(Sel<double>::A4(L), L.rp.p, L.v.p, L.v8.p, s);
+    }
+    if (L.r4.nw && !L.r4.v8.p) {  // fixed until the next setup
+      L.r4.v8.alloc(4 * (size_t)L.r4.nw * kWave);
+      launch_tile4_values_f64(Sel<double>::T4(L.r4), L.rrp.p, L.rv.p, L.r4.v8.p, s);
+    }
+    if (L.s4.nw) {
+      L.s4.v8.alloc(4 * (size_t)L.s4.nw * kWave);
+      launch_tile4_prolong_sweep(L.s4.nw, L.s4.wrow.p, L.s4.tag.p, L.s4.rp4.p, L.s4.ci4.p, L.aprp.p, L.apv.p,
+                                 L.prp.p, L.pci.p, L.pv.p, L.ir64.p, prm_.omega, nullptr, L.s4.v8.p, nullptr, s);
+    }
+  }
+  tiles64_ready_ = true;
 }
 
 // ---------------------------------------------------------------- coarse tail
@@ -915,6 +983,7 @@ void Hierarchy::fill_prolong_sweep(Level& L, int* miss, hipStream_t s) {
 void Hierarchy::choose_tail(hipStream_t s) {
   tail_ = -1;
   tail_ready_[0] = tail_ready_[1] = false;
+  tiles64_ready_ = false;
   tail_at_.clear();
   tail_line_.clear();
   const int last = (int)levels_.size() - 1;
@@ -994,7 +1063,7 @@ void Hierarchy::ensure_tail(int precision, hipStream_t s) {
 
 // ---------------------------------------------------------------- V-cycle
 template <class T>
-void Hierarchy::smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& zero, hipStream_t s) {
+void Hierarchy::smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& zero, hipStream_t s, bool tiles) {
   Level& L = levels_[l];
   const bool st = (l == 0 && stencil_);
   for (int it = 0; it < sweeps; ++it) {
@@ -1026,7 +1095,7 @@ void Hierarchy::smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& z
         launch_st7_jacobi_f32(S, (const float*)cur, (const float*)b, L.ir32.p, (float)prm_.omega, (float*)other, s);
       }
     } else {
-      Sel<T>::jacL(L, cur, b, prm_.omega, other, s);
+      Sel<T>::jacL(L, cur, b, prm_.omega, other, s, tiles);
     }
     std::swap(cur, other);
   }
@@ -1154,9 +1223,12 @@ void Hierarchy::level_times(int precision, int cycles, double* ms, double* cycle
   }
 }
 
+// tail: the preconditioner's cycle, which may use the tail matrix and the FP64 tiles
+// (ensure_tail and ensure_tiles64 come before it)
 template <class T>
 void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done, bool tail) {
   Level& L = levels_[l];
+  if (sizeof(T) == 4 && l == 0) ensure_sweeps32(s);  // done before a capture
   if (tail && l == tail_) {
     if constexpr (sizeof(T) == 8) launch_tail_mv_f64(L.n, tail_ld_, tail_b64_.p, b, x, s);
     else launch_tail_mv_f32(L.n, tail_ld_, tail_b32_.p, b, x, s);
@@ -1171,7 +1243,7 @@ void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s
   T* cur = x;
   T* other = Sel<T>::t(L);
   bool zero = x_zero && !first_sweep_done;
-  smooth<T>(l, b, cur, other, prm_.pre_smooth - (first_sweep_done ? 1 : 0), zero, s);
+  smooth<T>(l, b, cur, other, prm_.pre_smooth - (first_sweep_done ? 1 : 0), zero, s, tail);
   T* r = Sel<T>::r(L);
   if (zero) {
     Sel<T>::copy(r, b, L.n, s);  // no pre-smoothing: r = b - A*0
@@ -1184,27 +1256,26 @@ void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s
       launch_st7_residual_f32(S, (const float*)cur, (const float*)b, (float*)r, s);
     }
   } else {
-    Sel<T>::resL(L, cur, b, r, s);
+    Sel<T>::resL(L, cur, b, r, s, tail);
   }
   Level& C = levels_[l + 1];
   const bool fused = !C.coarsest && prm_.pre_smooth > 0 && !(tail && l + 1 == tail_);
   if (fused) {
     // restriction fused with the coarse level's first sweep from zero
-    Sel<T>::restrict_j0(L, r, Sel<T>::ir(C), prm_.omega, Sel<T>::b(C), Sel<T>::x(C), s);
+    Sel<T>::restrict_j0(L, r, Sel<T>::ir(C), prm_.omega, Sel<T>::b(C), Sel<T>::x(C), s, tail);
   } else {
-    Sel<T>::restrict_to(L, r, Sel<T>::b(C), s);
+    Sel<T>::restrict_to(L, r, Sel<T>::b(C), s, tail);
   }
   segment(l, m0, mark(s));
   vcycle_level<T>(l + 1, Sel<T>::b(C), Sel<T>::x(C), true, s, fused, tail);
   const int m1 = mark(s);
-  if constexpr (sizeof(T) == 4) {
-    if (!zero && prm_.post_smooth > 0 && L.s4.nw) {
-      // the sweeps after the fused one alternate between x and t and end in x
-      float* out = (prm_.post_smooth % 2 == 1) ? x : L.t32.p;
-      launch_prolong_sweep4_f32(Sel<T>::T4(L.s4), C.x32.p, r, L.ir32.p, (float)prm_.omega, cur, out, s);
+  if (!zero && prm_.post_smooth > 0) {
+    // the sweeps after the fused one alternate between x and t and end in x
+    T* out = (prm_.post_smooth % 2 == 1) ? x : Sel<T>::t(L);
+    if (Sel<T>::prolong_sweep(L, Sel<T>::x(C), r, prm_.omega, cur, out, s, tail)) {
       cur = out;
-      other = (cur == x) ? L.t32.p : x;
-      smooth<T>(l, b, cur, other, prm_.post_smooth - 1, zero, s);
+      other = (cur == x) ? Sel<T>::t(L) : x;
+      smooth<T>(l, b, cur, other, prm_.post_smooth - 1, zero, s, tail);
       segment(l, m1, mark(s));
       return;
     }
@@ -1223,7 +1294,7 @@ void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s
   }
   cur = target;
   other = (cur == x) ? Sel<T>::t(L) : x;
-  smooth<T>(l, b, cur, other, prm_.post_smooth, zero, s);
+  smooth<T>(l, b, cur, other, prm_.post_smooth, zero, s, tail);
   if (cur != x) Sel<T>::copy(x, cur, L.n, s);
   segment(l, m1, mark(s));
 }
@@ -1331,6 +1402,8 @@ void Hierarchy::vcycle_only(int precision, hipStream_t s) {
   const bool replay = graphs_ && !ktimer_enabled() && tail_ != 0;
   const int gi = precision == 32 ? 0 : 1;
   ensure_tail(precision, s);
+  if (precision == 64) ensure_tiles64(s);
+  else ensure_sweeps32(s);
   if (replay && !vexec_[gi]) capture_vcycle(precision);
   if (replay) IMPES_HIP_CHECK(hipGraphLaunch(vexec_[gi], s));
   else if (precision == 32) vcycle_level<float>(0, L0.b32.p, L0.x32.p, true, s, false, true);

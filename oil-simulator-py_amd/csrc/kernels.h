@@ -115,7 +115,20 @@ void launch_prolong_sweep4_f32(const Csr4F32& S, const float* e, const float* r,
                                float* x0, float* x, hipStream_t s);
 void launch_tile4_prolong_sweep(int nw, const int* wrow, const unsigned short* tag, const int* rp4, const int* ci4,
                                 const int* aprp, const double* apv, const int* prp, const int* pci, const double* pv, const double* ir,
-                                double w, float* v4, int* miss, hipStream_t s);
+                                double w, float* v4, double* v8, int* miss, hipStream_t s);
+// tiled patterns with FP64 values v8 (4 per chunk, 16-byte aligned; A.v4 is not read):
+// the values from CSR ones, and the passes above (launch_tile4_prolong_sweep fills v8
+// when it is given, else v4)
+void launch_tile4_values_f64(const Csr4F32& A, const int* rp, const double* v, double* v8, hipStream_t s);
+void launch_residual4_f64(const Csr4F32& A, const double* v8, const double* x, const double* b, double* r,
+                          hipStream_t s);
+void launch_jacobi4_f64(const Csr4F32& A, const double* v8, const double* xi, const double* b, const double* inv_relax,
+                        double w, double* xo, hipStream_t s);
+void launch_spmv4_f64(const Csr4F32& A, const double* v8, const double* x, double* y, hipStream_t s);
+void launch_restrict4_j0_f64(const Csr4F32& R, const double* v8, const double* r, const double* inv_relax_c, double w,
+                             double* bc, double* xc, hipStream_t s);
+void launch_prolong_sweep4_f64(const Csr4F32& S, const double* v8, const double* e, const double* r,
+                               const double* inv_relax, double w, double* x0, double* x, hipStream_t s);
 void launch_restrict4_j0_f32(const Csr4F32& R, const float* r, const float* inv_relax_c, float w, float* bc, float* xc,
                              hipStream_t s);
 

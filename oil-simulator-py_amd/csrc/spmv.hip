@@ -138,19 +138,31 @@ __global__ __launch_bounds__(kBlock) void k_csr4(int n, const int* __restrict__ 
 // two shuffles: 8.6 -> 7.6 us per sweep over the 1M-cell hierarchy's levels (level 1,
 // 58 MB: 15.2 -> 13.7 us), 4.2 -> 3.6 us over the 200k-cell hierarchy's; the sums are
 // the same bits.
-template <int MODE, bool OFF16>
+// FP64 values (two 16-byte loads per chunk) serve the FP64 cycle: against a group of lanes
+// per CSR row, sweeps over 116,000 rows 9.6 -> 7.4 us, over 35,000 rows of 29 entries
+// 8.4 -> 6.3 us.
+template <class T>
+__device__ __forceinline__ void ld_chunk(const T* __restrict__ v, long long q, T (&a)[4]) {
+#pragma unroll
+  for (int h = 0; h < 4 * (int)sizeof(T) / 16; ++h)
+    __builtin_memcpy(reinterpret_cast<unsigned char*>(a) + 16 * h,
+                     __builtin_assume_aligned(reinterpret_cast<const unsigned char*>(v + 4 * q) + 16 * h, 16), 16);
+}
+
+template <class T, int MODE, bool OFF16>
 __global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restrict__ wrow,
                                                        const unsigned short* __restrict__ tag,
                                                        const int4* __restrict__ ci4, const short4* __restrict__ co4,
-                                                       const float4* __restrict__ v4, const float* __restrict__ x,
-                                                       const float* __restrict__ b, const float* __restrict__ aux,
-                                                       float w, float* y, float* y2) {
+                                                       const T* __restrict__ v4, const T* __restrict__ x,
+                                                       const T* __restrict__ b, const T* __restrict__ aux, T w, T* y,
+                                                       T* y2) {
   constexpr int WPB = kBlock / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   for (int t = (int)xcd_block() * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); t < nw;
        t += gridDim.x * WPB) {
     const long long q = (long long)t * kWave + lane;
-    const float4 a = v4[q];
+    T a[4];
+    ld_chunk(v4, q, a);
     const unsigned tg = tag[q];
     int4 c;
     short4 o;
@@ -160,22 +172,22 @@ __global__ __launch_bounds__(kBlock) void k_csr4_tile(int nw, const int* __restr
     const int pos = (int)(tg >> 6 & 63u);
     const bool last = (tg >> 12) != 0;
     if (OFF16) c = make_int4(row + o.x, row + o.y, row + o.z, row + o.w);
-    float ob = 0.f, ox = 0.f, oa = 0.f;
+    T ob = T(0), ox = T(0), oa = T(0);
     if (last) {
       if (MODE == kRes || MODE == kJac || MODE == kProlongJac) ob = b[row];
       if (MODE == kJac) ox = x[row];
       if (MODE == kProlongJac) ox = y2[row];
       if (MODE == kJac || MODE == kRestrictJ0 || MODE == kProlongJac) oa = aux[row];
     }
-    float sum = 0.f;
-    sum += a.x * x[c.x];
-    sum += a.y * x[c.y];
-    sum += a.z * x[c.z];
-    sum += a.w * x[c.w];
+    T sum = T(0);
+    sum += a[0] * x[c.x];
+    sum += a[1] * x[c.y];
+    sum += a[2] * x[c.z];
+    sum += a[3] * x[c.w];
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
       if (!__any(pos >= d)) break;  // uniform
-      const float u = __shfl_up(sum, d, kWave);
+      const T u = __shfl_up(sum, d, kWave);
       if (pos >= d) sum += u;
     }
     if (last) {
@@ -285,10 +297,31 @@ __global__ __launch_bounds__(kBlock) void k_tile4_fill(int nw, const int* __rest
   if (lane == 0 && far > 0) atomicMax(maxabs, far);
 }
 
+// FP64 values of a tiled matrix from its CSR values
+__global__ __launch_bounds__(kBlock) void k_tile4_values_f64(int nw, const int* __restrict__ wrow,
+                                                             const unsigned short* __restrict__ tag,
+                                                             const int* __restrict__ rp4, const int* __restrict__ rp,
+                                                             const double* __restrict__ v, double2* __restrict__ v8) {
+  const int lane = threadIdx.x & (kWave - 1);
+  for (int t = (int)xcd_block() * (kBlock / kWave) + threadIdx.x / kWave; t < nw; t += gridDim.x * (kBlock / kWave)) {
+    const long long q = (long long)t * kWave + lane;
+    const unsigned tg = tag[q];
+    const int row = wrow[t] + (int)(tg & 63u), pos = (int)(tg >> 6 & 63u);
+    const bool used = (rp4[row] >> 2) + pos == q;  // not a spare chunk at the tile's end
+    const int e0 = rp[row] + 4 * pos, e1 = used ? rp[row + 1] : 0;
+    double a[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) a[m] = e0 + m < e1 ? v[e0 + m] : 0.0;
+    v8[2 * q] = make_double2(a[0], a[1]);
+    v8[2 * q + 1] = make_double2(a[2], a[3]);
+  }
+}
+
 // Values of a tiled P - w diag(ir) AP on AP's pattern (P's is part of it: A has its
 // diagonal): a lane per chunk, its row's few entries of P compared with the chunk's four
-// columns. Formed in FP64, rounded once. miss (or null): adds the entries of P that AP's
+// columns. Formed in FP64, rounded once for FP32. miss (or null): adds the entries of P that AP's
 // pattern lacks (a row without a diagonal entry).
+template <class T>
 __global__ __launch_bounds__(kBlock) void k_tile4_prolong_sweep(int nw, const int* __restrict__ wrow,
                                                                 const unsigned short* __restrict__ tag,
                                                                 const int* __restrict__ rp4,
@@ -299,7 +332,7 @@ __global__ __launch_bounds__(kBlock) void k_tile4_prolong_sweep(int nw, const in
                                                                 const int* __restrict__ pci,
                                                                 const double* __restrict__ pv,
                                                                 const double* __restrict__ ir, double w,
-                                                                float4* __restrict__ v4, int* __restrict__ miss) {
+                                                                T* __restrict__ v4, int* __restrict__ miss) {
   const int lane = threadIdx.x & (kWave - 1);
   int lack = 0;
   for (int t = (int)xcd_block() * (kBlock / kWave) + threadIdx.x / kWave; t < nw; t += gridDim.x * (kBlock / kWave)) {
@@ -325,7 +358,12 @@ __global__ __launch_bounds__(kBlock) void k_tile4_prolong_sweep(int nw, const in
       }
     }
     if (tg >> 12) lack += p1 - p0;
-    v4[q] = make_float4((float)a[0], (float)a[1], (float)a[2], (float)a[3]);
+    if constexpr (sizeof(T) == 4) {
+      reinterpret_cast<float4*>(v4)[q] = make_float4((float)a[0], (float)a[1], (float)a[2], (float)a[3]);
+    } else {
+      reinterpret_cast<double2*>(v4)[2 * q] = make_double2(a[0], a[1]);
+      reinterpret_cast<double2*>(v4)[2 * q + 1] = make_double2(a[2], a[3]);
+    }
   }
   if (!miss) return;
   lack = wave_sum(lack);
@@ -336,8 +374,24 @@ template <int MODE, bool OFF16>
 void csr4_tile_launch(const Csr4F32& A, const float* x, const float* b, const float* aux, float w, float* y,
                       hipStream_t s, float* y2 = nullptr) {
   const int grid = grid_for(A.nw, kBlock / kWave, 1 << 18);
-  klaunch(k_csr4_tile<MODE, OFF16>, dim3(grid), dim3(kBlock), 0, s, A.nw, A.wrow, A.tag, A.ci4, A.co4, A.v4, x, b, aux,
-          w, y, y2);
+  klaunch(k_csr4_tile<float, MODE, OFF16>, dim3(grid), dim3(kBlock), 0, s, A.nw, A.wrow, A.tag, A.ci4, A.co4,
+          reinterpret_cast<const float*>(A.v4), x, b, aux, w, y, y2);
+}
+
+// the same pattern with FP64 values v8
+template <int MODE>
+void csr4_tile_f64(const Csr4F32& A, const double* v8, const double* x, const double* b, const double* aux, double w,
+                   double* y, hipStream_t s, double* y2 = nullptr) {
+  if (A.n <= 0) return;
+  IMPES_REQUIRE(A.nw > 0 && ((uintptr_t)v8 & 15) == 0, "FP64 tiles: aligned values of a tiled pattern required");
+  const int grid = grid_for(A.nw, kBlock / kWave, 1 << 18);
+  if (A.co4)
+    klaunch(k_csr4_tile<double, MODE, true>, dim3(grid), dim3(kBlock), 0, s, A.nw, A.wrow, A.tag, A.ci4, A.co4, v8, x,
+            b, aux, w, y, y2);
+  else
+    klaunch(k_csr4_tile<double, MODE, false>, dim3(grid), dim3(kBlock), 0, s, A.nw, A.wrow, A.tag, A.ci4, A.co4, v8, x,
+            b, aux, w, y, y2);
+  IMPES_LAUNCH_CHECK();
 }
 
 template <int MODE, bool OFF16>
@@ -856,13 +910,45 @@ void launch_prolong_sweep4_f32(const Csr4F32& S, const float* e, const float* r,
   csr4_tile_launch<kProlongJac, false>(S, e, r, inv_relax, w, x, s, x0);
   IMPES_LAUNCH_CHECK();
 }
+void launch_tile4_values_f64(const Csr4F32& A, const int* rp, const double* v, double* v8, hipStream_t s) {
+  if (A.nw <= 0) return;
+  k_tile4_values_f64<<<grid_for(A.nw, kBlock / kWave, 1 << 18), kBlock, 0, s>>>(A.nw, A.wrow, A.tag, A.rp4, rp, v,
+                                                                               reinterpret_cast<double2*>(v8));
+  IMPES_LAUNCH_CHECK();
+}
+void launch_residual4_f64(const Csr4F32& A, const double* v8, const double* x, const double* b, double* r,
+                          hipStream_t s) {
+  KScope ks("csr_residual_f64", csr_bytes(A.n, A.nnz, 8, 2), s);
+  csr4_tile_f64<kRes>(A, v8, x, b, nullptr, 0.0, r, s);
+}
+void launch_jacobi4_f64(const Csr4F32& A, const double* v8, const double* xi, const double* b, const double* inv_relax,
+                        double w, double* xo, hipStream_t s) {
+  KScope ks("csr_jacobi_f64", csr_bytes(A.n, A.nnz, 8, 3), s);
+  csr4_tile_f64<kJac>(A, v8, xi, b, inv_relax, w, xo, s);
+}
+void launch_spmv4_f64(const Csr4F32& A, const double* v8, const double* x, double* y, hipStream_t s) {
+  csr4_tile_f64<kY>(A, v8, x, nullptr, nullptr, 0.0, y, s);
+}
+void launch_restrict4_j0_f64(const Csr4F32& R, const double* v8, const double* r, const double* inv_relax_c, double w,
+                             double* bc, double* xc, hipStream_t s) {
+  csr4_tile_f64<kRestrictJ0>(R, v8, r, nullptr, inv_relax_c, w, bc, s, xc);
+}
+void launch_prolong_sweep4_f64(const Csr4F32& S, const double* v8, const double* e, const double* r,
+                               const double* inv_relax, double w, double* x0, double* x, hipStream_t s) {
+  csr4_tile_f64<kProlongJac>(S, v8, e, r, inv_relax, w, x, s, x0);
+}
 void launch_tile4_prolong_sweep(int nw, const int* wrow, const unsigned short* tag, const int* rp4, const int* ci4,
                                 const int* aprp, const double* apv, const int* prp, const int* pci, const double* pv, const double* ir,
-                                double w, float* v4, int* miss, hipStream_t s) {
+                                double w, float* v4, double* v8, int* miss, hipStream_t s) {
   if (nw <= 0) return;
+  if (v8) {
+    k_tile4_prolong_sweep<<<grid_for(nw, kBlock / kWave, 1 << 18), kBlock, 0, s>>>(
+        nw, wrow, tag, rp4, reinterpret_cast<const int4*>(ci4), aprp, apv, prp, pci, pv, ir, w, v8, miss);
+    IMPES_LAUNCH_CHECK();
+    return;
+  }
   k_tile4_prolong_sweep<<<grid_for(nw, kBlock / kWave, 1 << 18), kBlock, 0, s>>>(
-      nw, wrow, tag, rp4, reinterpret_cast<const int4*>(ci4), aprp, apv, prp, pci, pv, ir, w, reinterpret_cast<float4*>(v4),
-      miss);
+      nw, wrow, tag, rp4, reinterpret_cast<const int4*>(ci4), aprp, apv, prp, pci, pv, ir, w, v4, miss);
   IMPES_LAUNCH_CHECK();
 }
 void launch_restrict_j0_f64(const CsrF64& R, const double* r, const double* inv_relax_c, double w, double* bc,

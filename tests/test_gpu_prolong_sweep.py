@@ -1,10 +1,11 @@
-"""Prolongation and first post-sweep as one pass (FP32 cycle) against the FP64 cycle, which
-makes two: every smoothing count that reaches it, odd and even, stencil and CSR finest
+"""Prolongation and first post-sweep as one pass and the FP64 preconditioner's tiled
+passes against the FP64 cycle, which has neither: every smoothing count that reaches it, odd and even, stencil and CSR finest
 levels, levels above and inside the tail, at setup and after an update, replayed from the
 captured graph; and the operators that keep the two passes: a row too long for a tile, a
 row without a diagonal entry.
 
-Bound: the bar of the FP32 cycle comparisons, a few hundred roundings deep."""
+FP64: rounding of sums of up to some hundred terms. FP32: the cycle's own rounding, a few
+hundred operations deep."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -66,4 +67,8 @@ def test_fp32_cycle_matches_fp64(dev, name):
             y = h.vcycle(b, precision=64).cpu().numpy()
             assert rel(h.vcycle(b, precision=32).cpu().numpy(), y) < 2e-5
             z = h.precondition(b, precision=64).cpu().numpy()
+            if kind != "no_diagonal":  # the tiled FP64 cycle against the untiled one
+                dh = h.dhalf_inv()
+                d = torch.tensor(A.diagonal(), device=dev)
+                assert rel(z, (dh * h.vcycle(dh * d * b, precision=64)).cpu().numpy()) < 1e-12
             assert rel(h.precondition(b, precision=32).cpu().numpy(), z) < 2e-5
