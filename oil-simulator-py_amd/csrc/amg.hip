@@ -27,6 +27,14 @@ void d2d(T* dst, const T* src, size_t n, hipStream_t s) {
   if (n) IMPES_HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyDeviceToDevice, s));
 }
 
+// Work recorded into a caller's graph has not run: what it prepares does not count as
+// prepared for calls outside that graph.
+bool recording(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  IMPES_HIP_CHECK(hipStreamIsCapturing(s, &st));
+  return st != hipStreamCaptureStatusNone;
+}
+
 // ---------------------------------------------------------------- stencil kernels
 __global__ void k_st7_count(int nx, int ny, int nz, int* __restrict__ cnt) {
   const long long n = (long long)nx * ny * nz;
@@ -940,7 +948,7 @@ void Hierarchy::build_prolong_sweeps(hipStream_t s) {
 void Hierarchy::ensure_sweeps32(hipStream_t s) {
   if (sweeps32_ready_) return;
   for (auto& L : levels_) fill_prolong_sweep(L, nullptr, s);
-  sweeps32_ready_ = true;
+  sweeps32_ready_ = !recording(s);
 }
 
 void Hierarchy::fill_prolong_sweep(Level& L, int* miss, hipStream_t s) {
@@ -970,7 +978,7 @@ void Hierarchy::ensure_tiles64(hipStream_t s) {
                                  L.prp.p, L.pci.p, L.pv.p, L.ir64.p, prm_.omega, nullptr, L.s4.v8.p, nullptr, s);
     }
   }
-  tiles64_ready_ = true;
+  tiles64_ready_ = !recording(s);
 }
 
 // ---------------------------------------------------------------- coarse tail
@@ -1058,7 +1066,7 @@ void Hierarchy::ensure_tail(int precision, hipStream_t s) {
   A.ld = tail_ld_;
   A.B = precision == 32 ? (void*)tail_b32_.p : (void*)tail_b64_.p;
   launch_tail_form(precision, A, s);
-  tail_ready_[gi] = true;
+  tail_ready_[gi] = !recording(s);
 }
 
 // ---------------------------------------------------------------- V-cycle
