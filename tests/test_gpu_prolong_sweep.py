@@ -72,3 +72,34 @@ def test_fp32_cycle_matches_fp64(dev, name):
                 d = torch.tensor(A.diagonal(), device=dev)
                 assert rel(z, (dh * h.vcycle(dh * d * b, precision=64)).cpu().numpy()) < 1e-12
             assert rel(h.precondition(b, precision=32).cpu().numpy(), z) < 2e-5
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("dims", [(12, 10, 10), (30, 24, 10)])  # the tail from level 0 on, levels above it
+def test_recorded_preparations_are_not_done(dev, dims, precision):
+    """A cycle recorded into a caller's graph after an update prepares its matrices when
+    the graph runs; an eager cycle before that prepares its own."""
+    import impes_hip as H
+
+    first, second = (to_dev(impes_like(*dims, seed=8, sigma=s)[0], dev) for s in (1.0, 1.3))
+    fresh, h = H.AmgHierarchy(), H.AmgHierarchy()
+    fresh.setup_csr(*first)
+    fresh.update_csr(second[2])
+    h.setup_csr(*first)
+    h.set_graphs(False)
+    v = torch.tensor(np.random.default_rng(0).standard_normal(first[0].numel() - 1), device=dev)
+    z = torch.empty_like(v)
+    h.precondition(v, precision=precision, out=z)
+    h.update_csr(second[2])
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        h.precondition(v, precision=precision, out=z)
+    ref = fresh.precondition(v, precision=precision)
+    assert torch.equal(h.precondition(v, precision=precision), ref)
+    for _ in range(3):
+        z.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, ref)
+        assert torch.equal(h.precondition(v, precision=precision), ref)
