@@ -72,7 +72,7 @@ struct Pad4 {
   DevBuf<int> rp4, ci4, wrow;
   DevBuf<unsigned short> tag;
   DevBuf<float> v4;
-  DevBuf<double> v8;  // FP64 values (Hierarchy::ensure_tiles64)
+  double* v8 = nullptr;  // FP64 values (in Hierarchy::tiles64_)
 };
 
 struct Level {
@@ -94,7 +94,7 @@ struct Level {
   DevBuf<int> wrow4;
   DevBuf<unsigned short> tag4;
   DevBuf<float> v4;
-  DevBuf<double> v8;         // FP64 values of the tiles (ensure_tiles64)
+  double* v8 = nullptr;      // FP64 values of the tiles (in Hierarchy::tiles64_)
   DevBuf<signed char> cf;  // final C/F markers (non-coarsest levels)
   // interpolation / restriction to the next level
   int nc = 0, pnnz = 0, pgroup = 1, rgroup = 1;
@@ -232,6 +232,7 @@ class Hierarchy {
   void build_prolong_sweeps(hipStream_t s);
   void ensure_sweeps32(hipStream_t s);
   void ensure_tiles64(hipStream_t s);
+  void alloc_derived();  // memory of what cycles prepare on first use
   void fill_prolong_sweep(Level& L, int* miss, hipStream_t s);  // values, after every numeric change
   void ensure_tail(int precision, hipStream_t s);
   template <class T>
@@ -273,6 +274,8 @@ class Hierarchy {
   DevBuf<unsigned char> tail_ell_[2];
   DevBuf<float> tail_b32_;
   DevBuf<double> tail_b64_;
+  DevBuf<double> tiles64_;           // FP64 values of all the levels' tiles
+  bool transfers64_ready_ = false;   // those of the restrictions, fixed until the next setup
 
   AmgParams prm_;
   // device memory of builds: slab-carved small blocks, releases deferred to the

@@ -225,11 +225,11 @@ struct Sel<double> {
     return Csr4F32{T.n, T.nnz, T.rp4.p, reinterpret_cast<const int4*>(T.ci4.p), nullptr, nullptr, T.nw, T.wrow.p, T.tag.p};
   }
   static void jacL(const Level& L, const double* xi, const double* b, double w, double* xo, hipStream_t s, bool tiles) {
-    if (tiles && L.v8.p) launch_jacobi4_f64(A4(L), L.v8.p, xi, b, L.ir64.p, w, xo, s);
+    if (tiles && L.v8) launch_jacobi4_f64(A4(L), L.v8, xi, b, L.ir64.p, w, xo, s);
     else launch_jacobi_f64(A(L), xi, b, L.ir64.p, w, xo, L.group, s);
   }
   static void resL(const Level& L, const double* x, const double* b, double* r, hipStream_t s, bool tiles) {
-    if (tiles && L.v8.p) launch_residual4_f64(A4(L), L.v8.p, x, b, r, s);
+    if (tiles && L.v8) launch_residual4_f64(A4(L), L.v8, x, b, r, s);
     else launch_residual_f64(A(L), x, b, r, L.group, s);
   }
   static void res(const CsrF64& A, const double* x, const double* b, double* r, int g, hipStream_t s) {
@@ -249,17 +249,17 @@ struct Sel<double> {
   // grid transfers of level L (P: n x nc, R: nc x n)
   static void restrict_j0(const Level& L, const double* r, const double* irc, double w, double* bc, double* xc,
                           hipStream_t s, bool tiles) {
-    if (tiles && L.r4.v8.p) launch_restrict4_j0_f64(T4(L.r4), L.r4.v8.p, r, irc, w, bc, xc, s);
+    if (tiles && L.r4.v8) launch_restrict4_j0_f64(T4(L.r4), L.r4.v8, r, irc, w, bc, xc, s);
     else launch_restrict_j0_f64(R(L), r, irc, w, bc, xc, L.rgroup, s);
   }
   static void restrict_to(const Level& L, const double* r, double* bc, hipStream_t s, bool tiles) {
-    if (tiles && L.r4.v8.p) launch_spmv4_f64(T4(L.r4), L.r4.v8.p, r, bc, s);
+    if (tiles && L.r4.v8) launch_spmv4_f64(T4(L.r4), L.r4.v8, r, bc, s);
     else launch_spmv_f64(R(L), r, bc, L.rgroup, s);
   }
   static bool prolong_sweep(const Level& L, const double* e, const double* r, double w, double* x0, double* x,
                             hipStream_t s, bool tiles) {
-    if (!tiles || !L.s4.v8.p) return false;
-    launch_prolong_sweep4_f64(T4(L.s4), L.s4.v8.p, e, r, L.ir64.p, w, x0, x, s);
+    if (!tiles || !L.s4.v8) return false;
+    launch_prolong_sweep4_f64(T4(L.s4), L.s4.v8, e, r, L.ir64.p, w, x0, x, s);
     return true;
   }
   static void prolong(const Level& L, const double* e, double* y, hipStream_t s) {
@@ -459,6 +459,7 @@ void Hierarchy::setup_impl(int n, int nnz, const int* rp, const int* ci, const d
   alloc_vectors();
   choose_tail(s);
   build_prolong_sweeps(s);
+  alloc_derived();
   IMPES_HIP_CHECK(hipStreamSynchronize(s));
   }
   last_setup_seconds = wall() - t0;
@@ -964,21 +965,44 @@ void Hierarchy::ensure_tiles64(hipStream_t s) {
   for (int l = 0; l < end; ++l) {
     Level& L = levels_[l];
     if (L.coarsest) break;
-    if (L.pad4 && L.nw4 > 0) {
-      L.v8.alloc(4 * (size_t)L.nw4 * kWave);
-      launch_tile4_values_f64(Sel<double>::A4(L), L.rp.p, L.v.p, L.v8.p, s);
-    }
-    if (L.r4.nw && !L.r4.v8.p) {  // fixed until the next setup
-      L.r4.v8.alloc(4 * (size_t)L.r4.nw * kWave);
-      launch_tile4_values_f64(Sel<double>::T4(L.r4), L.rrp.p, L.rv.p, L.r4.v8.p, s);
-    }
-    if (L.s4.nw) {
-      L.s4.v8.alloc(4 * (size_t)L.s4.nw * kWave);
+    if (L.v8) launch_tile4_values_f64(Sel<double>::A4(L), L.rp.p, L.v.p, L.v8, s);
+    if (L.r4.v8 && !transfers64_ready_) launch_tile4_values_f64(Sel<double>::T4(L.r4), L.rrp.p, L.rv.p, L.r4.v8, s);
+    if (L.s4.v8) {
       launch_tile4_prolong_sweep(L.s4.nw, L.s4.wrow.p, L.s4.tag.p, L.s4.rp4.p, L.s4.ci4.p, L.aprp.p, L.apv.p,
-                                 L.prp.p, L.pci.p, L.pv.p, L.ir64.p, prm_.omega, nullptr, L.s4.v8.p, nullptr, s);
+                                 L.prp.p, L.pci.p, L.pv.p, L.ir64.p, prm_.omega, nullptr, L.s4.v8, nullptr, s);
     }
   }
-  tiles64_ready_ = !recording(s);
+  tiles64_ready_ = transfers64_ready_ = !recording(s);
+}
+
+// Whatever a cycle prepares on its first use has its memory from the setup on (out of
+// the setup's pool): a cycle allocates nothing, so that its first run can be recorded
+// into a caller's graph. One block holds the FP64 tiles of all levels.
+void Hierarchy::alloc_derived() {
+  const int end = tail_ >= 0 ? tail_ : (int)levels_.size() - 1;
+  auto each = [&](auto&& f) {
+    for (int l = 0; l < end; ++l) {
+      Level& L = levels_[l];
+      if (L.coarsest) break;
+      if (L.pad4) f(L.v8, L.nw4);
+      f(L.r4.v8, L.r4.nw);
+      f(L.s4.v8, L.s4.nw);
+    }
+  };
+  size_t total = 0;
+  each([&](double*&, int nw) { total += 4 * (size_t)nw * kWave; });
+  tiles64_.alloc(total);
+  size_t at = 0;
+  each([&](double*& v8, int nw) {
+    v8 = nw > 0 ? tiles64_.p + at : nullptr;
+    at += 4 * (size_t)nw * kWave;
+  });
+  transfers64_ready_ = false;
+  if (tail_ < 0) return;
+  for (int gi = 0; gi < 2; ++gi) tail_ell_[gi].alloc(tail_ell_bytes(1, gi ? 64 : 32) * tail_line_.back());
+  const size_t nb = (size_t)levels_[tail_].n * tail_ld_;
+  tail_b32_.alloc(nb);
+  tail_b64_.alloc(nb);
 }
 
 // ---------------------------------------------------------------- coarse tail
@@ -1035,10 +1059,6 @@ void Hierarchy::ensure_tail(int precision, hipStream_t s) {
   if (tail_ < 0 || tail_ready_[gi]) return;
   const int last = (int)levels_.size() - 1;
   const size_t line = tail_ell_bytes(1, precision);
-  tail_ell_[gi].alloc(line * tail_line_.back());
-  const size_t nb = (size_t)levels_[tail_].n * tail_ld_;
-  if (precision == 32) tail_b32_.alloc(nb);
-  else tail_b64_.alloc(nb);
   TailArgs A;
   A.levels = last - tail_;
   for (int q = tail_; q <= last; ++q) {
