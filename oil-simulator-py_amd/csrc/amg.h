@@ -224,17 +224,17 @@ class Hierarchy {
   void refresh_stencil(hipStream_t s);
   void alloc_vectors();
   // first_sweep_done: x already holds the first pre-smoothing sweep from zero
-  // tail: levels from tail_ down as one matrix (ensure_tail has run)
+  // tail: the preconditioner's cycle, with levels from tail_ down as one matrix and the
+  // FP64 tiles. Whatever it reads beside the levels has been prepared.
   template <class T>
   void vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done = false,
                     bool tail = false);
   void choose_tail(hipStream_t s);
   void build_prolong_sweeps(hipStream_t s);
-  void ensure_sweeps32(hipStream_t s);
-  void ensure_tiles64(hipStream_t s);
-  void alloc_derived();  // memory of what cycles prepare on first use
+  void alloc_derived();
   void fill_prolong_sweep(Level& L, int* miss, hipStream_t s);  // values, after every numeric change
-  void ensure_tail(int precision, hipStream_t s);
+  void form_tail(int precision, hipStream_t s);
+  void form_tiles64(hipStream_t s);
   template <class T>
   void smooth(int l, const T* b, T*& cur, T* other, int sweeps, bool& zero, hipStream_t s, bool tiles = false);
   template <class T>
@@ -260,14 +260,29 @@ class Hierarchy {
   bool transposed_ = false;  // eager cycles of vcycle64/32 with nu1 and nu2 swapped
   hipGraphExec_t vexec_[2] = {nullptr, nullptr};  // [0] FP32, [1] FP64 V-cycle
 
-  // The preconditioner's cycle from level tail_ down as one matrix (tail.hip; -1:
-  // none), per precision ([0] FP32, [1] FP64): formed at the first cycle after a
-  // setup or update, which clear tail_ready_.
-  int tail_ = -1;
-  bool tail_ready_[2] = {false, false};
+  // What cycles read beside the levels, formed from them when a cycle first needs it
+  // after a setup or a numeric update: the matrix of the coarse end, the fused sweeps'
+  // FP32 values, the FP64 tiles of the operators and of the restrictions (these are
+  // fixed until the next setup). Work recorded into a caller's graph runs when the graph
+  // does, before or after any eager call, so:
+  //  - a recorded cycle that finds a form current relies on it, and from then on updates
+  //    bring the form up to date themselves; one that does not records the forming;
+  //  - a recorded update brings up to date what has been formed so far, and what has not
+  //    is formed anew by every cycle until the next setup.
+  enum Form { kTail32, kTail64, kSweeps32, kTiles64, kTransfers64, kForms };
+  struct Derived {
+    bool current = false;     // that of the operators, once the eager work has run
+    bool formed = false;      // since the setup
+    bool relied_on = false;   // by a recorded cycle
+    bool distrusted = false;  // a recorded update leaves it behind
+  };
+  Derived forms_[kForms];
+  void form(Form f, hipStream_t s);
+  void ensure(Form f, bool rec, hipStream_t s);
+  void prepare(int precision, bool tail, hipStream_t s);  // all that a cycle reads
+
+  int tail_ = -1;  // first level of the coarse end's matrix (tail.hip), -1: none
   int tail_ld_ = 0;
-  bool sweeps32_ready_ = false;  // the fused sweeps' FP32 values are those of the operators
-  bool tiles64_ready_ = false;  // the levels' FP64 tile values are those of the operators
   std::vector<long long> tail_at_;   // per level from tail_: first slice offset in tail_so_
   std::vector<long long> tail_line_; // per level from tail_: first line in tail_ell_ (last: the total)
   DevBuf<int> tail_so_;
@@ -275,7 +290,6 @@ class Hierarchy {
   DevBuf<float> tail_b32_;
   DevBuf<double> tail_b64_;
   DevBuf<double> tiles64_;           // FP64 values of all the levels' tiles
-  bool transfers64_ready_ = false;   // those of the restrictions, fixed until the next setup
 
   AmgParams prm_;
   // device memory of builds: slab-carved small blocks, releases deferred to the

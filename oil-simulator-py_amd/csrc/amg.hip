@@ -27,9 +27,9 @@ void d2d(T* dst, const T* src, size_t n, hipStream_t s) {
   if (n) IMPES_HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyDeviceToDevice, s));
 }
 
-// Work recorded into a caller's graph has not run: what it prepares does not count as
-// prepared for calls outside that graph.
+// Whether work on s is recorded into a caller's graph (the null stream's never is)
 bool recording(hipStream_t s) {
+  if (!s) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   IMPES_HIP_CHECK(hipStreamIsCapturing(s, &st));
   return st != hipStreamCaptureStatusNone;
@@ -440,6 +440,7 @@ void Hierarchy::setup_impl(int n, int nnz, const int* rp, const int* ci, const d
   // with hipFree, which waits for the device)
   PoolScope scope(pool_);
   drop_graphs();  // the level buffers are about to be rebuilt
+  for (Derived& d : forms_) d = Derived{};
   levels_.clear();
   levels_.emplace_back();
   Level& L0 = levels_[0];
@@ -850,8 +851,6 @@ void Hierarchy::update_csr_values(const double* v, hipStream_t s) {
 }
 
 void Hierarchy::update_levels(bool fine_done, hipStream_t s) {
-  tail_ready_[0] = tail_ready_[1] = false;
-  tiles64_ready_ = false;
   for (int l = 0; l + 1 < (int)levels_.size(); ++l) {
     Level& A = levels_[l];
     if (A.coarsest) break;
@@ -878,8 +877,14 @@ void Hierarchy::update_levels(bool fine_done, hipStream_t s) {
       else launch_pin_decide(L.n, L.rp.p, L.ci.p, L.v.p, L.pin_mode, L.pin.p, L.gj_bad.p, s);
     }
   }
-  sweeps32_ready_ = false;
   if (stencil_ && !fine_done) refresh_stencil(s);
+  const bool rec = recording(s);
+  for (Form f : {kTail32, kTail64, kSweeps32, kTiles64}) {
+    Derived& d = forms_[f];
+    if (rec && !d.formed) d.distrusted = true;
+    if (rec ? d.formed : d.relied_on) form(f, s);
+    if (!rec) d.current = d.relied_on;
+  }
 }
 
 void Hierarchy::update_stencil(const double* d, const double* ox, const double* oy, const double* oz, hipStream_t s) {
@@ -942,14 +947,7 @@ void Hierarchy::build_prolong_sweeps(hipStream_t s) {
   // a matrix with a row without a diagonal entry keeps the two passes
   if (read_scalar(miss.p, s) != 0)
     for (auto& L : levels_) L.s4 = Pad4{};
-  sweeps32_ready_ = true;
-}
-
-// the FP32 values, when a cycle first needs them after a numeric update
-void Hierarchy::ensure_sweeps32(hipStream_t s) {
-  if (sweeps32_ready_) return;
-  for (auto& L : levels_) fill_prolong_sweep(L, nullptr, s);
-  sweeps32_ready_ = !recording(s);
+  forms_[kSweeps32].current = forms_[kSweeps32].formed = true;
 }
 
 void Hierarchy::fill_prolong_sweep(Level& L, int* miss, hipStream_t s) {
@@ -957,27 +955,20 @@ void Hierarchy::fill_prolong_sweep(Level& L, int* miss, hipStream_t s) {
                              L.pv.p, L.ir64.p, prm_.omega, L.s4.v4.p, nullptr, miss, s);
 }
 
-// FP64 values of the tiles above the tail, when the FP64 preconditioner first needs them
-// after a numeric change (262,000 cells: 65 us a refresh, against about 30 us saved per cycle)
-void Hierarchy::ensure_tiles64(hipStream_t s) {
-  if (tiles64_ready_) return;
-  const int end = tail_ >= 0 ? tail_ : (int)levels_.size() - 1;
-  for (int l = 0; l < end; ++l) {
-    Level& L = levels_[l];
-    if (L.coarsest) break;
+// FP64 values of the tiles above the tail (262,000 cells: 65 us a refresh, against about
+// 30 us saved per cycle)
+void Hierarchy::form_tiles64(hipStream_t s) {
+  for (auto& L : levels_) {
     if (L.v8) launch_tile4_values_f64(Sel<double>::A4(L), L.rp.p, L.v.p, L.v8, s);
-    if (L.r4.v8 && !transfers64_ready_) launch_tile4_values_f64(Sel<double>::T4(L.r4), L.rrp.p, L.rv.p, L.r4.v8, s);
-    if (L.s4.v8) {
+    if (L.s4.v8)
       launch_tile4_prolong_sweep(L.s4.nw, L.s4.wrow.p, L.s4.tag.p, L.s4.rp4.p, L.s4.ci4.p, L.aprp.p, L.apv.p,
                                  L.prp.p, L.pci.p, L.pv.p, L.ir64.p, prm_.omega, nullptr, L.s4.v8, nullptr, s);
-    }
   }
-  tiles64_ready_ = transfers64_ready_ = !recording(s);
 }
 
-// Whatever a cycle prepares on its first use has its memory from the setup on (out of
-// the setup's pool): a cycle allocates nothing, so that its first run can be recorded
-// into a caller's graph. One block holds the FP64 tiles of all levels.
+// Whatever cycles form from the levels has its memory from the setup on (out of the
+// setup's pool): a cycle allocates nothing, so that its first run can be recorded into a
+// caller's graph. One block holds the FP64 tiles of all levels.
 void Hierarchy::alloc_derived() {
   const int end = tail_ >= 0 ? tail_ : (int)levels_.size() - 1;
   auto each = [&](auto&& f) {
@@ -997,12 +988,47 @@ void Hierarchy::alloc_derived() {
     v8 = nw > 0 ? tiles64_.p + at : nullptr;
     at += 4 * (size_t)nw * kWave;
   });
-  transfers64_ready_ = false;
   if (tail_ < 0) return;
   for (int gi = 0; gi < 2; ++gi) tail_ell_[gi].alloc(tail_ell_bytes(1, gi ? 64 : 32) * tail_line_.back());
   const size_t nb = (size_t)levels_[tail_].n * tail_ld_;
   tail_b32_.alloc(nb);
   tail_b64_.alloc(nb);
+}
+
+void Hierarchy::form(Form f, hipStream_t s) {
+  switch (f) {
+    case kTail32: form_tail(32, s); break;
+    case kTail64: form_tail(64, s); break;
+    case kSweeps32:
+      for (auto& L : levels_) fill_prolong_sweep(L, nullptr, s);
+      break;
+    case kTiles64: form_tiles64(s); break;
+    default:
+      for (auto& L : levels_)
+        if (L.r4.v8) launch_tile4_values_f64(Sel<double>::T4(L.r4), L.rrp.p, L.rv.p, L.r4.v8, s);
+  }
+}
+
+void Hierarchy::ensure(Form f, bool rec, hipStream_t s) {
+  Derived& d = forms_[f];
+  if (d.current && !d.distrusted) {
+    d.relied_on = d.relied_on || rec;
+    return;
+  }
+  form(f, s);
+  d.formed = true;
+  if (!rec) d.current = true;
+}
+
+void Hierarchy::prepare(int precision, bool tail, hipStream_t s) {
+  const bool rec = recording(s);
+  if (tail && tail_ >= 0) ensure(precision == 32 ? kTail32 : kTail64, rec, s);
+  if (precision == 32) {
+    ensure(kSweeps32, rec, s);
+  } else if (tail) {
+    ensure(kTransfers64, rec, s);
+    ensure(kTiles64, rec, s);
+  }
 }
 
 // ---------------------------------------------------------------- coarse tail
@@ -1014,8 +1040,6 @@ void Hierarchy::alloc_derived() {
 // at 2,046 rows and 91,000 entries and 360 us above a 518-row coarsest level.
 void Hierarchy::choose_tail(hipStream_t s) {
   tail_ = -1;
-  tail_ready_[0] = tail_ready_[1] = false;
-  tiles64_ready_ = false;
   tail_at_.clear();
   tail_line_.clear();
   const int last = (int)levels_.size() - 1;
@@ -1054,9 +1078,9 @@ void Hierarchy::choose_tail(hipStream_t s) {
   }
 }
 
-void Hierarchy::ensure_tail(int precision, hipStream_t s) {
+void Hierarchy::form_tail(int precision, hipStream_t s) {
+  if (tail_ < 0) return;
   const int gi = precision == 32 ? 0 : 1;
-  if (tail_ < 0 || tail_ready_[gi]) return;
   const int last = (int)levels_.size() - 1;
   const size_t line = tail_ell_bytes(1, precision);
   TailArgs A;
@@ -1086,7 +1110,6 @@ void Hierarchy::ensure_tail(int precision, hipStream_t s) {
   A.ld = tail_ld_;
   A.B = precision == 32 ? (void*)tail_b32_.p : (void*)tail_b64_.p;
   launch_tail_form(precision, A, s);
-  tail_ready_[gi] = !recording(s);
 }
 
 // ---------------------------------------------------------------- V-cycle
@@ -1217,6 +1240,7 @@ void Hierarchy::level_times(int precision, int cycles, double* ms, double* cycle
     }
   } done{this, c};
   Level& L0 = levels_[0];
+  prepare(precision, false, s);
   IMPES_HIP_CHECK(hipStreamSynchronize(s));
   clock_ = &c;
   for (int i = 0; i < cycles; ++i) {
@@ -1251,12 +1275,9 @@ void Hierarchy::level_times(int precision, int cycles, double* ms, double* cycle
   }
 }
 
-// tail: the preconditioner's cycle, which may use the tail matrix and the FP64 tiles
-// (ensure_tail and ensure_tiles64 come before it)
 template <class T>
 void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done, bool tail) {
   Level& L = levels_[l];
-  if (sizeof(T) == 4 && l == 0) ensure_sweeps32(s);  // done before a capture
   if (tail && l == tail_) {
     if constexpr (sizeof(T) == 8) launch_tail_mv_f64(L.n, tail_ld_, tail_b64_.p, b, x, s);
     else launch_tail_mv_f32(L.n, tail_ld_, tail_b32_.p, b, x, s);
@@ -1346,6 +1367,7 @@ void Hierarchy::vcycle64(const double* b, double* x, bool x_zero, hipStream_t s)
 void Hierarchy::vcycle32(const float* b, float* x, bool x_zero, hipStream_t s) {
   IMPES_REQUIRE(!levels_.empty(), "vcycle before setup");
   SmoothSwap sw(prm_, transposed_);
+  prepare(32, false, s);
   vcycle_level<float>(0, b, x, x_zero, s);
 }
 
@@ -1375,6 +1397,7 @@ int Hierarchy::cycles_impl(const CycleWork& w, int precision, const double* b, d
   Level& L0 = levels_[0];
   const long long n = L0.n;
   double hv[2];
+  prepare(precision, false, s);
   launch_scale_f64(w.b, dh_.p, b, n, s);  // bs = dh .* b
   if (use_x0) launch_div_f64(w.x, x, dh_.p, n, s);  // xs = x0 ./ dh
   launch_dot_f64(w.b, w.b, n, w.sc, w.part, s);
@@ -1429,9 +1452,7 @@ void Hierarchy::vcycle_only(int precision, hipStream_t s) {
   // a cycle that is one product needs no graph (its launch costs the host more)
   const bool replay = graphs_ && !ktimer_enabled() && tail_ != 0;
   const int gi = precision == 32 ? 0 : 1;
-  ensure_tail(precision, s);
-  if (precision == 64) ensure_tiles64(s);
-  else ensure_sweeps32(s);
+  prepare(precision, true, s);
   if (replay && !vexec_[gi]) capture_vcycle(precision);
   if (replay) IMPES_HIP_CHECK(hipGraphLaunch(vexec_[gi], s));
   else if (precision == 32) vcycle_level<float>(0, L0.b32.p, L0.x32.p, true, s, false, true);

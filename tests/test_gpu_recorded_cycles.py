@@ -82,19 +82,96 @@ kinds = pytest.mark.parametrize("kind", ["csr", "st7"])
 @params
 @grids
 @kinds
-def test_recorded_cycle_as_the_first_call(dev, dims, kind, precision):
-    """The first cycle after a setup goes into a graph: nothing is allocated in it."""
+def test_recorded_cycle_after_eager_updates(dev, dims, kind, precision):
+    """Warm up, record, update eagerly, replay."""
     op = Operators(dims, kind, dev)
-    refs = [op.reference(q, (precision,))[0] for q in range(1)]
+    refs = [op.reference(q, (precision,))[0] for q in range(3)]
+    h = op.setup()
+    z = h.precondition(op.v, precision=precision).clone()
+    g = record(lambda: h.precondition(op.v, precision=precision, out=z))
+    for q in (1, 2, 1):
+        op.load(q)
+        op.update(h)
+        z.zero_()
+        g.replay()
+        same([z], [refs[q]], f"replay after update {q}")
+        same([h.precondition(op.v, precision=precision)], [refs[q]], f"eager cycle after update {q}")
+
+
+@params
+@grids
+@kinds
+def test_recorded_update_with_eager_cycles(dev, dims, kind, precision):
+    """Record an update, run an eager cycle, replay the update with new values, run an
+    eager cycle; the update recorded with no cycle before it, after one of this
+    precision, and after one of the other."""
+    op = Operators(dims, kind, dev)
+    refs = [op.reference(q) for q in range(4)]
+    for warm in ((), (precision,), (96 - precision,)):
+        h = op.setup()
+        for p in warm:
+            op.results(h, (p,))
+        op.load(0)
+        g = record(lambda: op.update(h))
+        same(op.results(h), refs[0], f"warmed up {warm}: recorded, not run")
+        for q in (1, 2):
+            op.load(q)
+            g.replay()
+            same(op.results(h), refs[q], f"warmed up {warm}: replay {q}")
+        op.load(3)
+        op.update(h)
+        same(op.results(h), refs[3], f"warmed up {warm}: eager update")
+        op.load(1)
+        g.replay()
+        same(op.results(h), refs[1], f"warmed up {warm}: replay after it")
+
+
+@params
+@grids
+@kinds
+def test_recorded_cycle_as_the_first_call(dev, dims, kind, precision):
+    """The first cycle after a setup goes into a graph: nothing is allocated in it, and
+    it serves the operators of later updates."""
+    op = Operators(dims, kind, dev)
+    refs = [op.reference(q, (precision,))[0] for q in range(3)]
     h = op.setup()
     z = torch.empty_like(op.v)
     g = record(lambda: h.precondition(op.v, precision=precision, out=z))
     same([h.precondition(op.v, precision=precision)], [refs[0]], "eager cycle before the first replay")
-    for q in (0, 0):
+    for q in (0, 1, 2):
         if q:
             op.load(q)
             op.update(h)
         z.zero_()
         g.replay()
         same([z], [refs[q]], f"replay {q}")
+        same([h.precondition(op.v, precision=precision)], [refs[q]], f"eager cycle {q}")
+
+
+@params
+@grids
+@kinds
+def test_update_and_cycles_in_one_graph(dev, dims, kind, precision):
+    """An update with two cycles behind it, recorded after a warm-up, and a graph of
+    cycles alone beside it."""
+    op = Operators(dims, kind, dev)
+    refs = [op.reference(q, (precision,))[0] for q in range(3)]
+    h = op.setup()
+    z = [h.precondition(op.v, precision=precision).clone() for _ in range(3)]
+    op.load(0)
+
+    def body():
+        op.update(h)
+        for k in range(2):
+            h.precondition(op.v, precision=precision, out=z[k])
+
+    both = record(body)
+    alone = record(lambda: h.precondition(op.v, precision=precision, out=z[2]))
+    for q in (1, 2, 0, 1):
+        op.load(q)
+        for a in z:
+            a.zero_()
+        both.replay()
+        alone.replay()
+        same(z, [refs[q]] * 3, f"replay {q}")
         same([h.precondition(op.v, precision=precision)], [refs[q]], f"eager cycle {q}")
