@@ -989,7 +989,7 @@ void Hierarchy::alloc_derived() {
     at += 4 * (size_t)nw * kWave;
   });
   if (tail_ < 0) return;
-  for (int gi = 0; gi < 2; ++gi) tail_ell_[gi].alloc(tail_ell_bytes(1, gi ? 64 : 32) * tail_line_.back());
+  tail_ell_.alloc(tail_ell_bytes(tail_line_.back()));
   const size_t nb = (size_t)levels_[tail_].n * tail_ld_;
   tail_b32_.alloc(nb);
   tail_b64_.alloc(nb);
@@ -1035,9 +1035,9 @@ void Hierarchy::prepare(int precision, bool tail, hipStream_t s) {
 // The tail starts at the finest level that tail.hip's limits admit (both precisions),
 // down to a dense coarsest level. The limits: each cycle saves about 17 us per level
 // (six launches of ~3.2 us against one product of 4-6 us) and runs ten times and more
-// per update; forming costs 45-50 us at 1,200 rows and 8,600 entries below them, 107
-// us in FP64 at 1,343 rows and 16,700 entries (two rounds of workgroups), but 168 us
-// at 2,046 rows and 91,000 entries and 360 us above a 518-row coarsest level.
+// per update; forming costs 66-84 us at 1,072-1,343 rows, 136 us at 852 rows with 24
+// entries each, but it took 168 us at 2,046 rows and 91,000 entries and 360 us above a
+// 518-row coarsest level (with FP32 operations).
 void Hierarchy::choose_tail(hipStream_t s) {
   tail_ = -1;
   tail_at_.clear();
@@ -1051,12 +1051,12 @@ void Hierarchy::choose_tail(hipStream_t s) {
     TailArgs A;
     A.levels = last - l;
     for (int q = l; q <= last; ++q) A.lv[q - l].n = levels_[q].n;
-    if (tail_lds_layout(A, 32) > kTailLds || tail_lds_layout(A, 64) > kTailLds) continue;
+    if (!tail_fits(A)) continue;
     tail_ = l;
     break;
   }
   if (tail_ < 0) return;
-  tail_ld_ = (levels_[tail_].n + 7) / 8 * 8;
+  tail_ld_ = tail_ld(levels_[tail_].n);
   // slice offsets of every level but the coarsest
   int slots = 0;
   for (int q = tail_; q < last; ++q) {
@@ -1080,9 +1080,7 @@ void Hierarchy::choose_tail(hipStream_t s) {
 
 void Hierarchy::form_tail(int precision, hipStream_t s) {
   if (tail_ < 0) return;
-  const int gi = precision == 32 ? 0 : 1;
   const int last = (int)levels_.size() - 1;
-  const size_t line = tail_ell_bytes(1, precision);
   TailArgs A;
   A.levels = last - tail_;
   for (int q = tail_; q <= last; ++q) {
@@ -1091,8 +1089,8 @@ void Hierarchy::form_tail(int precision, hipStream_t s) {
     t.n = L.n;
     if (q == last) break;
     t.so = (int)tail_at_[q - tail_];
-    unsigned char* ell = tail_ell_[gi].p + line * tail_line_[q - tail_];
-    launch_tail_pack(precision, L.n, L.rp.p, L.ci.p, L.v.p, tail_so_.p + t.so, ell, s);
+    unsigned char* ell = tail_ell_.p + tail_ell_bytes(tail_line_[q - tail_]);
+    launch_tail_pack(L.n, L.rp.p, L.ci.p, L.v.p, tail_so_.p + t.so, ell, s);
     t.ell = ell;
     t.ir = L.ir64.p;
     t.prp = L.prp.p; t.pci = L.pci.p; t.pv = L.pv.p;

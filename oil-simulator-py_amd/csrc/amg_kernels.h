@@ -147,16 +147,15 @@ struct TailArgs {
   int pre = 0, post = 0;
   double omega = 0.0;
   int part = 0, splits = 0;  // LDS offset and count of the coarsest solve's partial sums
-  int ld = 0;         // row stride of B, a multiple of 8
-  void* B = nullptr;  // float (precision 32) or double
+  int ld = 0;         // row stride of B (tail_ld)
+  void* B = nullptr;  // float (precision 32) or double; formed in FP64
 };
 int tail_slices(int n);
 void launch_tail_slices(int n, const int* rp, int* so, hipStream_t s);  // tail_slices(n) + 1 offsets
-size_t tail_ell_bytes(long long lines, int precision);
-void launch_tail_pack(int precision, int n, const int* rp, const int* ci, const double* v, const int* so, void* ell,
-                      hipStream_t s);
-// assigns the LDS offsets; bytes of LDS (above kTailLds: does not fit)
-size_t tail_lds_layout(TailArgs& A, int precision);
+size_t tail_ell_bytes(long long lines);
+void launch_tail_pack(int n, const int* rp, const int* ci, const double* v, const int* so, void* ell, hipStream_t s);
+bool tail_fits(const TailArgs& A);  // from the levels' sizes
+constexpr int tail_ld(int n) { return (n + 12) / 8 * 8; }  // row stride of B: n and the last workgroup's padding
 void launch_tail_form(int precision, TailArgs A, hipStream_t s);
 void launch_tail_mv_f32(int n, int ld, const float* B, const float* b, float* x, hipStream_t s);
 void launch_tail_mv_f64(int n, int ld, const double* B, const double* b, double* x, hipStream_t s);

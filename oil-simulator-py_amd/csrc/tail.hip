@@ -13,6 +13,13 @@
 // are read in sliced form (64 rows per slice, entry k of a slice's rows side by side),
 // a row per lane: each load is one contiguous 64-entry line, and the M values of the
 // gathered row are one or two 16-byte LDS reads.
+//
+// B is formed in FP64 for both cycles and rounded once for the FP32 one. An FP32 cycle
+// level by level applies the coarsest inverse in FP64, so a B of FP32 operations would
+// hold fewer bits than what it replaces: over 48 operators of 400-1,600 rows its error
+// against the FP64 cycle was 1.05 times the level-by-level FP32 cycle's in the mean and
+// up to 4.3 times; rounded once it is 0.55 times (the rest is the rounding of b). The
+// FP64 operations cost 72 us against 50 at 1,200 rows, once per update.
 #include <algorithm>
 #include <vector>
 
@@ -25,9 +32,8 @@ namespace {
 
 constexpr int kTailThreads = 1024;
 
-template <class T>
 struct EllEntry {
-  T v;
+  double v;
   int c;
 };
 
@@ -55,21 +61,19 @@ __global__ __launch_bounds__(kTailThreads) void k_tail_slices(int n, const int* 
   if (lane == ns - 1) so[ns] = sum;
 }
 
-// The sliced operator in the cycle's precision: padding entries have value 0 and
-// their own row as column.
-template <class T>
+// The sliced operator: padding entries have value 0 and their own row as column.
 __global__ __launch_bounds__(256) void k_tail_pack(int n, const int* __restrict__ rp, const int* __restrict__ ci,
                                                    const double* __restrict__ v, const int* __restrict__ so,
-                                                   EllEntry<T>* __restrict__ ell) {
+                                                   EllEntry* __restrict__ ell) {
   // a wave per quarter of a slice's width: the rows' loads are spread over four waves
   const int sl = blockIdx.x, lane = threadIdx.x & (kWave - 1), part = threadIdx.x / kWave;
   const int r = sl * kWave + lane;
   const int k1 = so[sl + 1] - so[sl];
   const int e0 = r < n ? rp[r] : 0, len = r < n ? rp[r + 1] - e0 : 0;
   for (int k = part; k < k1; k += 256 / kWave) {
-    EllEntry<T> e{T(0), r < n ? r : 0};
+    EllEntry e{0.0, r < n ? r : 0};
     if (k < len) {
-      e.v = (T)v[e0 + k];
+      e.v = v[e0 + k];
       e.c = ci[e0 + k];
     }
     ell[(long long)(so[sl] + k) * kWave + lane] = e;
@@ -124,29 +128,29 @@ template <class T, int M>
 __device__ __forceinline__ RowPair<T, M> rows_times(const TailLevel& L, const int* __restrict__ so, int i,
                                                     const Cols<T, M>& X) {
   RowPair<T, M> r{};
-  const EllEntry<T>* ell = static_cast<const EllEntry<T>*>(L.ell) + i % kWave;
+  const EllEntry* ell = static_cast<const EllEntry*>(L.ell) + i % kWave;
   const int s0 = i / kWave, s1 = s0 + kTailThreads / kWave, ns = (L.n + kWave - 1) / kWave;
   const int q0 = s0 < ns ? so[s0] : 0, w0 = s0 < ns ? so[s0 + 1] - q0 : 0;
   const int q1 = s1 < ns ? so[s1] : 0, w1 = s1 < ns ? so[s1 + 1] - q1 : 0;
-  const EllEntry<T>* e0 = ell + (long long)q0 * kWave;
-  const EllEntry<T>* e1 = ell + (long long)q1 * kWave;
+  const EllEntry* e0 = ell + (long long)q0 * kWave;
+  const EllEntry* e1 = ell + (long long)q1 * kWave;
   const int both = w0 < w1 ? w0 : w1;
   int k = 0;
 #pragma unroll 4
   for (; k < both; ++k) {
-    const EllEntry<T> x = e0[k * kWave], y = e1[k * kWave];
+    const EllEntry x = e0[k * kWave], y = e1[k * kWave];
     add<T, M>(r.a, x.v, X.get(x.c));
     add<T, M>(r.b, y.v, X.get(y.c));
   }
   const int k0 = k;
 #pragma unroll 8
   for (k = k0; k < w0; ++k) {
-    const EllEntry<T> x = e0[k * kWave];
+    const EllEntry x = e0[k * kWave];
     add<T, M>(r.a, x.v, X.get(x.c));
   }
 #pragma unroll 8
   for (k = k0; k < w1; ++k) {
-    const EllEntry<T> y = e1[k * kWave];
+    const EllEntry y = e1[k * kWave];
     add<T, M>(r.b, y.v, X.get(y.c));
   }
   return r;
@@ -169,12 +173,13 @@ constexpr int kRowLanes = 4;
 // identity's columns). The coarsest level's solve sums in FP64 over the transposed
 // inverse, so that a wave reads contiguous lines: two rows per thread and the columns
 // split over the remaining threads; its x overwrites its b.
-// What bounds it: at 1,200 rows the ~17 dependent phases of 1-4 us (45 us together);
-// at 2,046 rows with 45 entries each the LDS reads of the gathered rows, 29 us per
-// pass over the operator.
+// What bounds it: at 1,200 rows the ~17 dependent phases of 1-6 us (72 us together);
+// on dense levels (852 rows with 24 entries each: 136 us) the LDS reads of the gathered
+// rows.
 constexpr int kTailSlices = kTailLevels * (kTailMax / kWave + 1);
-template <class T, int M>
+template <class S, int M>
 __global__ __launch_bounds__(kTailThreads) void k_tail_form(TailArgs A) {
+  using T = double;
   extern __shared__ __align__(16) unsigned char raw[];
   __shared__ int so[kTailSlices];
   T* lds = reinterpret_cast<T*>(raw);
@@ -314,12 +319,16 @@ __global__ __launch_bounds__(kTailThreads) void k_tail_form(TailArgs A) {
     __syncthreads();
     for (int it = 0; it < A.post; ++it) sweep(l);
   }
-  // the row stride is a multiple of M, so the last columns' padding has its place
-  T* B = static_cast<T*>(A.B);
+  // the row stride holds the last workgroup's padding columns
+  S* B = static_cast<S*>(A.B);
   const Cols<T, M> xb = cur(0);
   for (int i = tid; i < A.lv[0].n; i += kTailThreads) {
     const Vec<T, M> x = xb.get(i);
-    __builtin_memcpy(__builtin_assume_aligned(B + (long long)i * A.ld + c0, 16), &x, sizeof(x));
+    Vec<S, M> r;
+#pragma unroll
+    for (int m = 0; m < M; ++m) r.v[m] = (S)x.v[m];
+    constexpr int align = sizeof(r) % 16 == 0 ? 16 : 8;  // c0 is a multiple of M, ld of 8
+    __builtin_memcpy(__builtin_assume_aligned(B + (long long)i * A.ld + c0, align), &r, sizeof(r));
   }
 }
 
@@ -350,11 +359,11 @@ __global__ __launch_bounds__(256) void k_tail_mv(int n, int ld, const T* __restr
   if (lane == 0) x[r] = (T)t;
 }
 
-template <class T, int M>
+template <class S, int M>
 void form(const TailArgs& A, size_t lds, hipStream_t s) {
-  IMPES_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail_form<T, M>),
+  IMPES_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail_form<S, M>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  k_tail_form<T, M><<<div_up(A.lv[0].n, M), kTailThreads, lds, s>>>(A);
+  k_tail_form<S, M><<<div_up(A.lv[0].n, M), kTailThreads, lds, s>>>(A);
   IMPES_LAUNCH_CHECK();
 }
 
@@ -367,63 +376,81 @@ void launch_tail_slices(int n, const int* rp, int* so, hipStream_t s) {
   IMPES_LAUNCH_CHECK();
 }
 
-size_t tail_ell_bytes(long long slots, int precision) {
-  return (size_t)slots * kWave * (precision == 32 ? sizeof(EllEntry<float>) : sizeof(EllEntry<double>));
-}
+size_t tail_ell_bytes(long long lines) { return (size_t)lines * kWave * sizeof(EllEntry); }
 
-void launch_tail_pack(int precision, int n, const int* rp, const int* ci, const double* v, const int* so, void* ell,
-                      hipStream_t s) {
-  if (precision == 32)
-    k_tail_pack<float><<<tail_slices(n), 256, 0, s>>>(n, rp, ci, v, so, static_cast<EllEntry<float>*>(ell));
-  else
-    k_tail_pack<double><<<tail_slices(n), 256, 0, s>>>(n, rp, ci, v, so, static_cast<EllEntry<double>*>(ell));
+void launch_tail_pack(int n, const int* rp, const int* ci, const double* v, const int* so, void* ell, hipStream_t s) {
+  k_tail_pack<<<tail_slices(n), 256, 0, s>>>(n, rp, ci, v, so, static_cast<EllEntry*>(ell));
   IMPES_LAUNCH_CHECK();
 }
 
-// 16 bytes of columns per row while that takes at most one workgroup per CU, else 32
-// (a second round of workgroups costs as much as the first: 87 against 42 us at 1,200
-// rows)
-static int tail_cols(int precision, int n0) {
-  const int narrow = precision == 32 ? 4 : 2;
-  return div_up(n0, narrow) <= 256 ? narrow : 2 * narrow;
-}
-
-size_t tail_lds_layout(TailArgs& A, int precision) {
-  const int M = tail_cols(precision, A.lv[0].n);
-  const size_t ts = precision == 32 ? 4 : 8;
+// LDS offsets for M columns a workgroup; the bytes. Once a level's residual has been
+// restricted, the buffer that held it is free until the level's first post-sweep: the
+// next level's x and y lie in it where they fit, or the coarsest solve's partial sums.
+static size_t layout(TailArgs& A, int M) {
   long long at = 0;
   auto take = [&](int n) {
     const long long o = at;
     at += (long long)n * M;
     return (int)o;
   };
+  int room = 0, free_at = 0;  // rows and offset of the level above's free buffer
   for (int l = 0; l <= A.levels; ++l) {
     TailLevel& L = A.lv[l];
-    L.x = take(L.n);
-    L.y = l < A.levels ? take(L.n) : 0;
-    L.b = l == A.levels ? L.x : (l > 0 ? take(L.n) : 0);
+    if (l > 0) L.b = take(L.n);
+    if (l == A.levels) {
+      L.x = L.b;
+      L.y = 0;
+      break;
+    }
+    const bool inside = 2 * L.n <= room;
+    L.x = inside ? free_at : take(L.n);
+    L.y = inside ? free_at + L.n * M : take(L.n);
+    room = L.n;
+    free_at = A.pre > 1 && (A.pre - 1) % 2 == 1 ? L.x : L.y;  // the residual's (cur after the sweeps is the other)
   }
-  // the coarsest solve's partial sums: one split per group of threads over the row
-  // pairs, as many as fit
+  // one split per group of threads over the row pairs, as many as fit
   const int n = A.lv[A.levels].n;
-  const size_t one = (size_t)n * M * sizeof(double), used = (size_t)at * ts;
+  const size_t used = (size_t)at * sizeof(double), one = (size_t)n * M * sizeof(double);
   const int groups = kTailThreads / (div_up((n + 1) / 2, kWave) * kWave);
-  const size_t fit = used < kTailLds ? (kTailLds - used) / one : 0;
-  A.splits = (int)std::min<size_t>(groups, fit);
-  A.part = (int)at;
-  return A.splits > 0 ? used + A.splits * one : kTailLds + 1;
+  const int in_room = std::min(groups, room / n);
+  const int behind = used < kTailLds ? (int)std::min<size_t>(groups, (kTailLds - used) / one) : 0;
+  A.splits = std::max(in_room, behind);
+  A.part = in_room >= behind ? free_at : (int)at;
+  if (A.splits == 0) return kTailLds + 1;
+  return in_room >= behind ? used : used + A.splits * one;
+}
+
+// Columns a workgroup: the fewest that take at most one workgroup per CU, since a second
+// round of workgroups costs as much as the first (1,200 rows: 99 us with 4, in two
+// rounds, 72 with 6; 1,072 rows 118 and 84), where six columns fit the LDS; else 4.
+static int tail_cols(TailArgs& A) {
+  for (int M : {2, 4, 6})
+    if (div_up(A.lv[0].n, M) <= 256 && layout(A, M) <= kTailLds) return M;
+  return 4;
+}
+
+// Two or four columns of every vector side by side (x and y, b below the first level,
+// the partial sums) fit the LDS: up to about 1,500 rows. Larger ones would fit as well
+// with the shared buffers, but take two rounds of long passes and do not pay.
+bool tail_fits(const TailArgs& A) {
+  const int n0 = A.lv[0].n, nc = A.lv[A.levels].n;
+  long long rows = 2LL * n0 + (n0 > 512 && n0 <= 1024 ? 2LL : 3LL) * nc;
+  for (int l = 1; l < A.levels; ++l) rows += 3LL * A.lv[l].n;
+  return rows * (n0 <= 512 ? 16 : 32) <= (long long)kTailLds;
 }
 
 void launch_tail_form(int precision, TailArgs A, hipStream_t s) {
-  const size_t lds = tail_lds_layout(A, precision);
+  const int M = tail_cols(A);
+  const size_t lds = layout(A, M);
   IMPES_REQUIRE(lds <= kTailLds, "tail: vectors exceed LDS");
-  const int M = tail_cols(precision, A.lv[0].n);
-  IMPES_REQUIRE(A.ld % M == 0 && A.ld >= div_up(A.lv[0].n, M) * M, "tail: row stride");
+  IMPES_REQUIRE(A.ld % 2 == 0 && A.ld >= div_up(A.lv[0].n, M) * M, "tail: row stride");
   if (precision == 32) {
-    if (M == 8) form<float, 8>(A, lds, s);
-    else form<float, 4>(A, lds, s);
+    if (M == 6) form<float, 6>(A, lds, s);
+    else if (M == 4) form<float, 4>(A, lds, s);
+    else form<float, 2>(A, lds, s);
   } else {
-    if (M == 4) form<double, 4>(A, lds, s);
+    if (M == 6) form<double, 6>(A, lds, s);
+    else if (M == 4) form<double, 4>(A, lds, s);
     else form<double, 2>(A, lds, s);
   }
 }
