@@ -202,6 +202,8 @@ class SetupPool {
 
 // Gives the cached idle blocks of every device back to it.
 void release_cached_memory();
+// hipMalloc; where the device is out of memory, once more without the cached blocks.
+void* device_malloc(size_t bytes);
 
 // The pool that DevBuf allocations use on this thread (null outside a scope).
 std::shared_ptr<SetupPool> current_setup_pool();
@@ -263,7 +265,7 @@ struct DevBuf {
       p = static_cast<T*>(sp->alloc(count * sizeof(T)));
       pool = std::move(sp);
     } else {
-      IMPES_HIP_CHECK(hipMalloc((void**)&p, count * sizeof(T)));
+      p = static_cast<T*>(device_malloc(count * sizeof(T)));
     }
     n = count;
   }

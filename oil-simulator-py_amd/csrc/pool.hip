@@ -14,8 +14,8 @@ namespace {
 // Idle device blocks kept for the next build on the same device (a build of a
 // 500,000-cell hierarchy took 5 ms in 120 hipMalloc calls and its destruction 26 ms
 // in as many hipFree calls). At most kBlockCacheBytes per device; more is freed at
-// once. An allocation that fails gives the whole cache back and tries again, and
-// trim() does so on request. Blocks enter only once the device has finished with
+// once. An allocation of the library that runs out of memory gives the whole cache back
+// and tries again (device_malloc), and trim() does so on request. Blocks enter only once the device has finished with
 // them (the callers below), so any stream may take them.
 constexpr size_t kBlockCacheBytes = size_t(4) << 30;
 struct BlockCache {
@@ -36,16 +36,8 @@ struct BlockCache {
         return p;
       }
     }
-    void* p = nullptr;
-    hipError_t rc = hipMalloc(&p, want);
-    if (rc != hipSuccess) {
-      (void)hipGetLastError();
-      trim();
-      rc = hipMalloc(&p, want);
-    }
-    IMPES_HIP_CHECK(rc);
     *got = want;
-    return p;
+    return device_malloc(want);
   }
   void give(int dev, void* p, size_t size) {
     {
@@ -89,6 +81,18 @@ bool device_idle(int dev) {
 }  // namespace
 
 void release_cached_memory() { block_cache().trim(); }
+
+void* device_malloc(size_t bytes) {
+  void* p = nullptr;
+  hipError_t rc = hipMalloc(&p, bytes);
+  if (rc == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    release_cached_memory();
+    rc = hipMalloc(&p, bytes);
+  }
+  IMPES_HIP_CHECK(rc);
+  return p;
+}
 
 struct SetupPool::Impl {
   struct Slab {

@@ -75,7 +75,8 @@ def copy_f64(y, x):
 
 
 def release_cached_memory():
-    """Give the device memory kept between hierarchy builds (at most 4 GiB) back."""
+    """Give the device memory kept between hierarchy builds (at most 4 GiB) back, for
+    allocators outside the library (torch's cannot reclaim it)."""
     call("impes_release_cached_memory")
 
 
