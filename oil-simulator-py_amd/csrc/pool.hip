@@ -68,12 +68,16 @@ BlockCache& block_cache() {
   return *c;
 }
 
-// Waits for a device; false when that fails (its blocks are then freed, not kept).
+// Waits for a device; false when that fails (its blocks are then freed, not kept). By
+// hipFree, which waits for all of the device's work: hipDeviceSynchronize would end every
+// capture in progress, those of other threads included.
 bool device_idle(int dev) {
   int cur = 0;
   if (hipGetDevice(&cur) != hipSuccess) return false;
   if (cur != dev && hipSetDevice(dev) != hipSuccess) return false;
-  const bool ok = hipDeviceSynchronize() == hipSuccess;
+  void* p = nullptr;
+  const bool ok = hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess;
+  if (!ok) (void)hipGetLastError();
   if (cur != dev) (void)hipSetDevice(cur);
   return ok;
 }
