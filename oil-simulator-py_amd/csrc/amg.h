@@ -286,9 +286,10 @@ class Hierarchy {
   std::vector<long long> tail_at_;   // per level from tail_: first slice offset in tail_so_
   std::vector<long long> tail_line_; // per level from tail_: first line in tail_ell_ (last: the total)
   DevBuf<int> tail_so_;
-  DevBuf<unsigned char> tail_ell_;
-  DevBuf<float> tail_b32_;
-  DevBuf<double> tail_b64_;
+  DevBuf<unsigned char> tail_mem_;  // one block: the matrix per precision, the sliced operators
+  double* tail_b64_ = nullptr;
+  float* tail_b32_ = nullptr;
+  unsigned char* tail_ell_ = nullptr;
   DevBuf<double> tiles64_;           // FP64 values of all the levels' tiles
 
   AmgParams prm_;

@@ -968,7 +968,8 @@ void Hierarchy::form_tiles64(hipStream_t s) {
 
 // Whatever cycles form from the levels has its memory from the setup on (out of the
 // setup's pool): a cycle allocates nothing, so that its first run can be recorded into a
-// caller's graph. One block holds the FP64 tiles of all levels.
+// caller's graph. One block holds the FP64 tiles of all levels, one the coarse end's
+// matrices: an allocation that the pool has not kept costs 0.03-0.8 ms.
 void Hierarchy::alloc_derived() {
   const int end = tail_ >= 0 ? tail_ : (int)levels_.size() - 1;
   auto each = [&](auto&& f) {
@@ -989,10 +990,11 @@ void Hierarchy::alloc_derived() {
     at += 4 * (size_t)nw * kWave;
   });
   if (tail_ < 0) return;
-  tail_ell_.alloc(tail_ell_bytes(tail_line_.back()));
-  const size_t nb = (size_t)levels_[tail_].n * tail_ld_;
-  tail_b32_.alloc(nb);
-  tail_b64_.alloc(nb);
+  const size_t nb = (size_t)levels_[tail_].n * tail_ld_;  // a multiple of 8
+  tail_mem_.alloc(nb * (sizeof(double) + sizeof(float)) + tail_ell_bytes(tail_line_.back()));
+  tail_b64_ = reinterpret_cast<double*>(tail_mem_.p);
+  tail_b32_ = reinterpret_cast<float*>(tail_b64_ + nb);
+  tail_ell_ = reinterpret_cast<unsigned char*>(tail_b32_ + nb);
 }
 
 void Hierarchy::form(Form f, hipStream_t s) {
@@ -1089,7 +1091,7 @@ void Hierarchy::form_tail(int precision, hipStream_t s) {
     t.n = L.n;
     if (q == last) break;
     t.so = (int)tail_at_[q - tail_];
-    unsigned char* ell = tail_ell_.p + tail_ell_bytes(tail_line_[q - tail_]);
+    unsigned char* ell = tail_ell_ + tail_ell_bytes(tail_line_[q - tail_]);
     launch_tail_pack(L.n, L.rp.p, L.ci.p, L.v.p, tail_so_.p + t.so, ell, s);
     t.ell = ell;
     t.ir = L.ir64.p;
@@ -1106,7 +1108,7 @@ void Hierarchy::form_tail(int precision, hipStream_t s) {
   A.post = prm_.post_smooth;
   A.omega = prm_.omega;
   A.ld = tail_ld_;
-  A.B = precision == 32 ? (void*)tail_b32_.p : (void*)tail_b64_.p;
+  A.B = precision == 32 ? (void*)tail_b32_ : (void*)tail_b64_;
   launch_tail_form(precision, A, s);
 }
 
@@ -1277,8 +1279,8 @@ template <class T>
 void Hierarchy::vcycle_level(int l, const T* b, T* x, bool x_zero, hipStream_t s, bool first_sweep_done, bool tail) {
   Level& L = levels_[l];
   if (tail && l == tail_) {
-    if constexpr (sizeof(T) == 8) launch_tail_mv_f64(L.n, tail_ld_, tail_b64_.p, b, x, s);
-    else launch_tail_mv_f32(L.n, tail_ld_, tail_b32_.p, b, x, s);
+    if constexpr (sizeof(T) == 8) launch_tail_mv_f64(L.n, tail_ld_, tail_b64_, b, x, s);
+    else launch_tail_mv_f32(L.n, tail_ld_, tail_b32_, b, x, s);
     return;
   }
   const int m0 = mark(s);
