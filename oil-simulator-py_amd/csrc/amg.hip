@@ -609,7 +609,7 @@ void Hierarchy::build_levels(hipStream_t s) {
     cvals.alloc(ncand);
     launch_interp_expand(n, A.nnz, A.rp.p, A.ci.p, A.v.p, strong.p, A.cf.p, sum_strong.p, cnt_c.p, f2c.p, cand_ptr.p, keys.p,
                          cvals.p, s);
-    segmented_sort_u64(keys.p, cand_ptr.p, n, s);
+    segmented_sort_u64(keys.p, cand_ptr.p, n, ncand, s);
     oc.alloc(ncand);
     ov.alloc(ncand);
     pcnt.alloc(n);
@@ -636,7 +636,7 @@ void Hierarchy::build_levels(hipStream_t s) {
       DevBuf<unsigned long long> tkeys;
       tkeys.alloc(A.pnnz);
       launch_transpose_fill(n, A.prp.p, A.pci.p, A.rrp.p, cursor.p, tkeys.p, s);
-      segmented_sort_u64(tkeys.p, rrp64.p, nc, s);
+      segmented_sort_u64(tkeys.p, rrp64.p, nc, A.pnnz, s);
       A.rci.alloc(A.pnnz);
       A.rv.alloc(A.pnnz);
       launch_transpose_finish(A.pnnz, tkeys.p, A.pv.p, A.rci.p, A.rv.p, s);
@@ -660,7 +660,7 @@ void Hierarchy::build_levels(hipStream_t s) {
       ex_e.alloc(tot);
       ex_f.alloc(tot);
       launch_spgemm_expand(nrows, lnnz, tot, lrp, lci, mrp, mci, pptr.p, pk.p, ex_e.p, ex_f.p, s);
-      segmented_sort_u64(pk.p, pptr.p, nrows, s);
+      segmented_sort_u64(pk.p, pptr.p, nrows, tot, s);
       uc.alloc(nrows);
       launch_spgemm_unique_count(nrows, pptr.p, pk.p, uc.p, s);
       crp.alloc(nrows + 1);

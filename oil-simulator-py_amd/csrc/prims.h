@@ -12,9 +12,10 @@ namespace impes {
 void scan_i32_to_i64(const int* in, long long* out, long long n, hipStream_t s);
 void scan_i32_to_i32(const int* in, int* out, long long n, hipStream_t s);
 
-// Sort every segment [seg[i], seg[i+1]) of `keys` ascending. Does not wait for the
-// stream: the number of segments per length class stays on the device.
-void segmented_sort_u64(unsigned long long* keys, const long long* seg, long long nseg, hipStream_t s);
+// Sort every segment [seg[i], seg[i+1]) of the `total` keys ascending. Does not wait for
+// the stream: the number of segments per length class stays on the device.
+void segmented_sort_u64(unsigned long long* keys, const long long* seg, long long nseg, long long total,
+                        hipStream_t s);
 
 // Partial sums of an int32 array, and of the count of int8 entries equal to v, into
 // part (kSumParts values); returns how many were written (Readback::sum adds them up).

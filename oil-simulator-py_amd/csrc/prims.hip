@@ -251,25 +251,43 @@ __global__ __launch_bounds__(NT) void k_segsort_bin(unsigned long long* __restri
   }
 }
 
-// Few segments: a workgroup per segment whatever its length, without the classes
-// (nine launches otherwise, which bind a small level's sort): the same network in LDS,
-// or in place above kSortAnyLds keys.
+// Few segments: a workgroup per segment without the classes (nine launches otherwise,
+// which bind a small level's sort), the same network in LDS. Segments above kSortAnyLds
+// keys are left to k_segsort_few_long.
 constexpr int kSortAny = 4096, kSortAnyLds = 4096;
 __global__ __launch_bounds__(256) void k_segsort_any(unsigned long long* __restrict__ keys,
                                                      const long long* __restrict__ seg) {
   __shared__ unsigned long long sk[kSortAnyLds];
   const long long b = seg[blockIdx.x], len = seg[blockIdx.x + 1] - b;
-  if (len <= 1) return;
-  if (len > kSortAnyLds) {
-    bitonic_any(keys + b, len);
-    return;
-  }
+  if (len <= 1 || len > kSortAnyLds) return;
   int p2 = 2;
   while (p2 < len) p2 <<= 1;
   for (int t = threadIdx.x; t < p2; t += 256) sk[t] = (t < len) ? keys[b + t] : ~0ull;
   __syncthreads();
   bitonic_block(sk, (long long)p2);
   for (int t = threadIdx.x; t < len; t += 256) keys[b + t] = sk[t];
+}
+
+// The long ones among few segments: in LDS up to 8192 keys, else in place. With 256
+// threads to such a segment (in k_segsort_any) the sorts of a hierarchy of 20,000 rows and
+// 2M entries took 166 ms, with 1024 they take 60; looking the lengths over takes about 3 us.
+constexpr int kSortLongLds = 8192;
+__global__ __launch_bounds__(1024) void k_segsort_few_long(unsigned long long* __restrict__ keys,
+                                                           const long long* __restrict__ seg, int nseg) {
+  __shared__ unsigned long long sk[kSortLongLds];
+  for (int sg = blockIdx.x; sg < nseg; sg += gridDim.x) {
+    const long long b = seg[sg], len = seg[sg + 1] - b;
+    if (len <= kSortAnyLds) continue;
+    if (len > kSortLongLds) {
+      bitonic_any(keys + b, len);
+      continue;
+    }
+    for (int t = threadIdx.x; t < kSortLongLds; t += 1024) sk[t] = (t < len) ? keys[b + t] : ~0ull;
+    __syncthreads();
+    bitonic_block(sk, (long long)kSortLongLds);
+    for (int t = threadIdx.x; t < len; t += 1024) keys[b + t] = sk[t];
+    __syncthreads();
+  }
 }
 
 // Segments longer than the LDS classes, a workgroup each, in place
@@ -423,11 +441,15 @@ __global__ __launch_bounds__(kScanBlock) void k_select_pick(int shift, long long
 void scan_i32_to_i64(const int* in, long long* out, long long n, hipStream_t s) { scan_impl<long long>(in, out, n, s); }
 void scan_i32_to_i32(const int* in, int* out, long long n, hipStream_t s) { scan_impl<int>(in, out, n, s); }
 
-void segmented_sort_u64(unsigned long long* keys, const long long* seg, long long nseg, hipStream_t s) {
+void segmented_sort_u64(unsigned long long* keys, const long long* seg, long long nseg, long long total,
+                        hipStream_t s) {
   if (nseg <= 0) return;
   IMPES_REQUIRE(nseg < (1LL << 31), "segmented sort: too many segments");
   if (nseg <= kSortAny) {
     k_segsort_any<<<(int)nseg, 256, 0, s>>>(keys, seg);
+    IMPES_LAUNCH_CHECK();
+    if (total <= kSortAnyLds) return;
+    k_segsort_few_long<<<(int)(nseg < 512 ? nseg : 512), 1024, 0, s>>>(keys, seg, (int)nseg);
     IMPES_LAUNCH_CHECK();
     return;
   }

@@ -26,11 +26,26 @@ def hub(n, leaves):
     return (A.tocsr() + H + sp.diags(-np.asarray(H.sum(1)).ravel())).tocsr()
 
 
+def dense(n, per):
+    """A random M-matrix of about `per` entries in a row."""
+    rng = np.random.default_rng(0)
+    B = sp.random(n, n, per / (2.0 * n), random_state=rng, format="csr", data_rvs=lambda k: np.exp(rng.standard_normal(k)))
+    B = B + B.T
+    B.setdiag(0.0)
+    B.eliminate_zeros()
+    A = sp.csr_matrix(sp.diags(np.asarray(B.sum(1)).ravel() + 0.01) - B)
+    A.sort_indices()
+    return A
+
+
 CASES = {
     "tiny": (lambda: impes_like(5, 4, 3)[0], dict(coarsest_size=4, max_levels=25), 1),
     "odd": (lambda: impes_like(17, 13, 3, seed=2)[0], dict(coarsest_size=10, max_levels=25), 1),
     "wide": (lambda: impes_like(40, 40, 20, seed=3)[0], {}, 1),
     "hub": (lambda: hub((24, 24, 24), 9000), dict(coarsest_size=100), 2049),
+    # few rows with product lists beyond a workgroup's LDS (the sort's long segments)
+    "hub_few_rows": (lambda: hub((15, 15, 15), 3000), dict(coarsest_size=100), 2049),
+    "dense_few_rows": (lambda: dense(700, 300), dict(coarsest_size=20, max_levels=25), 1),
 }
 
 
