@@ -201,6 +201,8 @@ class Hierarchy {
   const double* diag0() const { return diag0_.p; }   // unscaled fine diagonal
   const Level& level(int l) const { return levels_[l]; }
   bool is_stencil() const { return stencil_; }
+  // a row of the fine CSR operator is too long for a tile (more than 256 entries)
+  bool long_rows() const { return !stencil_ && levels_[0].pad4 && levels_[0].nw4 == 0; }
   const AmgParams& params() const { return prm_; }
   double last_setup_seconds = 0.0;
 

@@ -658,8 +658,10 @@ void Fgmres::solve(const Operator& A, Hierarchy* M, int precision, const double*
   // kernels; else CGS2's three passes and a normalisation
   const bool lagged = M != nullptr && m <= kMaxFusedGs && !cgs2_;
   // one workgroup per step where the system is small (fgmres_small.hip); its rows are
-  // walked by one lane each, so long CSR rows keep the kernels with lanes per row
-  const bool small = lagged && n <= kSmallRows && (A.stencil || A.csr.nnz <= kSmallRowNnz * n);
+  // walked by one lane each, so long CSR rows keep the kernels with lanes per row, many
+  // of them or a single one (a row of 3,600 entries costs its lane 90 us a step)
+  const bool small =
+      lagged && n <= kSmallRows && (A.stencil || (A.csr.nnz <= kSmallRowNnz * n && !M->long_rows()));
   const SmallOperator So{A.stencil, A.st, A.csr, A.dinv, (int)n};
   float* b32 = small && precision == 32 ? (float*)M->vcycle_in(32) : nullptr;
   double* b64 = small && precision == 64 ? (double*)M->vcycle_in(64) : nullptr;

@@ -8,6 +8,7 @@ Bars: the asked relative residual times a condition allowance for the solution; 
 same number of steps up to one (the stopping test sees another rounding)."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import scipy.sparse.linalg as spl
 import torch
 
@@ -78,3 +79,30 @@ def test_small_error_check_start_and_zero_rhs(dev, kind):
     assert np.max(np.abs(x1 - y)) <= 1e-8 * np.max(np.abs(y))
     *_, x2, st2 = _solve(dev, (20, 20, 3), kind, 32, 30, b=np.zeros(A.shape[0]), x0=y)
     assert st2["converged"] and not x2.any()
+
+
+@pytest.mark.parametrize("leaves", [200, 1500])
+def test_one_long_row(dev, leaves):
+    """A small system with one row of some hundred or thousand entries: on both sides of
+    the length from which the separate kernels take it."""
+    import impes_hip as H
+    from test_gpu_solver import to_dev
+
+    A = impes_like(40, 40, 1, wells=0)[0]
+    n = A.shape[0]
+    at = np.random.default_rng(0).choice(n - 1, size=leaves, replace=False)
+    E = sp.coo_matrix((np.full(leaves, -1e-13), (np.full(leaves, n - 1), at)), shape=(n, n))
+    E = (E + E.T).tocsr()
+    A = (A + E + sp.diags(-np.asarray(E.sum(1)).ravel())).tocsr()
+    A.sort_indices()
+    csr = to_dev(A, dev)
+    b = A @ np.random.default_rng(1).standard_normal(A.shape[0])
+    for precision in (32, 64):
+        h = H.AmgHierarchy(coarsest_size=60)
+        h.setup_csr(*csr)
+        x = torch.zeros(A.shape[0], dtype=torch.float64, device=dev)
+        d = A.diagonal()
+        st = H.FgmresSolver().solve_csr(h, *csr, torch.tensor(1.0 / d, device=dev), torch.tensor(b, device=dev), x,
+                                        precision=precision, rtol=1e-10)
+        assert st["converged"]
+        assert np.linalg.norm((b - A @ x.cpu().numpy()) / d) <= 1.01e-10 * np.linalg.norm(b / d)
