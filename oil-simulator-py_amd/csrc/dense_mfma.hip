@@ -102,7 +102,15 @@ __device__ __forceinline__ void tile_put(const TileRegs& t, double* __restrict__
 // column's entries in order (repeated columns are adjacent) and the row is written
 // out. Padding rows are identity rows; a pinned DOF 0 keeps only a_00 = 1 in its row
 // and column. A one-thread scatter of the row took 14.8 us at 450 rows.
+// A level far from 1 (a_00 beyond 2^+-400) is scaled by a power of two, and its inverse
+// with it in the last launch: the pivot blocks' 2 x 2 determinants would leave the range
+// of doubles where the pivots do not. Entries may still differ by 30 orders and more.
 constexpr int kFillThreads = 256;
+__device__ __forceinline__ double range_scale(double a00) {
+  if (!(fabs(a00) > 0.0 && fabs(a00) <= 1.7976931348623157e308)) return 1.0;
+  const int e = ilogb(a00);
+  return e >= -400 && e <= 400 ? 1.0 : ldexp(1.0, e > 0 ? -e : (e < -1000 ? 1000 : -e));
+}
 __global__ __launch_bounds__(kFillThreads) void k_fill_padded(int n, int n_pad, const int* __restrict__ rp,
                                                               const int* __restrict__ ci, const double* __restrict__ v,
                                                               const int* __restrict__ pin_flag, double* __restrict__ M) {
@@ -115,12 +123,13 @@ __global__ __launch_bounds__(kFillThreads) void k_fill_padded(int n, int n_pad, 
     if (threadIdx.x == 0) row[r] = 1.0;
   } else {
     const int e0 = rp[r], e1 = rp[r + 1];
+    const double scale = range_scale(*v);
     for (int e = e0 + threadIdx.x; e < e1; e += kFillThreads) {
       const int c = ci[e];
       if ((e > e0 && ci[e - 1] == c) || (pin && c == 0)) continue;
       double sum = v[e];
       for (int q = e + 1; q < e1 && ci[q] == c; ++q) sum += v[q];
-      row[c] = sum;
+      row[c] = sum * scale;
     }
   }
   __syncthreads();
@@ -257,11 +266,12 @@ __device__ __forceinline__ bool invert_block(v4d (&acc)[4], double* __restrict__
 // sym_rows > 0, block b checks row b - 1 for symmetry, |a_ij - a_ji| <= 1e-10
 // sqrt(a_ii a_jj) (the rounding asymmetry of a Galerkin product passes, a
 // non-symmetric operator does not; well rows can exceed interior rows by 15 orders,
-// so the scale is per entry), and for a positive diagonal, and keeps the diagonal.
+// so the scale is per entry), and for a positive diagonal, and keeps the diagonal. a00:
+// the level's first entry, from which a result takes its scale (range_scale).
 __global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n, int n_pad, int sym_rows, const double* __restrict__ M,
                                                           double* __restrict__ P, double* __restrict__ PT,
                                                           double* __restrict__ dg, double tol,
-                                                          int* __restrict__ bad) {
+                                                          int* __restrict__ bad, const double* __restrict__ a00) {
   if (blockIdx.x > 0) {
     const int r = blockIdx.x - 1;
     const double dr = M[(long long)r * n_pad + r];
@@ -293,14 +303,16 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n, int n_pad, int 
     }
   __syncthreads();
   if (!invert_block(acc, lds, dg ? d0 : nullptr, tol, min(n, kB))) *bad = 1;
+  const double scale = PT ? range_scale(*a00) : 1.0;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       int r, c;
       tile_pos(t, e, r, c);
-      P[r * kB + c] = acc[t][e];
-      if (PT) PT[c * kB + r] = acc[t][e];
+      const double x = acc[t][e] * scale;
+      P[r * kB + c] = x;
+      if (PT) PT[c * kB + r] = x;
     }
 }
 
@@ -310,23 +322,25 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_diag(int n, int n_pad, int 
 // its own row-k block stores. The longest path of a launch is the workgroup that
 // also inverts the next pivot block (fetches, two products of 1.7 us, the inverse);
 // every tile it needs is fetched before the first product. The last block column
-// also writes the transposed inverse (AnT). One launch per block
+// also scales the inverse (a00, range_scale) and writes its transpose (AnT). One launch per block
 // column: 47-49 -> 13-24 us at 83-576 rows.
 __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n, int n_pad, const double* __restrict__ A,
                                                           double* __restrict__ An, const double* __restrict__ P,
                                                           double* __restrict__ Pn, double* __restrict__ AnT,
                                                           const double* __restrict__ dg, double tol,
-                                                          int* __restrict__ bad) {
+                                                          int* __restrict__ bad, const double* __restrict__ a00) {
   __shared__ double As[kB * kLdA], Bs[kB * kLdB], Cs[kB * kLdA];
   __shared__ double d0[kB];  // the next pivot block's entries of dg
   const int j = blockIdx.x, i = blockIdx.y;
   const double* blk = A + (long long)i * kB * n_pad + (long long)j * kB;
   double* out = An + (long long)i * kB * n_pad + (long long)j * kB;
   double* outT = AnT ? AnT + (long long)j * kB * n_pad + (long long)i * kB : nullptr;
+  const double scale = AnT ? range_scale(*a00) : 1.0;
   if (i == k && j == k) {
     for (int q = threadIdx.x; q < kB * kB; q += blockDim.x) {
-      out[(long long)(q / kB) * n_pad + q % kB] = P[q];
-      if (outT) outT[(long long)(q % kB) * n_pad + q / kB] = P[q];
+      const double x = P[q] * scale;
+      out[(long long)(q / kB) * n_pad + q % kB] = x;
+      if (outT) outT[(long long)(q % kB) * n_pad + q / kB] = x;
     }
     return;
   }
@@ -348,8 +362,9 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n, int n_pa
       for (int e = 0; e < 4; ++e) {
         int r, c;
         tile_pos(t, e, r, c);
-        out[(long long)r * n_pad + c] = -acc[t][e];
-        if (outT) outT[(long long)c * n_pad + r] = -acc[t][e];
+        const double x = -acc[t][e] * scale;
+        out[(long long)r * n_pad + c] = x;
+        if (outT) outT[(long long)c * n_pad + r] = x;
       }
     return;
   }
@@ -366,8 +381,9 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n, int n_pa
       for (int e = 0; e < 4; ++e) {
         int r, c;
         tile_pos(t, e, r, c);
-        out[(long long)r * n_pad + c] = acc[t][e];
-        if (outT) outT[(long long)c * n_pad + r] = acc[t][e];
+        const double x = acc[t][e] * scale;
+        out[(long long)r * n_pad + c] = x;
+        if (outT) outT[(long long)c * n_pad + r] = x;
       }
     return;
   }
@@ -406,8 +422,8 @@ __global__ __launch_bounds__(kGemmThreads) void k_gj_step(int k, int n, int n_pa
       int r, c;
       tile_pos(t, e, r, c);
       own[t][e] -= acc[t][e];
-      out[(long long)r * n_pad + c] = own[t][e];
-      if (outT) outT[(long long)c * n_pad + r] = own[t][e];
+      out[(long long)r * n_pad + c] = own[t][e] * scale;
+      if (outT) outT[(long long)c * n_pad + r] = own[t][e] * scale;
     }
   if (i != k + 1 || j != k + 1 || Pn == nullptr) return;
   // this block is the next step's pivot block: its inverse goes to step k + 1 in Pn
@@ -473,13 +489,14 @@ void launch_dense_inverse_mfma(int n, const int* rp, const int* ci, const double
   // workgroup writes P_{k+1} into the other half. With one block its inverse is the
   // result (n_pad = 64 = the leading dimension of P).
   k_gj_diag<<<1 + (strict ? n : 0), kGemmThreads, 0, s>>>(n, n_pad, strict ? n : 0, cur, nb == 1 ? M : P,
-                                                              nb == 1 ? MT : nullptr, dg, tol, bad);
+                                                              nb == 1 ? MT : nullptr, dg, tol, bad, v);
   IMPES_LAUNCH_CHECK();
   if (nb == 1) return;
   for (int k = 0; k < nb; ++k) {
     double* Pk = P + (k & 1) * kB * kB;
     double* Pn = (k + 1 < nb) ? P + ((k + 1) & 1) * kB * kB : nullptr;
-    k_gj_step<<<dim3(nb, nb), kGemmThreads, 0, s>>>(k, n, n_pad, cur, nxt, Pk, Pn, k + 1 == nb ? MT : nullptr, dg, tol, bad);
+    k_gj_step<<<dim3(nb, nb), kGemmThreads, 0, s>>>(k, n, n_pad, cur, nxt, Pk, Pn, k + 1 == nb ? MT : nullptr, dg,
+                                                    tol, bad, v);
     IMPES_LAUNCH_CHECK();
     std::swap(cur, nxt);
   }

@@ -71,3 +71,19 @@ def test_not_spd_falls_back_to_pivoting(dev, n, kind):
     for M in (A, C):
         h.update_csr(_csr(M, dev)[2])
         _check(h, M, s, dev)
+
+
+@pytest.mark.parametrize("scale", [1e-300, 1e-160, 1e160, 1e300])
+@pytest.mark.parametrize("n", [40, 100, 300, 577])
+def test_operators_far_from_one(dev, n, scale):
+    """Products of two entries leave the range of doubles, the entries do not."""
+    import impes_hip as H
+
+    B = np.random.default_rng(n).standard_normal((n, n))
+    A = B @ B.T / n + np.eye(n)
+    h = H.AmgHierarchy(coarsest_size=2000, dense_max=2000, coarse_pin=0, equil_threshold=0.0)
+    h.setup_csr(*_csr(A * scale, dev))
+    b = np.random.default_rng(1).standard_normal(n)
+    x = h.vcycle(torch.tensor(b * scale, device=dev), precision=64).cpu().numpy()
+    y = np.linalg.solve(A, b)
+    assert np.linalg.norm(x - y) <= 4 * n * 2.2e-16 * np.linalg.cond(A) * np.linalg.norm(y)
