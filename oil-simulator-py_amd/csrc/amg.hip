@@ -923,13 +923,16 @@ LevelInfo Hierarchy::info(int l) const {
 // After the coarse correction e the first post-sweep is x + P e + w D^-1 (b - A (x + P
 // e)) = x + w D^-1 r + (P - w D^-1 A P) e, with the residual r that the restriction has
 // left: one pass over a matrix with the pattern of AP (already formed for the Galerkin
-// product) instead of one over P and one over A. FP32 cycle, in tiles.
+// product) instead of one over P and one over A. In tiles: the FP32 cycle and the FP64
+// preconditioner.
 // Measured, the pass and its share of the refresh against the two passes and the gap
 // between them: CSR levels of 16,000 rows 3.6 against 7.6 us, of 82,000 rows 5.9 against
 // 9.3, of 409,000 rows 19.2 against 21.4. A stencil level's sweep is cheaper than its
-// matrix (7 values a cell, no columns): 76,800 cells 4.1 against 6.4 us, 200,000 cells
-// 7.9 against 8.4, beyond that the two passes.
-constexpr int kSweepStencilMax = 1 << 18;
+// matrix (7 values a cell, no columns). What a cycle gains and an update pays for it,
+// about ten cycles to an update: 7,200 cells FP32 2.3 and 1.5 us (FP64 2.9 and 3); 32,000
+// cells 3.0 and 3 (2.5 and 4); 76,800 cells 1.7 and 5 (1.8 and 13); 99,000 cells 0.2 and
+// 12 (1.1 and 10); 169,275 cells 0.1 and 6 (0.7 and 15); from 200,000 cells a loss in both.
+constexpr int kSweepStencilMax = 3 << 15;
 void Hierarchy::build_prolong_sweeps(hipStream_t s) {
   for (auto& L : levels_) L.s4 = Pad4{};
   if (prm_.post_smooth < 1 && prm_.pre_smooth < 1) return;
