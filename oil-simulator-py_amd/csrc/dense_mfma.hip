@@ -97,11 +97,11 @@ __device__ __forceinline__ void tile_put(const TileRegs& t, double* __restrict__
   }
 }
 
-// Dense n_pad x n_pad from CSR (sorted columns): one workgroup per row; the row is
-// zeroed in LDS, then the thread of the first entry of each column adds that
-// column's entries in order (repeated columns are adjacent) and the row is written
-// out. Padding rows are identity rows; a pinned DOF 0 keeps only a_00 = 1 in its row
-// and column. A one-thread scatter of the row took 14.8 us at 450 rows.
+// Dense n_pad x n_pad from CSR: one workgroup per row; the row is zeroed in LDS, then the
+// thread of the first entry of each column adds that column's entries in order (repeated
+// columns are adjacent where the columns are sorted, as a setup's own levels have them;
+// else one thread adds the row up) and the row is written out. Padding rows are identity
+// rows; a pinned DOF 0 keeps only a_00 = 1 in its row and column. A one-thread scatter of the row took 14.8 us at 450 rows.
 // A level far from 1 (a_00 beyond 2^+-400) is scaled by a power of two, and its inverse
 // with it in the last launch: the pivot blocks' 2 x 2 determinants would leave the range
 // of doubles where the pivots do not. Entries may still differ by 30 orders and more.
@@ -124,12 +124,19 @@ __global__ __launch_bounds__(kFillThreads) void k_fill_padded(int n, int n_pad, 
   } else {
     const int e0 = rp[r], e1 = rp[r + 1];
     const double scale = range_scale(*v);
-    for (int e = e0 + threadIdx.x; e < e1; e += kFillThreads) {
-      const int c = ci[e];
-      if ((e > e0 && ci[e - 1] == c) || (pin && c == 0)) continue;
-      double sum = v[e];
-      for (int q = e + 1; q < e1 && ci[q] == c; ++q) sum += v[q];
-      row[c] = sum * scale;
+    bool sorted = true;
+    for (int e = e0 + 1 + threadIdx.x; e < e1; e += kFillThreads) sorted = sorted && ci[e - 1] <= ci[e];
+    if (__syncthreads_and(sorted)) {
+      for (int e = e0 + threadIdx.x; e < e1; e += kFillThreads) {
+        const int c = ci[e];
+        if ((e > e0 && ci[e - 1] == c) || (pin && c == 0)) continue;
+        double sum = v[e];
+        for (int q = e + 1; q < e1 && ci[q] == c; ++q) sum += v[q];
+        row[c] = sum * scale;
+      }
+    } else if (threadIdx.x == 0) {
+      for (int e = e0; e < e1; ++e)
+        if (!(pin && ci[e] == 0)) row[ci[e]] += v[e] * scale;
     }
   }
   __syncthreads();

@@ -87,3 +87,18 @@ def test_operators_far_from_one(dev, n, scale):
     x = h.vcycle(torch.tensor(b * scale, device=dev), precision=64).cpu().numpy()
     y = np.linalg.solve(A, b)
     assert np.linalg.norm(x - y) <= 4 * n * 2.2e-16 * np.linalg.cond(A) * np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("n", [50, 64, 130, 300, 600])
+def test_repeated_columns_in_any_order(dev, n):
+    """Every entry given as two, in two sweeps over the columns: they add up. Each half
+    is positive definite, so that a lost one would not show as a failed elimination."""
+    import impes_hip as H
+
+    halves = [_spd(n, n + k)[0] for k in range(2)]
+    A = halves[0] + halves[1]
+    h = H.AmgHierarchy(coarsest_size=2000, dense_max=2000, coarse_pin=0)
+    rp = torch.arange(0, 2 * n * n + 1, 2 * n, dtype=torch.int32, device=dev)
+    ci = torch.arange(n, dtype=torch.int32, device=dev).repeat(2 * n)
+    h.setup_csr(rp, ci, torch.tensor(np.hstack(halves).ravel(), device=dev))
+    _check(h, A, np.sqrt(np.diag(A)), dev)
