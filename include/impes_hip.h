@@ -349,7 +349,10 @@ int impes_model_amg_setup_seconds(const impes_model* m, double* out);
  * time per cycle of level l's own launches (sweeps, residual, restriction,
  * prolongation, or the coarsest solve; children excluded); bytes_host[l] (may be
  * NULL) = the algorithmic HBM bytes of those launches per visit; *cycle_ms = mean
- * time of the same cycle replayed from its HIP graph. precision 32 or 64. */
+ * time of the preconditioner's cycle as the solver runs it (replayed from its HIP
+ * graph): the same launches for precision 32 on a hierarchy whose coarse end is not
+ * applied as one matrix, as at 1M cells; else that matrix stands for its levels, and
+ * precision 64 runs on padded operators. precision 32 or 64. */
 int impes_model_amg_level_times(impes_model* m, int precision, int cycles, double* ms_host, double* bytes_host,
                                 int max_levels, double* cycle_ms, void* stream);
 

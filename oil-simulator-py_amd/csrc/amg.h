@@ -148,7 +148,8 @@ class Hierarchy {
   // Preconditioner of the row-scaled system D^-1 A x = D^-1 b:
   // z = S .* V(S .* D .* v)  with S = D^-1/2 (equilibrated) or I.
   // The V-cycle between the two scalings is replayed from a HIP graph captured on
-  // first use after each setup (its buffers are fixed; updates keep them).
+  // first use after each setup (its buffers are fixed; updates keep them). Recorded into
+  // a caller's graph (graphs off), it applies the operators as of each replay.
   void precondition(int precision, const double* v, double* z, hipStream_t s);
   // The same preconditioner in three parts, for a caller that fuses the two
   // scalings into its own kernels: write in_scale() .* v (in the hierarchy's
@@ -161,14 +162,16 @@ class Hierarchy {
   void vcycle_only(int precision, hipStream_t s);
   void set_graphs(bool on) { graphs_ = on; }
   bool graphs() const { return graphs_; }
-  // Measurement: `cycles` eager V-cycles on the current V-cycle input with HIP
-  // events between the phases of every level; ms[l] = the mean stream time of
-  // level l's own launches per cycle (its sweeps, residual, restriction and
-  // prolongation, or the coarsest solve; its children excluded), l < num_levels.
-  // Then `cycles` graph replays of the same cycle: *cycle_ms = their mean.
+  // Measurement: `cycles` eager V-cycles on the current V-cycle input, level by level
+  // as vcycle64/32 run them, with HIP events between the phases of every level; ms[l] =
+  // the mean stream time of level l's own launches per cycle (its sweeps, residual,
+  // restriction and prolongation, or the coarsest solve; its children excluded), l <
+  // num_levels. Then *cycle_ms = the mean of `cycles` preconditioner cycles
+  // (vcycle_only): replays of the same launches in FP32 on a hierarchy without a matrix
+  // of the coarse end; else with that matrix, and in FP64 on the tiles.
   void level_times(int precision, int cycles, double* ms, double* cycle_ms, hipStream_t s);
-  // Algorithmic HBM bytes of one visit of level l in a zero-start cycle of the given
-  // precision, attributed like level_times: every operator and vector pass of the
+  // Algorithmic HBM bytes of one visit of level l in that level-by-level cycle from zero
+  // in the given precision, attributed like level_times: every operator and vector pass of the
   // level's own launches, each array once (row pointers, column indices and values
   // of A, R or P once per pass, the gathered vector once, the other vectors once).
   double level_bytes(int l, int precision) const;

@@ -2,7 +2,6 @@
 // All launchers enqueue on the given stream and never synchronise.
 #pragma once
 
-
 #include "common.h"
 
 namespace impes {
@@ -91,12 +90,12 @@ void launch_tile4_rows(int n, const int* rp, const long long* base, int* wrow, i
 // first entry (rectangular; 0 for an empty row). co4 and maxabs may be null.
 void launch_tile4_fill(int nw, const int* wrow, const int* rp, const int* ci, const double* v, const int* rp4,
                        int* ci4, short* co4, float* v4, unsigned short* tag, int* maxabs, bool square, hipStream_t s);
-// Plain form: lanes per row of the padded kernels from the padded entry count;
+// Plain form: lanes per row of the padded kernels from the padded entry count
 int csr4_group_for(int n_rows, long long nnz4);
-// padded row lengths: cnt[r] = rows' lengths rounded up to 4 (an empty row gets 4);
+// cnt[r] = row r's length rounded up to 4 (4 for an empty row)
 void launch_csr4_count(int n, const int* rp, int* cnt, hipStream_t s);
-// padded pattern (ci4 sized rp4[n]) and FP32 values (rounded from FP64), padding as
-// above (square);
+// padded columns (rp4[n] of them) and FP32 values (rounded from FP64); padding entries
+// as in the tiles of a square matrix
 void launch_csr4_pattern(int n, const int* rp, const int* ci, const int* rp4, int* ci4, hipStream_t s);
 void launch_csr4_values(int n, const int* rp, const double* v, const int* rp4, float* v4, hipStream_t s);
 // co4[e] = ci4[e] - row (16-bit) over nnz4 entries, *maxabs as above
@@ -105,17 +104,18 @@ void launch_csr4_offsets(int n, const int* rp4, const int* ci4, short* co4, int*
 void launch_residual4_f32(const Csr4F32& A, int group, const float* x, const float* b, float* r, hipStream_t s);
 void launch_jacobi4_f32(const Csr4F32& A, int group, const float* xi, const float* b, const float* inv_relax, float w,
                         float* xo, hipStream_t s);
-// restriction on a padded operator with wave tiles (A.nw > 0; column indices in ci4): y = A x; and y = A x with y2 = w inv_relax2 .* y (fused with the coarse
-// level's first sweep from zero)
+// restriction on a padded operator with wave tiles (A.nw > 0; column indices in ci4):
+// y = A x; and y = A x with y2 = w inv_relax2 .* y (fused with the coarse level's first
+// sweep from zero)
 void launch_spmv4_f32(const Csr4F32& A, const float* x, float* y, hipStream_t s);
 // prolongation and the sweep after it, S = P - w diag(inv_relax) AP in tiles: x = x0 +
-// w inv_relax .* r + S e (r = b - A x0; x may be x0); and the values of S, with the count of P's entries outside
-// its pattern added to *miss (or null)
+// w inv_relax .* r + S e (r = b - A x0; x may be x0); and the values of S, with the count
+// of P's entries outside its pattern added to *miss (or null)
 void launch_prolong_sweep4_f32(const Csr4F32& S, const float* e, const float* r, const float* inv_relax, float w,
                                float* x0, float* x, hipStream_t s);
 void launch_tile4_prolong_sweep(int nw, const int* wrow, const unsigned short* tag, const int* rp4, const int* ci4,
-                                const int* aprp, const double* apv, const int* prp, const int* pci, const double* pv, const double* ir,
-                                double w, float* v4, double* v8, int* miss, hipStream_t s);
+                                const int* aprp, const double* apv, const int* prp, const int* pci, const double* pv,
+                                const double* ir, double w, float* v4, double* v8, int* miss, hipStream_t s);
 // tiled patterns with FP64 values v8 (4 per chunk, 16-byte aligned; A.v4 is not read):
 // the values from CSR ones, and the passes above (launch_tile4_prolong_sweep fills v8
 // when it is given, else v4)

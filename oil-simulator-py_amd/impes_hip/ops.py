@@ -185,8 +185,9 @@ class AmgHierarchy:
 
     def level_times(self, precision=32, cycles=20):
         """Per-level V-cycle figures on the hierarchy's current V-cycle input
-        (impes_amg_level_times): (ms per eager cycle of each level's own launches,
-        their algorithmic bytes per visit, ms of one graph-replayed cycle)."""
+        (impes_amg_level_times): (ms of each level's own launches per eager cycle, level
+        by level; their algorithmic bytes per visit; ms of one cycle as the solver runs
+        it, replayed from its graph)."""
         ms, by = (C.c_double * 64)(), (C.c_double * 64)()
         cyc = C.c_double()
         call("impes_amg_level_times", self._h, int(precision), int(cycles), ms, by, 64, C.byref(cyc), stream_ptr())
@@ -468,8 +469,9 @@ class ImpesModel:
 
     def amg_level_times(self, precision=32, cycles=20):
         """Per-level V-cycle figures of the pressure hierarchy
-        (impes_model_amg_level_times): (ms per eager cycle of each level's own
-        launches, their algorithmic bytes per visit, ms of one graph-replayed cycle)."""
+        (impes_model_amg_level_times): (ms of each level's own launches per eager
+        cycle, level by level; their algorithmic bytes per visit; ms of one cycle as the
+        solver runs it, replayed from its graph)."""
         ms, by = (C.c_double * 64)(), (C.c_double * 64)()
         cyc = C.c_double()
         call("impes_model_amg_level_times", self._h, int(precision), int(cycles), ms, by, 64, C.byref(cyc),
