@@ -1,4 +1,7 @@
 // Scans, segmented sort and small reductions for the AMG setup phase.
+#include <mutex>
+#include <vector>
+
 #include "prims.h"
 
 namespace impes {
@@ -330,14 +333,35 @@ __global__ __launch_bounds__(8 * kWave) void k_readback(ReadItems it, long long*
   if (lane == 0) out[w] = v;
 }
 
-// Pinned words of the calling thread's readbacks, allocated on first use and kept
-// (one small block per thread; it must not outlive the HIP runtime, so it is not
-// freed at the thread's end).
-long long* readback_words() {
-  thread_local long long* words = nullptr;
-  if (!words) IMPES_HIP_CHECK(hipHostMalloc((void**)&words, 8 * sizeof(long long), hipHostMallocMapped | hipHostMallocPortable));
-  return words;
-}
+// Pinned words of a readback: from those that no other thread uses, so there are as many
+// as readbacks ever ran at once, however many threads come and go. They stay until the
+// process ends (after the HIP runtime may be gone).
+struct ReadbackWords {
+  long long* p = nullptr;
+  static std::mutex& lock() {
+    static std::mutex* m = new std::mutex();
+    return *m;
+  }
+  static std::vector<long long*>& unused() {
+    static std::vector<long long*>* v = new std::vector<long long*>();
+    return *v;
+  }
+  ReadbackWords() {
+    {
+      std::lock_guard<std::mutex> g(lock());
+      if (!unused().empty()) {
+        p = unused().back();
+        unused().pop_back();
+        return;
+      }
+    }
+    IMPES_HIP_CHECK(hipHostMalloc((void**)&p, 8 * sizeof(long long), hipHostMallocMapped | hipHostMallocPortable));
+  }
+  void give_back() {  // once the device has written them (a failed readback keeps its words)
+    std::lock_guard<std::mutex> g(lock());
+    unused().push_back(p);
+  }
+};
 
 // Order statistic of max(|x|, floor) by its bit pattern (positive doubles order like
 // their bits), digit by digit from the top: a histogram of the digit over the values
@@ -501,7 +525,8 @@ int Readback::add(const void* p, int bytes, int m) {
 
 void Readback::fetch(hipStream_t s) {
   if (n_ == 0) return;
-  long long* w = readback_words();
+  ReadbackWords words;
+  long long* w = words.p;
   long long* dev = nullptr;
   IMPES_HIP_CHECK(hipHostGetDevicePointer((void**)&dev, w, 0));
   ReadItems it{};
@@ -514,6 +539,7 @@ void Readback::fetch(hipStream_t s) {
   IMPES_LAUNCH_CHECK();
   IMPES_HIP_CHECK(hipStreamSynchronize(s));
   for (int q = 0; q < n_; ++q) v_[q] = static_cast<volatile long long*>(w)[q];
+  words.give_back();
 }
 
 long long sum_i32(const int* x, long long n, hipStream_t s) {

@@ -167,3 +167,29 @@ def test_builds_leave_other_threads_captures_alone(dev):
     for th in threads:
         th.join()
     assert not errors, errors[0]
+
+
+def test_threads_that_come_and_go_leave_nothing_behind(dev):
+    """Hierarchies built by one short-lived thread after another: the process's mappings
+    of device and pinned memory do not grow."""
+    import impes_hip as H
+
+    csr = _csr(impes_like(8, 8, 4, seed=3)[0], dev)
+
+    def work():
+        h = H.AmgHierarchy()
+        h.setup_csr(*csr)
+        h.close()
+
+    def mappings():
+        with open("/proc/self/maps") as f:
+            return sum("renderD" in line or "kfd" in line for line in f)
+
+    counts = []
+    for _ in range(3):
+        for _ in range(20):
+            th = threading.Thread(target=work)
+            th.start()
+            th.join()
+        counts.append(mappings())
+    assert counts[-1] - counts[0] <= 4, counts  # one a thread would be 40
