@@ -148,8 +148,9 @@ class Hierarchy {
   // Preconditioner of the row-scaled system D^-1 A x = D^-1 b:
   // z = S .* V(S .* D .* v)  with S = D^-1/2 (equilibrated) or I.
   // The V-cycle between the two scalings is replayed from a HIP graph captured on
-  // first use after each setup (its buffers are fixed; updates keep them). Recorded into
-  // a caller's graph (graphs off), it applies the operators as of each replay.
+  // first use after each setup (its buffers are fixed; updates keep them). On a stream
+  // that records a caller's graph its launches go there one by one; each replay of that
+  // graph applies the operators of the time.
   void precondition(int precision, const double* v, double* z, hipStream_t s);
   // The same preconditioner in three parts, for a caller that fuses the two
   // scalings into its own kernels: write in_scale() .* v (in the hierarchy's
@@ -284,7 +285,7 @@ class Hierarchy {
   Derived forms_[kForms];
   void form(Form f, hipStream_t s);
   void ensure(Form f, bool rec, hipStream_t s);
-  void prepare(int precision, bool tail, hipStream_t s);  // all that a cycle reads
+  void prepare(int precision, bool tail, bool rec, hipStream_t s);  // all that a cycle reads; rec: s records
 
   int tail_ = -1;  // first level of the coarse end's matrix (tail.hip), -1: none
   int tail_ld_ = 0;

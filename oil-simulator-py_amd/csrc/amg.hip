@@ -1025,8 +1025,7 @@ void Hierarchy::ensure(Form f, bool rec, hipStream_t s) {
   if (!rec) d.current = true;
 }
 
-void Hierarchy::prepare(int precision, bool tail, hipStream_t s) {
-  const bool rec = recording(s);
+void Hierarchy::prepare(int precision, bool tail, bool rec, hipStream_t s) {
   if (tail && tail_ >= 0) ensure(precision == 32 ? kTail32 : kTail64, rec, s);
   if (precision == 32) {
     ensure(kSweeps32, rec, s);
@@ -1243,7 +1242,7 @@ void Hierarchy::level_times(int precision, int cycles, double* ms, double* cycle
     }
   } done{this, c};
   Level& L0 = levels_[0];
-  prepare(precision, false, s);
+  prepare(precision, false, recording(s), s);
   IMPES_HIP_CHECK(hipStreamSynchronize(s));
   clock_ = &c;
   for (int i = 0; i < cycles; ++i) {
@@ -1370,7 +1369,7 @@ void Hierarchy::vcycle64(const double* b, double* x, bool x_zero, hipStream_t s)
 void Hierarchy::vcycle32(const float* b, float* x, bool x_zero, hipStream_t s) {
   IMPES_REQUIRE(!levels_.empty(), "vcycle before setup");
   SmoothSwap sw(prm_, transposed_);
-  prepare(32, false, s);
+  prepare(32, false, recording(s), s);
   vcycle_level<float>(0, b, x, x_zero, s);
 }
 
@@ -1400,7 +1399,7 @@ int Hierarchy::cycles_impl(const CycleWork& w, int precision, const double* b, d
   Level& L0 = levels_[0];
   const long long n = L0.n;
   double hv[2];
-  prepare(precision, false, s);
+  prepare(precision, false, recording(s), s);
   launch_scale_f64(w.b, dh_.p, b, n, s);  // bs = dh .* b
   if (use_x0) launch_div_f64(w.x, x, dh_.p, n, s);  // xs = x0 ./ dh
   launch_dot_f64(w.b, w.b, n, w.sc, w.part, s);
@@ -1452,10 +1451,13 @@ const void* Hierarchy::vcycle_out(int precision) const {
 void Hierarchy::vcycle_only(int precision, hipStream_t s) {
   IMPES_REQUIRE(!levels_.empty(), "preconditioner before setup");
   Level& L0 = levels_[0];
-  // a cycle that is one product needs no graph (its launch costs the host more)
-  const bool replay = graphs_ && !ktimer_enabled() && tail_ != 0;
+  const bool rec = recording(s);
+  // a cycle that is one product needs no graph (its launch costs the host more); into a
+  // caller's graph go the launches themselves (a replay recorded there, with its capture
+  // in the caller's, gave wrong results)
+  const bool replay = graphs_ && !rec && !ktimer_enabled() && tail_ != 0;
   const int gi = precision == 32 ? 0 : 1;
-  prepare(precision, true, s);
+  prepare(precision, true, rec, s);
   if (replay && !vexec_[gi]) capture_vcycle(precision);
   if (replay) IMPES_HIP_CHECK(hipGraphLaunch(vexec_[gi], s));
   else if (precision == 32) vcycle_level<float>(0, L0.b32.p, L0.x32.p, true, s, false, true);

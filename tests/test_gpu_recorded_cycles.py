@@ -21,8 +21,8 @@ SIGMAS = (1.0, 1.3, 0.7, 1.1)
 class Operators:
     """One pattern, several values, and what a fresh hierarchy makes of each."""
 
-    def __init__(self, dims, kind, dev):
-        self.dims, self.kind = dims, kind
+    def __init__(self, dims, kind, dev, graphs):
+        self.dims, self.kind, self.graphs = dims, kind, graphs
         self.csr = [to_dev(impes_like(*dims, seed=8, sigma=s)[0], dev) for s in SIGMAS]
         self.st = [[torch.tensor(a, dtype=torch.float64, device=dev) for a in impes_like(*dims, seed=8, sigma=s)[1:]]
                    for s in SIGMAS]
@@ -42,7 +42,7 @@ class Operators:
             h.setup_st7(self.dims, *self.st[0])
         else:
             h.setup_csr(*self.csr[0])
-        h.set_graphs(False)
+        h.set_graphs(self.graphs)
         return h
 
     def update(self, h):
@@ -77,14 +77,16 @@ def same(got, ref, what):
 params = pytest.mark.parametrize("precision", [64, 32])
 grids = pytest.mark.parametrize("dims", GRIDS)
 kinds = pytest.mark.parametrize("kind", ["csr", "st7"])
+graphs_ = pytest.mark.parametrize("graphs", [True, False])  # eager cycles replayed from a graph of their own
 
 
 @params
 @grids
 @kinds
-def test_recorded_cycle_after_eager_updates(dev, dims, kind, precision):
+@graphs_
+def test_recorded_cycle_after_eager_updates(dev, dims, kind, precision, graphs):
     """Warm up, record, update eagerly, replay."""
-    op = Operators(dims, kind, dev)
+    op = Operators(dims, kind, dev, graphs)
     refs = [op.reference(q, (precision,))[0] for q in range(3)]
     h = op.setup()
     z = h.precondition(op.v, precision=precision).clone()
@@ -101,11 +103,12 @@ def test_recorded_cycle_after_eager_updates(dev, dims, kind, precision):
 @params
 @grids
 @kinds
-def test_recorded_update_with_eager_cycles(dev, dims, kind, precision):
+@graphs_
+def test_recorded_update_with_eager_cycles(dev, dims, kind, precision, graphs):
     """Record an update, run an eager cycle, replay the update with new values, run an
     eager cycle; the update recorded with no cycle before it, after one of this
     precision, and after one of the other."""
-    op = Operators(dims, kind, dev)
+    op = Operators(dims, kind, dev, graphs)
     refs = [op.reference(q) for q in range(4)]
     for warm in ((), (precision,), (96 - precision,)):
         h = op.setup()
@@ -129,10 +132,11 @@ def test_recorded_update_with_eager_cycles(dev, dims, kind, precision):
 @params
 @grids
 @kinds
-def test_recorded_cycle_as_the_first_call(dev, dims, kind, precision):
+@graphs_
+def test_recorded_cycle_as_the_first_call(dev, dims, kind, precision, graphs):
     """The first cycle after a setup goes into a graph: nothing is allocated in it, and
     it serves the operators of later updates."""
-    op = Operators(dims, kind, dev)
+    op = Operators(dims, kind, dev, graphs)
     refs = [op.reference(q, (precision,))[0] for q in range(3)]
     h = op.setup()
     z = torch.empty_like(op.v)
@@ -151,10 +155,11 @@ def test_recorded_cycle_as_the_first_call(dev, dims, kind, precision):
 @params
 @grids
 @kinds
-def test_update_and_cycles_in_one_graph(dev, dims, kind, precision):
+@graphs_
+def test_update_and_cycles_in_one_graph(dev, dims, kind, precision, graphs):
     """An update with two cycles behind it, recorded after a warm-up, and a graph of
     cycles alone beside it."""
-    op = Operators(dims, kind, dev)
+    op = Operators(dims, kind, dev, graphs)
     refs = [op.reference(q, (precision,))[0] for q in range(3)]
     h = op.setup()
     z = [h.precondition(op.v, precision=precision).clone() for _ in range(3)]
