@@ -370,9 +370,23 @@ void launch_st7_to_csr_values(int nx, int ny, int nz, const double* d, const dou
 }
 
 // ---------------------------------------------------------------- setup
+namespace {
+// A setup that fails leaves no hierarchy (its levels lack their vectors and inverse).
+struct SetupGuard {
+  std::vector<Level>& levels;
+  bool done = false;
+  explicit SetupGuard(std::vector<Level>& l) : levels(l) {}
+  ~SetupGuard() {
+    if (!done) levels.clear();
+  }
+};
+}  // namespace
+
 void Hierarchy::setup_csr(int n, int nnz, const int* rp, const int* ci, const double* v, hipStream_t s) {
+  SetupGuard guard(levels_);
   stencil_ = false;
   setup_impl(n, nnz, rp, ci, v, s);
+  guard.done = true;
 }
 
 Hierarchy::Hierarchy(const AmgParams& p) : prm_(p) {
@@ -470,6 +484,7 @@ void Hierarchy::setup_stencil(int nx, int ny, int nz, const double* d, const dou
                               const double* oz, hipStream_t s) {
   const long long n = (long long)nx * ny * nz;
   IMPES_REQUIRE(n >= 1 && n < (1LL << 30), "amg setup: bad stencil grid");
+  SetupGuard guard(levels_);
   stencil_ = true;
   nx_ = nx; ny_ = ny; nz_ = nz;
   st_d_.alloc(n); st_x_.alloc(n); st_y_.alloc(n); st_z_.alloc(n);
@@ -486,6 +501,7 @@ void Hierarchy::setup_stencil(int nx, int ny, int nz, const double* d, const dou
   launch_st7_pattern_fill(nx, ny, nz, rp.p, ci.p, s);
   launch_st7_to_csr_values(nx, ny, nz, d, ox, oy, oz, rp.p, v.p, s);
   setup_impl((int)n, nnz, rp.p, ci.p, v.p, s);
+  guard.done = true;
 }
 
 void Hierarchy::equil_factors(const double* diag, bool decide, hipStream_t s) {

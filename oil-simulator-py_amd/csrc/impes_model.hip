@@ -1097,8 +1097,9 @@ void Model::assemble(double dt, const double* p, const double* sw, const double*
 
 void Model::solve(int precision, double rtol, int restart, int maxit, double* p_new, SolveStats& st, hipStream_t s) {
   if (!amg_) {
-    amg_ = std::make_unique<Hierarchy>(amg_prm_);
-    amg_->setup_stencil(grid.nx, grid.ny, grid.nz, diag.p, ox.p, oy.p, oz.p, s);
+    auto h = std::make_unique<Hierarchy>(amg_prm_);
+    h->setup_stencil(grid.nx, grid.ny, grid.nz, diag.p, ox.p, oy.p, oz.p, s);
+    amg_ = std::move(h);  // a setup that fails is tried again by the next solve
   } else {
     amg_->update_stencil(diag.p, ox.p, oy.p, oz.p, s);
   }

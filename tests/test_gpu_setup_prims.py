@@ -193,3 +193,31 @@ def test_threads_that_come_and_go_leave_nothing_behind(dev):
             th.join()
         counts.append(mappings())
     assert counts[-1] - counts[0] <= 4, counts  # one a thread would be 40
+
+
+@pytest.mark.parametrize("first", [False, True])
+def test_failed_setup_leaves_no_hierarchy(dev, first):
+    """A pattern that is not symmetric is refused; so is every use of the handle until a
+    setup succeeds, whether it had a hierarchy before or not."""
+    import impes_hip as H
+
+    A, *_ = impes_like(12, 10, 9, seed=3)
+    good = _csr(A, dev)
+    B = A.tolil()
+    B[5, 700] = -1e-11
+    B = sp.csr_matrix(B)
+    B.sort_indices()
+    b = torch.ones(A.shape[0], dtype=torch.float64, device=dev)
+    h, ref = H.AmgHierarchy(), H.AmgHierarchy()
+    ref.setup_csr(*good)
+    z = ref.precondition(b)
+    if first:
+        h.setup_csr(*good)
+        assert torch.equal(h.precondition(b), z)
+    with pytest.raises(H.ImpesError):
+        h.setup_csr(*_csr(B, dev))
+    for use in (lambda: h.precondition(b), lambda: h.vcycle(b), lambda: h.cycles(b), lambda: h.update_csr(good[2])):
+        with pytest.raises(H.ImpesError):
+            use()
+    h.setup_csr(*good)
+    assert torch.equal(h.precondition(b), z)
