@@ -957,8 +957,11 @@ Model::Model(const Grid& g, const FluidParams& f, int pvt_n, const double* pvt_h
     }
     pvt_P_.alloc(pvt_n);
     pvt_tab_.alloc(tab.size());
-    IMPES_HIP_CHECK(hipMemcpy(pvt_P_.p, P.data(), sizeof(double) * pvt_n, hipMemcpyHostToDevice));
-    IMPES_HIP_CHECK(hipMemcpy(pvt_tab_.p, tab.data(), sizeof(double2) * tab.size(), hipMemcpyHostToDevice));
+    // not hipMemcpy, which ends captures of other threads
+    IMPES_HIP_CHECK(hipMemcpyAsync(pvt_P_.p, P.data(), sizeof(double) * pvt_n, hipMemcpyHostToDevice, nullptr));
+    IMPES_HIP_CHECK(
+        hipMemcpyAsync(pvt_tab_.p, tab.data(), sizeof(double2) * tab.size(), hipMemcpyHostToDevice, nullptr));
+    IMPES_HIP_CHECK(hipStreamSynchronize(nullptr));
     pvt.n = pvt_n;
     pvt.P = pvt_P_.p;
     pvt.tab = pvt_tab_.p;
@@ -969,9 +972,7 @@ Model::Model(const Grid& g, const FluidParams& f, int pvt_n, const double* pvt_h
   if (gravity_) for (auto* b : {&rho_w_, &rho_o_, &rho_g_, &grav_}) b->alloc(n);
   if (F.pc_scale > 0.0) pc_.alloc(n);
   if (F.pcog_scale > 0.0) pcog_.alloc(n);
-  IMPES_HIP_CHECK(hipMemset(qw_.p, 0, n * sizeof(double)));
-  IMPES_HIP_CHECK(hipMemset(qg_.p, 0, n * sizeof(double)));
-  IMPES_HIP_CHECK(hipMemset(qo_.p, 0, n * sizeof(double)));
+  for (auto* b : {&qw_, &qg_, &qo_}) launch_fill_f64(b->p, 0.0, n, nullptr);
   part_.alloc((size_t)kTransBlocks * (kLedgerQ + 1));  // the demand's partials and the ledgers'
   set_wells(w, nullptr);
   IMPES_HIP_CHECK(hipStreamSynchronize(nullptr));

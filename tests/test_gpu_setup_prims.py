@@ -125,10 +125,13 @@ def test_update_after_a_reused_build(dev):
 
 
 def test_builds_leave_other_threads_captures_alone(dev):
-    """Hierarchies are built and destroyed while another thread records a graph of its
-    own (the first preconditioner call of a hierarchy records one as well)."""
+    """Hierarchies and simulators are built, used and destroyed while another thread
+    records a graph of its own (the first preconditioner call of a hierarchy records one
+    as well)."""
     import impes_hip as H
+    from simulator.cases import baseline_case, build
 
+    cfg, fields = baseline_case(1, dims=(8, 8, 3))
     A, *_ = impes_like(20, 18, 9, seed=3)
     csr = _csr(A, dev)
     b = torch.ones(A.shape[0], dtype=torch.float64, device=dev)
@@ -144,6 +147,7 @@ def test_builds_leave_other_threads_captures_alone(dev):
                     h.precondition(b, precision=32)
                     st.synchronize()
                     h.close()
+                    assert build(cfg, fields, "cuda:0").run_step(86400.0)
         except Exception as e:  # noqa: BLE001
             errors.append(e)
 
